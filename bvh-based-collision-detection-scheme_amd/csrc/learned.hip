@@ -20,8 +20,10 @@
 //   6-15 fraction of leaves whose external-front count c falls in bin floor(log2(1 + c)) (last bin 9+)
 // Numerics: weights rounded to bf16 (nearest even), layer inputs rounded to bf16 before the two
 // hidden products, fp32 accumulation (v_mfma_f32_16x16x16_bf16 for inference), fp32 biases
-// and output layer. Training: per-sample fp32 forward/backward of the MSE loss through the
-// same rounding (straight-through), block-reduced gradients, Adam on fp32 master weights.
+// and output layer. Training: fp32 forward/backward of the MSE loss through the same
+// rounding (straight-through) on v_mfma_f32_16x16x4_f32, gradients summed in a fixed order, Adam on
+// fp32 master weights.
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -40,6 +42,8 @@ constexpr int kOffW1 = 0, kOffB1 = kH * kIn, kOffW2 = kOffB1 + kH, kOffB2 = kOff
               kOffB3 = kOffW3 + kH, kNParam = kOffB3 + 1;
 static_assert(kNParam == BVHCD_MLP_NPARAM, "parameter packing");
 constexpr int32_t kTreeletLeaves = 4096;
+constexpr unsigned kTrainGrid = 256;      // training workgroups at most: one per CU
+constexpr int kGradStride = kNParam + 1;  // a training workgroup's sums: gradients, then the loss
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -61,6 +65,7 @@ struct LearnedState {
     float* m = nullptr;
     float* v = nullptr;
     float* loss = nullptr;
+    float* part = nullptr;     // training: per-workgroup gradient and loss sums
     int64_t adam_t = 0;
     float* x = nullptr;        // io scratch
     float* y = nullptr;
@@ -101,7 +106,8 @@ LearnedState* learned_create(hipStream_t) {
               hipMalloc(&L->grad, sizeof(float) * kNParam) == hipSuccess &&
               hipMalloc(&L->m, sizeof(float) * kNParam) == hipSuccess &&
               hipMalloc(&L->v, sizeof(float) * kNParam) == hipSuccess &&
-              hipMalloc(&L->loss, sizeof(float) * 4) == hipSuccess;
+              hipMalloc(&L->loss, sizeof(float) * 4) == hipSuccess &&
+              hipMalloc(&L->part, sizeof(float) * kTrainGrid * kGradStride) == hipSuccess;
     if (!ok) {
         learned_destroy(L);
         return nullptr;
@@ -111,7 +117,7 @@ LearnedState* learned_create(hipStream_t) {
 
 void learned_destroy(LearnedState* L) {
     if (!L) return;
-    for (void* p : {(void*)L->params, (void*)L->wbf, (void*)L->grad, (void*)L->m, (void*)L->v, (void*)L->loss,
+    for (void* p : {(void*)L->params, (void*)L->wbf, (void*)L->grad, (void*)L->m, (void*)L->v, (void*)L->loss, (void*)L->part,
                     (void*)L->x, (void*)L->y, (void*)L->t, (void*)L->roots, (void*)L->flags, (void*)L->pos,
                     (void*)L->total, (void*)L->feats, (void*)L->cand_cnt, (void*)L->cand_of_leaf, (void*)L->lcnt,
                     (void*)L->cand_of_int, (void*)L->gate, (void*)L->score})
@@ -302,85 +308,236 @@ int learned_forward_noalloc(LearnedState* L, int device, const float* feats, int
 }
 
 // ---------------------------------------------------------------- training (fp32)
-constexpr int kTrainBlock = 64;
+// Loss and gradients of one batch, every contraction on v_mfma_f32_16x16x4_f32 (fp32 operands,
+// fp32 accumulation; the rounded bf16 values of the forward are exact in fp32). A wave takes 16
+// rows at a time and keeps its gradient sums of both weight matrices in accumulators (80
+// registers) over all its rows. With lane l = 16 q + r and i = 0..3, an operand register holds
+// A[m = r][k] / B[k][n = r] for one k per lane and step, and D[m = 4 q + i][n = r]; taking step s
+// of a 16-wide k block as k = 4 q + s
+//  * makes a lane's operands over the 4 steps consecutive (one 16-byte LDS read), and
+//  * makes D of one product (rows 4 q + i, column r) the A or B operand of the row-contracted
+//    weight gradients as it stands; only the two products contracted over units (layer 2, and
+//    the gradient of layer 1's output) go through an LDS transpose (16 x 64 tile of the wave, row
+//    stride 68: writes and reads free of bank conflicts).
+// Each workgroup leaves its sums in `part` (kGradStride words), which k_train_finish adds up in a
+// fixed order: repeated runs give the same bits. Bound by MFMA issue and the launch itself:
+// 49,061 rows take 0.03 ms. (One thread per row, adding each of its 5313 gradients to the
+// workgroup's LDS sums, took 19.5 ms: all 64 lanes added to one LDS word at a time.)
+constexpr int kTrainBlock = 256;
+constexpr int kTrainWaves = kTrainBlock / 64;
+constexpr int kS1 = 20, kS2 = 68;                // LDS row strides: W1 (16 wide), 64-wide tiles
+
+__device__ inline void wave_lds_sync() {  // LDS operations of one wave complete in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ inline f32x4 mfma_f32_k16(const f32x4& a, const f32x4& b, f32x4 c) {  // 4 steps: k = 16
+#pragma unroll
+    for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
+    return c;
+}
 
 __global__ void __launch_bounds__(kTrainBlock) k_mlp_grad(const float* __restrict__ x, const float* __restrict__ tgt,
                                                           int64_t rows, const float* __restrict__ p,
-                                                          float* __restrict__ grad, float* __restrict__ loss) {
-    __shared__ float W1[kH * kIn], W2[kH * kH], W3[kH], B1[kH], B2[kH];
-    __shared__ float g[kNParam];
-    __shared__ float lsum;
-    for (int i = threadIdx.x; i < kH * kIn; i += kTrainBlock) W1[i] = rbf(p[kOffW1 + i]);
-    for (int i = threadIdx.x; i < kH * kH; i += kTrainBlock) W2[i] = rbf(p[kOffW2 + i]);
-    for (int i = threadIdx.x; i < kH; i += kTrainBlock) {
-        W3[i] = rbf(p[kOffW3 + i]);
-        B1[i] = p[kOffB1 + i];
-        B2[i] = p[kOffB2 + i];
+                                                          float* __restrict__ part) {
+    __shared__ __attribute__((aligned(16))) float W1[kH * kS1], W2[kH * kS2], W2t[kH * kS2];
+    __shared__ __attribute__((aligned(16))) float tile[kTrainWaves][16 * kS2];
+    __shared__ float sum[kGradStride];
+    const int w = threadIdx.x >> 6, lane = lane_id(), q = lane >> 4, r = lane & 15;
+    for (int i = threadIdx.x; i < kH * kIn; i += kTrainBlock) W1[(i / kIn) * kS1 + i % kIn] = rbf(p[kOffW1 + i]);
+    for (int i = threadIdx.x; i < kH * kH; i += kTrainBlock) {
+        const float v = rbf(p[kOffW2 + i]);
+        W2[(i / kH) * kS2 + i % kH] = v;
+        W2t[(i % kH) * kS2 + i / kH] = v;
     }
-    for (int i = threadIdx.x; i < kNParam; i += kTrainBlock) g[i] = 0.f;
-    if (threadIdx.x == 0) lsum = 0.f;
+    for (int i = threadIdx.x; i < kGradStride; i += kTrainBlock) sum[i] = 0.f;
     __syncthreads();
-    const float b3 = p[kOffB3];
-    const float inv_n = 1.0f / (float)rows;
-    for (int64_t row = (int64_t)blockIdx.x * kTrainBlock + threadIdx.x; row < rows;
-         row += (int64_t)gridDim.x * kTrainBlock) {
-        float xq[kIn];
-        for (int i = 0; i < kIn; ++i) xq[i] = rbf(x[row * kIn + i]);
-        float z1[kH], z2[kH];
-        for (int j = 0; j < kH; ++j) {
-            float acc = 0.f;
-            for (int i = 0; i < kIn; ++i) acc += W1[j * kIn + i] * xq[i];
-            z1[j] = acc + B1[j];
+    float* const tl = tile[w];
+    float b1[4], b2[4], w3[4];  // this lane's units 16 t + r
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        b1[t] = p[kOffB1 + 16 * t + r];
+        b2[t] = p[kOffB2 + 16 * t + r];
+        w3[t] = rbf(p[kOffW3 + 16 * t + r]);
+    }
+    const float b3 = p[kOffB3], inv_n = 1.0f / (float)rows;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 g2[4][4], g1[4];  // gradients of W2 [unit tile][input tile] and of W1 [unit tile]
+    float gw3[4], gb2[4], gb1[4], gb3 = 0.f, loss = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        g1[t] = zero;
+        gw3[t] = gb2[t] = gb1[t] = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) g2[t][u] = zero;
+    }
+    const int64_t tiles = (rows + 15) / 16;
+    for (int64_t tn = (int64_t)blockIdx.x * kTrainWaves + w; tn < tiles; tn += (int64_t)gridDim.x * kTrainWaves) {
+        const int64_t row0 = 16 * tn;
+        f32x4 xa, xb, tg;  // x[r][4 q + s] (layer 1), x[4 q + s][r] (gradient of W1), targets of rows 4 q + i
+        bool ok[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            ok[s] = row0 + 4 * q + s < rows;
+            xa[s] = row0 + r < rows ? rbf(x[(row0 + r) * kIn + 4 * q + s]) : 0.f;
+            xb[s] = ok[s] ? rbf(x[(row0 + 4 * q + s) * kIn + r]) : 0.f;
+            tg[s] = ok[s] ? tgt[row0 + 4 * q + s] : 0.f;
         }
-        for (int j = 0; j < kH; ++j) {
-            float acc = 0.f;
-            for (int k = 0; k < kH; ++k) acc += W2[j * kH + k] * rbf(fmaxf(z1[k], 0.f));
-            z2[j] = acc + B2[j];
-        }
-        float yv = b3;
-        for (int j = 0; j < kH; ++j) yv += W3[j] * fmaxf(z2[j], 0.f);
-        const float res = yv - tgt[row];
-        atomicAdd(&lsum, res * res * inv_n);
-        const float dy = 2.f * res * inv_n;
-        atomicAdd(&g[kOffB3], dy);
-        for (int j = 0; j < kH; ++j) {
-            const float h2 = fmaxf(z2[j], 0.f);
-            atomicAdd(&g[kOffW3 + j], dy * h2);
-            z2[j] = z2[j] > 0.f ? dy * W3[j] : 0.f;  // now dz2
-            atomicAdd(&g[kOffB2 + j], z2[j]);
-        }
-        for (int k = 0; k < kH; ++k) {
-            const float h1q = rbf(fmaxf(z1[k], 0.f));
-            float dh1 = 0.f;
-            for (int j = 0; j < kH; ++j) {
-                atomicAdd(&g[kOffW2 + j * kH + k], z2[j] * h1q);
-                dh1 += W2[j * kH + k] * z2[j];
+        f32x4 h1[4], d1[4], dz2[4];  // units 16 t + r of rows 4 q + i
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {  // layer 1
+            const f32x4 b = *reinterpret_cast<const f32x4*>(&W1[(16 * t + r) * kS1 + 4 * q]);
+            const f32x4 z = mfma_f32_k16(xa, b, zero);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float z1 = z[i] + b1[t];
+                d1[t][i] = z1 > 0.f ? 1.f : 0.f;
+                h1[t][i] = ok[i] ? rbf(fmaxf(z1, 0.f)) : 0.f;
+                tl[(4 * q + i) * kS2 + 16 * t + r] = h1[t][i];
             }
-            z1[k] = z1[k] > 0.f ? dh1 : 0.f;  // now dz1
-            atomicAdd(&g[kOffB1 + k], z1[k]);
-            for (int i = 0; i < kIn; ++i) atomicAdd(&g[kOffW1 + k * kIn + i], z1[k] * xq[i]);
+        }
+        wave_lds_sync();
+        f32x4 a[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = *reinterpret_cast<const f32x4*>(&tl[r * kS2 + 16 * c + 4 * q]);
+        wave_lds_sync();  // the tile is rewritten below
+        f32x4 z2[4], y = zero;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {  // layer 2 and this lane's part of the output layer
+            z2[t] = zero;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const f32x4 b = *reinterpret_cast<const f32x4*>(&W2[(16 * t + r) * kS2 + 16 * c + 4 * q]);
+                z2[t] = mfma_f32_k16(a[c], b, z2[t]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                z2[t][i] += b2[t];
+                y[i] += w3[t] * fmaxf(z2[t][i], 0.f);
+            }
+        }
+        f32x4 dy;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) y[i] += __shfl_xor(y[i], off);
+            const float res = ok[i] ? y[i] + b3 - tg[i] : 0.f;
+            if (r == 0) loss += res * res * inv_n;
+            dy[i] = 2.f * res * inv_n;
+            if (r == 0) gb3 += dy[i];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                gw3[t] += ok[i] ? dy[i] * fmaxf(z2[t][i], 0.f) : 0.f;
+                dz2[t][i] = z2[t][i] > 0.f ? dy[i] * w3[t] : 0.f;
+                gb2[t] += dz2[t][i];
+                tl[(4 * q + i) * kS2 + 16 * t + r] = dz2[t][i];
+            }
+        wave_lds_sync();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = *reinterpret_cast<const f32x4*>(&tl[r * kS2 + 16 * c + 4 * q]);
+        wave_lds_sync();
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 dh = zero;  // gradient of layer 1's output
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const f32x4 b = *reinterpret_cast<const f32x4*>(&W2t[(16 * t + r) * kS2 + 16 * c + 4 * q]);
+                dh = mfma_f32_k16(a[c], b, dh);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                dh[i] = d1[t][i] > 0.f ? dh[i] : 0.f;
+                gb1[t] += dh[i];
+            }
+            g1[t] = mfma_f32_k16(dh, xb, g1[t]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) g2[t][u] = mfma_f32_k16(dz2[t], h1[u], g2[t][u]);
         }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < kNParam; i += kTrainBlock)
-        if (g[i] != 0.f) atomicAdd(&grad[i], g[i]);
-    if (threadIdx.x == 0) atomicAdd(loss, lsum);
+    // per-unit sums: the four row groups of a wave hold partial sums of the same unit
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            gw3[t] += __shfl_xor(gw3[t], off);
+            gb2[t] += __shfl_xor(gb2[t], off);
+            gb1[t] += __shfl_xor(gb1[t], off);
+        }
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+        gb3 += __shfl_xor(gb3, off);
+        loss += __shfl_xor(loss, off);
+    }
+    for (int ww = 0; ww < kTrainWaves; ++ww) {  // waves add in turn: a fixed order
+        if (w == ww) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int unit = 16 * t + 4 * q + i;
+                    sum[kOffW1 + unit * kIn + r] += g1[t][i];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) sum[kOffW2 + unit * kH + 16 * u + r] += g2[t][u][i];
+                }
+                if (q == 0) {
+                    sum[kOffW3 + 16 * t + r] += gw3[t];
+                    sum[kOffB2 + 16 * t + r] += gb2[t];
+                    sum[kOffB1 + 16 * t + r] += gb1[t];
+                }
+            }
+            if (lane == 0) {
+                sum[kOffB3] += gb3;
+                sum[kNParam] += loss;
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < kGradStride; i += kTrainBlock) part[(int64_t)blockIdx.x * kGradStride + i] = sum[i];
 }
 
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v,
-                       float lr, float bc1, float bc2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kNParam) return;
-    const float gi = g[i];
+// Adds up the workgroups' sums (column per lane, 16 slices of workgroups per column, then the
+// slices in order) into the gradient and the loss; with ADAM also takes the step and refreshes
+// the bf16 copy of the weights.
+template <bool ADAM>
+__global__ void __launch_bounds__(1024) k_train_finish(const float* __restrict__ part, unsigned blocks,
+                                                       float* __restrict__ grad, float* __restrict__ loss,
+                                                       float* __restrict__ p, float* __restrict__ m,
+                                                       float* __restrict__ v, uint16_t* __restrict__ wbf, float lr,
+                                                       float bc1, float bc2) {
+    __shared__ float slice[16][64];
+    const int lane = lane_id(), s = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    float acc = 0.f;
+    if (i < kGradStride)
+        for (unsigned b = s; b < blocks; b += 16) acc += part[(int64_t)b * kGradStride + i];
+    slice[s][lane] = acc;
+    __syncthreads();
+    if (s != 0 || i >= kGradStride) return;
+    float gi = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) gi += slice[k][lane];
+    if (i == kNParam) {
+        *loss = gi;
+        return;
+    }
+    grad[i] = gi;
+    if (!ADAM) return;
     const float mi = 0.9f * m[i] + 0.1f * gi;
     const float vi = 0.999f * v[i] + 0.001f * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
+    const float pi = p[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
+    p[i] = pi;
+    wbf[i] = f2bf(pi);
 }
+constexpr unsigned kFinishGrid = (kGradStride + 63) / 64;
 
-static int run_grad(LearnedState* L, const float* feats, const float* targets, int64_t rows, int where,
-                    hipStream_t s) {
+// Launches the gradient kernel over the batch; `blocks` = the workgroups whose sums are in L->part.
+static int run_grad(LearnedState* L, const float* feats, const float* targets, int64_t rows, int where, hipStream_t s,
+                    unsigned* blocks) {
     const float* dx = feats;
     const float* dt = targets;
     if (where != BVHCD_MEM_DEVICE) {
@@ -391,18 +548,19 @@ static int run_grad(LearnedState* L, const float* feats, const float* targets, i
         dx = L->x;
         dt = L->t;
     }
-    (void)hipMemsetAsync(L->grad, 0, sizeof(float) * kNParam, s);
-    (void)hipMemsetAsync(L->loss, 0, sizeof(float), s);
-    unsigned blocks = (unsigned)((rows + kTrainBlock - 1) / kTrainBlock);
-    if (blocks > 512) blocks = 512;
-    hipLaunchKernelGGL(k_mlp_grad, dim3(blocks), dim3(kTrainBlock), 0, s, dx, dt, rows, L->params, L->grad, L->loss);
+    const int64_t per = 16 * kTrainWaves;
+    *blocks = (unsigned)std::min<int64_t>((rows + per - 1) / per, kTrainGrid);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(*blocks), dim3(kTrainBlock), 0, s, dx, dt, rows, L->params, L->part);
     return hipGetLastError() == hipSuccess ? BVHCD_OK : BVHCD_E_DEVICE;
 }
 
 int learned_grad(LearnedState* L, const float* feats, const float* targets, int64_t rows, float* grad, float* loss,
                  int where, hipStream_t s, std::string* err) {
-    int st = run_grad(L, feats, targets, rows, where, s);
+    unsigned blocks = 0;
+    int st = run_grad(L, feats, targets, rows, where, s, &blocks);
     if (st) return st;
+    hipLaunchKernelGGL(k_train_finish<false>, dim3(kFinishGrid), dim3(1024), 0, s, L->part, blocks, L->grad, L->loss,
+                       nullptr, nullptr, nullptr, nullptr, 0.f, 1.f, 1.f);
     float lv = 0;
     if (hipMemcpyAsync(grad, L->grad, sizeof(float) * kNParam, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipMemcpyAsync(&lv, L->loss, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -416,13 +574,14 @@ int learned_grad(LearnedState* L, const float* feats, const float* targets, int6
 
 int learned_train_step(LearnedState* L, const float* feats, const float* targets, int64_t rows, float lr, float* loss,
                        int where, hipStream_t s, std::string* err) {
-    int st = run_grad(L, feats, targets, rows, where, s);
+    unsigned blocks = 0;
+    int st = run_grad(L, feats, targets, rows, where, s, &blocks);
     if (st) return st;
     L->adam_t++;
     const float bc1 = 1.0f - powf(0.9f, (float)L->adam_t), bc2 = 1.0f - powf(0.999f, (float)L->adam_t);
-    hipLaunchKernelGGL(k_adam, dim3(grid_for(kNParam)), dim3(kBlock), 0, s, L->params, L->grad, L->m, L->v, lr, bc1,
-                       bc2);
-    if (refresh_bf16(L, s)) return BVHCD_E_DEVICE;
+    hipLaunchKernelGGL(k_train_finish<true>, dim3(kFinishGrid), dim3(1024), 0, s, L->part, blocks, L->grad, L->loss,
+                       L->params, L->m, L->v, L->wbf, lr, bc1, bc2);
+    if (hipGetLastError() != hipSuccess) return BVHCD_E_DEVICE;
     float lv = 0;
     if (hipMemcpyAsync(&lv, L->loss, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {

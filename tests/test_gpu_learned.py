@@ -78,6 +78,30 @@ def test_mlp_gradient_matches_reference(pkg):
     ctx.close()
 
 
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 64, 65, 1000, 16384, 16385, 40007])
+def test_mlp_gradient_row_tiles(pkg, rows):
+    """Row counts around the 16-row tiles, the workgroup's 64 rows and the full grid's 16384: the
+    gradient against the quantised float64 reference, and the same bits on a second run. Both
+    round the same values to bf16; an activation within fp32 rounding of a bf16 tie can still
+    round the other way (2^-8 of that row's value): 1e-3 of the gradient's norm on many rows,
+    1e-2 on one tile's, where a single such row weighs more."""
+    print(f"[gpu] mlp gradient, {rows} rows", flush=True)
+    ctx = pkg.CollisionContext(16, 48)
+    p = mlp_ref.init_params(21)
+    ctx.mlp_set_weights(p)
+    x = _feature_rows(rows, 5)
+    t = np.random.default_rng(6).normal(size=rows).astype(np.float32)
+    g, loss = ctx.mlp_grad(x, t)
+    lref, gref = mlp_ref.loss_and_grad(p, x, t, quant=True)
+    tol = 1e-2 if rows <= 65 else 1e-3
+    assert loss == pytest.approx(lref, rel=tol)
+    assert np.linalg.norm(g - gref) <= tol * np.linalg.norm(gref)
+    again, loss2 = ctx.mlp_grad(x, t)
+    np.testing.assert_array_equal(g, again)
+    assert loss == loss2
+    ctx.close()
+
+
 def test_mlp_training_step_and_convergence(pkg):
     print("[gpu] mlp training", flush=True)
     ctx = pkg.CollisionContext(16, 48)
