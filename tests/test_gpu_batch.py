@@ -175,3 +175,29 @@ def test_keep_launch_shapes(pkg, oracle, grid, unroll, block):
         pkg.autotune_set(pkg.TUNE_KEEP, sc.num_tris, 2048, 1)
         pkg.autotune_set(pkg.TUNE_NARROW, sc.num_tris, 4096, 1)
         ctx.close()
+
+
+@pytest.mark.parametrize("num", [1, 64, 4096, 4097])
+def test_batch_grouping_by_scene_count(pkg, num):
+    """Hits grouped by scene at the scene counts around the LDS-counted limit (4096): scene k is a
+    fan of 2 + k % 5 triangles around one vertex (every pair of them is a hit) plus one far
+    triangle, so scene k's pairs are known."""
+    print(f"[gpu] batch grouping, {num} scenes", flush=True)
+    tris = np.array([2 + k % 5 for k in range(num)])
+    faces, xyz = [], []
+    for m in tris:
+        a = np.linspace(0.0, 1.5, m + 1)
+        ring = np.stack([np.cos(a), np.sin(a), 0.1 * a], 1)
+        xyz.append(np.concatenate([[[0.0, 0.0, 0.0]], ring, [[9, 9, 9], [9.1, 9, 9], [9, 9.1, 9]]]).astype(np.float32))
+        f = [[0, i + 1, i + 2] for i in range(m)] + [[m + 2, m + 3, m + 4]]
+        faces.append(np.array(f, np.int32))
+    b = pkg.Batch([len(f) for f in faces], [len(v) for v in xyz])
+    b.set_topology(np.concatenate(faces))
+    b.update_vertices(np.concatenate(xyz))
+    for op in (pkg.BVH_BUILD, pkg.BVH_REFIT):
+        b.step(op, use_graph=False)
+        np.testing.assert_array_equal(b.pair_counts(), tris * (tris - 1) // 2)
+        for k in sorted({0, num // 2, num - 1}):
+            want = [(i, j) for i in range(tris[k]) for j in range(i + 1, tris[k])]
+            np.testing.assert_array_equal(_set(b.pairs(k)), np.array(want, np.int32).reshape(-1, 2))
+    b.close()
