@@ -10,8 +10,8 @@
 //    subtree (a scene boundary differs in a bit above the Morton bits, i.e. a larger delta than
 //    anything inside a scene); each scene's subtree is the LBVH the scene alone would get;
 //  * refit and the narrow phase run once over all triangles;
-//  * the self-CD traversal is one persistent launch: waves take 64-query chunks from a global
-//    counter and each query walks only its own scene's leaves to its right;
+//  * the self-CD traversal is one launch: a wave takes 64 queries at a time, each paired only with
+//    its own scene's leaves to its right;
 //  * the narrow-phase hits are grouped per scene on the device (counts, exclusive scan,
 //    scatter) into scene-local triangle ids;
 //  * every launch of a frame reads its sizes from device memory and clears its counters with
@@ -46,7 +46,6 @@ struct bvhcd_batch {
     uint32_t* scnt = nullptr;         // S + 1 hits per scene, then exclusive offsets
     uint32_t* scur = nullptr;         // S + 1 scatter cursors
     uint32_t* gtbl = nullptr;         // hits per scene and workgroup (S <= kGroupScenes)
-    uint32_t* queue = nullptr;        // traversal work counter
     int2* grouped = nullptr;          // pair_cap, hits grouped by scene (scene-local ids)
     bool topo = false, built = false, keys_in_tmp = false;
     hipGraph_t graph[2] = {nullptr, nullptr};          // [0] build frame, [1] refit frame
@@ -326,7 +325,7 @@ void record_frame(bvhcd_batch* b, int bvh_op, unsigned grid) {
         launch_refit_prep(d, n, s);
     }
     launch_refit(d, n, s);
-    launch_batch_cd(d, n, b->keys, b->scene_last, b->queue, grid, s);
+    launch_batch_cd(d, n, b->keys, b->scene_last, grid, s);
     launch_narrow(d, s, true);  // launch_batch_cd reset the counters
     launch_pair_totals(d, s, true);
     if (b->S <= kGroupScenes) {
@@ -474,7 +473,6 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     ok &= balloc(b, b->scnt, S + 1);
     ok &= balloc(b, b->scur, S + 1);
     ok &= balloc(b, b->gtbl, (size_t)gtbl_n);
-    ok &= balloc(b, b->queue, 4);
     if (!ok) {
         for (void* p : b->allocs) (void)hipFree(p);
         if (b->own_stream) (void)hipStreamDestroy(b->stream);
@@ -621,7 +619,7 @@ int bvhcd_batch_get_pairs(bvhcd_batch* b, int32_t scene, int32_t* out, int64_t c
 
 const char* bvhcd_batch_last_error(const bvhcd_batch* b) { return b ? b->err.c_str() : "null batch"; }
 
-// Autotune of the persistent traversal's grid (workgroups resident on the device): every
+// Autotune of the traversal's grid (workgroups, each taking groups of queries in turn): every
 // candidate replays the refit frame a few times on the batch's current data, timed with
 // events; the fastest is kept for this size class (process-wide table) and the frame graphs are
 // re-captured on their next use.
@@ -633,10 +631,10 @@ int bvhcd_batch_autotune(bvhcd_batch* b) {
         return bfail(b, BVHCD_E_DEVICE, "event create failed");
     float best_ms = 1e30f;
     unsigned best = batch_grid(b);
-    for (unsigned g : {256u, 512u, 1024u, 2048u, 4096u, 8192u}) {
-        launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, b->queue, g, b->stream);  // warm-up
+    for (unsigned g : {1024u, 2048u, 4096u, 8192u, 0xFFFFFFu}) {
+        launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, g, b->stream);  // warm-up
         (void)hipEventRecord(e0, b->stream);
-        for (int r = 0; r < 3; ++r) launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, b->queue, g, b->stream);
+        for (int r = 0; r < 3; ++r) launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, g, b->stream);
         (void)hipEventRecord(e1, b->stream);
         if (hipEventSynchronize(e1) != hipSuccess) {
             (void)hipEventDestroy(e0);

@@ -156,7 +156,9 @@ struct DevState {
     uint32_t* int_mark = nullptr;
     int32_t* int_rx = nullptr;
     int32_t* int_ry = nullptr;
-    int4* itopo = nullptr;          // T-1 packed (lc, rc, par, mark)
+    int4* itopo = nullptr;          // T-1: children and parent as (id << 1 | bit), last leaf: x, y = left,
+                                    // right child with bit 0 = leaf (the encoding of escapes), z = parent
+                                    // with bit 0 = this node is its right child (negative: root), w = rangey
     // refit schedule, rebuilt after every topology change (treelet chunks + top tree)
     int32_t* rp_cstart = nullptr;   // chunks + 1: first leaf of each chunk, then T
     int2* rp_cinfo = nullptr;       // chunks: (internal nodes, deepest level | treelet roots << 16)

@@ -618,7 +618,7 @@ static unsigned stream_grid() { return 2048; }
 // process-wide and not locked.
 namespace {
 constexpr int kClasses = 40;
-const unsigned kDefaultGrid[TK_COUNT] = {2048u, 4096u, 2048u};
+const unsigned kDefaultGrid[TK_COUNT] = {2048u, 4096u, 0xFFFFFFu};  // batched traversal: one group per wave
 unsigned g_grid[TK_COUNT][kClasses] = {};
 struct TuneTrial {
     int kernel, cls;
@@ -766,54 +766,307 @@ __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, DevState d, Fron
     add_visits(d, v);
 }
 
+// ---------------------------------------------------------------- pairs of 64 queries at a time
+// The overlapping leaf pairs (q, j > q) of a whole tree, without a front. A wave takes 64 queries
+// (neighbouring sorted leaves) together and works in two steps:
+//  * nodes: the tree from its root, 64 nodes per round off a per-wave LDS stack, each lane testing
+//    one node against the boxes of the 64 queries and dropping subtrees that hold no leaf after the
+//    first query. A run of neighbouring leaves can jump (Morton order), and one box around a jump
+//    covers everything between: the run is cut at its three widest jumps and a node is tested
+//    against the four pieces' boxes (2M-triangle folded cloth: 481 nodes per wave instead of 793,
+//    the worst wave 2281 instead of 59425);
+//  * leaves: each leaf reached (170 per wave there) is loaded once for the wave (scalar load) and
+//    tested by every lane against its own query; hits go to the wave's LDS list.
+// Every node test serves 64 queries and every leaf record is fetched once per wave, where a walk
+// or a front entry per query fetches two 32-byte records per test. A pair is found exactly when the
+// leaves' boxes overlap, as in a query's own walk: a node's box holds its leaves' boxes and a piece's
+// box its queries', so no ancestor of an overlapping leaf is dropped. (Boxes given by the caller can
+// hold NaN, for which that is not so: they take the walks and fronts.)
+// skip_adj: pairs of triangles that share a vertex are removed when the LDS list is flushed (64 pairs
+// per step; the query's vertex ids come from its lane).
+// Bound by instruction issue (61 % of the VALU and 63 % of the scalar slots busy; half the node
+// rounds run with few nodes). Folded cloths: 180k triangles 185 -> 145 us (against the queries' own
+// walks sharing a wave's lanes), 64 scenes of 2.6M triangles 1.04 -> 0.56 ms (against a walk per
+// lane). KEEP's test of a front stays where there is one: 0.56 ms against 0.60 ms here on the 2M
+// cloth, and 12 us against 43 us on 2,560 triangles, where the tree's depth in rounds is what counts.
+constexpr uint32_t kGroupStack = 512;  // encoded nodes per wave (2 KB)
+constexpr uint32_t kGroupStage = 512;  // staged pairs per wave (4 KB): flushes of 257..512 pairs
+constexpr int kGroupPieces = 4;
+struct GroupLds {
+    uint32_t stack[kWaves][kGroupStack];
+    uint32_t cand[kWaves][128];        // leaves reached, tested 64 at a time
+    int2 pairs[kWaves][kGroupStage];
+    uint32_t fill[kWaves][2];          // [1]: segment rotor (stage_flush)
+};
+__device__ inline float lane_f(float v, int lane) {
+    return i2f(__builtin_amdgcn_readlane(f2i(v), lane));
+}
+__device__ inline uint32_t wave_max(uint32_t v) {
+    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
+    return v;
+}
+typedef const __attribute__((address_space(4))) float4 const_float4;  // loaded through the scalar cache
+
+template <bool BATCH>
+__global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
+                                                     const uint64_t* __restrict__ keys,
+                                                     const int32_t* __restrict__ scene_last) {
+    __shared__ GroupLds lds;
+    const int w = threadIdx.x >> 6, lane = lane_id();
+    lds_u32* const stk = (lds_u32*)lds.stack[w];
+    lds_u32* const cand = (lds_u32*)lds.cand[w];
+    lds_int2* const sb = (lds_int2*)lds.pairs[w];
+    lds_u32* const sf = (lds_u32*)lds.fill[w];
+    if (lane == 0) sf[1] = rotor_start();
+    const SegPairSink sink = pair_segments(d, 0, 4u);
+    uint32_t* const ovf = &d.ctr[C_OVF];
+    const bool drop_adj = d.skip_adj != 0;
+    // each XCD takes one contiguous eighth of the groups; the grid is a multiple of the XCDs
+    const uint32_t groups = ((uint32_t)n + 63u) / 64u, share = (groups + kXcds - 1) / kXcds;
+    const uint32_t xcd = blockIdx.x % kXcds, end_gi = min((xcd + 1) * share, groups);
+    uint32_t visits = 0;
+    for (uint32_t gi = xcd * share + (blockIdx.x / kXcds) * kWaves + w; gi < end_gi;  // wave-uniform
+         gi += gridDim.x / kXcds * kWaves) {
+        const int32_t g0 = (int32_t)(gi * 64u), q = g0 + lane;
+        const bool valid = q < n;
+        Box qb = empty_box();
+        int32_t after = INT32_MAX, last = n - 1;  // this lane's leaves: (after, last]
+        int32_t f0 = 0, f1 = 0, f2 = 0;           // its triangle's vertices
+        if (valid) {
+            const float4 lo = d.leaf[q].lo, hi = d.leaf[q].hi;
+            qb = rec_box(lo, hi);
+            after = q;
+            if (BATCH) last = scene_last[(int32_t)(keys[q] >> 30)];
+            if (drop_adj) {
+                f0 = d.lfaces[3 * (int64_t)q];
+                f1 = d.lfaces[3 * (int64_t)q + 1];
+                f2 = d.lfaces[3 * (int64_t)q + 2];
+            }
+        }
+        // the wave's last leaf (scenes follow one another in leaf order)
+        const int32_t glast =
+            BATCH ? __builtin_amdgcn_readlane(last, min(63, n - 1 - g0)) : n - 1;
+        // cut the 64 queries at their widest jumps between box centres
+        const float cx = qb.mnx + qb.mxx, cy = qb.mny + qb.mxy, cz = qb.mnz + qb.mxz;
+        const float gap = fabsf(__shfl_down(cx, 1) - cx) + fabsf(__shfl_down(cy, 1) - cy) + fabsf(__shfl_down(cz, 1) - cz);
+        uint32_t key = lane < 63 && q + 1 < n ? (((uint32_t)f2i(gap) & 0x7FFFFFC0u) | (uint32_t)lane) : 0u;
+        uint64_t heads = 1ull;  // first lanes of the pieces
+#pragma unroll
+        for (int c = 1; c < kGroupPieces; ++c) {
+            const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max(key));
+            if (k == 0u) break;
+            heads |= 2ull << (k & 63u);
+            if (lane == (int)(k & 63u)) key = 0u;
+        }
+        const int first = 63 - __clzll((long long)(heads & ((2ull << lane) - 1ull)));  // this lane's piece
+        Box pb = qb;
+        for (int off = 1; off < 64; off <<= 1) {  // box of the piece up to this lane
+            const Box o{__shfl_up(pb.mnx, off), __shfl_up(pb.mny, off), __shfl_up(pb.mnz, off),
+                        __shfl_up(pb.mxx, off), __shfl_up(pb.mxy, off), __shfl_up(pb.mxz, off)};
+            if (lane - off >= first) pb = box_merge(pb, o);
+        }
+        Box piece[kGroupPieces];
+#pragma unroll
+        for (int c = 0; c < kGroupPieces; ++c) {  // wave-uniform (scalar registers)
+            const uint64_t rest = heads & (heads - 1ull);  // without its first piece
+            const int end = rest ? __ffsll((long long)rest) - 2 : 63;
+            piece[c] = Box{lane_f(pb.mnx, end), lane_f(pb.mny, end), lane_f(pb.mnz, end),
+                           lane_f(pb.mxx, end), lane_f(pb.mxy, end), lane_f(pb.mxz, end)};
+            if (rest) heads = rest;  // fewer pieces: the last one again
+        }
+
+        uint32_t fill = 0;
+        auto flush = [&]() {
+            uint32_t f = fill;
+            if (drop_adj) {  // compacted in place: every step writes below what it has read
+                f = 0;
+                for (uint32_t b = 0; b < fill; b += 128) {
+                    int2 p[2];
+                    int32_t v[2][3];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const uint32_t i = b + 64u * u + lane;
+                        p[u] = i < fill ? make_int2(sb[i].x, sb[i].y) : make_int2(g0, g0);
+                        const int32_t* fc = d.lfaces + 3 * (int64_t)p[u].y;
+                        v[u][0] = fc[0];
+                        v[u][1] = fc[1];
+                        v[u][2] = fc[2];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const int src = p[u].x - g0;
+                        const int32_t a0 = __shfl(f0, src), a1 = __shfl(f1, src), a2 = __shfl(f2, src);
+                        const bool share = a0 == v[u][0] || a0 == v[u][1] || a0 == v[u][2] || a1 == v[u][0] ||
+                                           a1 == v[u][1] || a1 == v[u][2] || a2 == v[u][0] || a2 == v[u][1] ||
+                                           a2 == v[u][2];
+                        const bool keep = b + 64u * u + lane < fill && !share;
+                        const uint64_t m = __ballot(keep);
+                        if (keep) {
+                            const uint32_t slot = f + (uint32_t)__popcll(m & lanes_below());
+                            sb[slot].x = p[u].x;
+                            sb[slot].y = p[u].y;
+                        }
+                        f += (uint32_t)__popcll(m);
+                    }
+                }
+            }
+            if (f) stage_flush(sink, ovf, sb, sf, f, ~0ull);
+            fill = 0;
+        };
+        auto emit = [&](bool hit, int32_t j) {  // room for 64 pairs is the caller's business
+            const uint64_t m = __ballot(hit);
+            if (m == 0ull) return;
+            if (hit) {
+                const uint32_t slot = fill + (uint32_t)__popcll(m & lanes_below());
+                sb[slot].x = q;
+                sb[slot].y = j;
+            }
+            fill += (uint32_t)__popcll(m);
+        };
+        // tests the first k (<= 64) of the leaves reached, four loaded at a time
+        auto test_leaves = [&](uint32_t k) {
+            const int32_t cv = (int32_t)cand[min((uint32_t)lane, k - 1u)];
+            for (uint32_t c = 0; c < k; c += 4) {
+                if (fill > kGroupStage - 256u) flush();
+                float4 lo[4], hi[4];
+                int32_t j[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    j[u] = __builtin_amdgcn_readlane(cv, (int)(c + u));
+                    const_float4* r = (const_float4*)(uintptr_t)&d.leaf[j[u]];
+                    lo[u] = make_float4(r[0].x, r[0].y, r[0].z, r[0].w);
+                    hi[u] = make_float4(r[1].x, r[1].y, r[1].z, r[1].w);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    emit(c + u < k && j[u] > after && (!BATCH || j[u] <= last) && box_overlap(qb, lo[u], hi[u]), j[u]);
+            }
+        };
+        uint32_t top = 1, ncand = 0;  // wave-uniform
+        if (lane == 0) stk[0] = (uint32_t)d.leaf_lca[0];
+        // every node enters the stack at most once; the bound only guards against a corrupted tree
+        // (flag 16, reported as a device error, instead of a hang)
+        const int64_t limit = 2 * d.maxT + 16;
+        for (int64_t round = 0; top > 0; ++round) {
+            if (round > limit) {
+                if (lane == 0) atomicOr(ovf, 16u);
+                break;
+            }
+            const uint32_t take = max(1u, min(min(top, 64u), kGroupStack - top));
+            top -= take;
+            const bool act = (uint32_t)lane < take;
+            const int32_t e = act ? (int32_t)stk[top + lane] : 0, nd = e >> 1;
+            const bool leaf = e & 1;
+            bool hit = false;
+            float4 hi = make_float4(0.f, 0.f, 0.f, 0.f);
+            int4 tp = make_int4(0, 0, 0, 0);
+            if (act) {
+                const NodeRec* r = leaf ? &d.leaf[nd] : &d.inode[nd];
+                const float4 lo = r->lo;
+                hi = r->hi;
+                if (!leaf) tp = d.itopo[nd];
+                ++visits;
+                const int32_t begin = leaf ? nd : f2i(lo.w), end = leaf ? nd : tp.w;  // its leaves
+                bool any = false;
+#pragma unroll
+                for (int c = 0; c < kGroupPieces; ++c) any |= box_overlap(piece[c], lo, hi);
+                hit = any && end > g0 && (!BATCH || begin <= glast);
+            }
+            const uint64_t mi = __ballot(hit && !leaf), ml = __ballot(hit && leaf);
+            if (mi) {
+                const uint32_t slot = top + 2u * (uint32_t)__popcll(mi & lanes_below());
+                const bool fits = slot + 2u <= kGroupStack;
+                if (hit && !leaf && fits) {
+                    stk[slot] = (uint32_t)tp.x;
+                    stk[slot + 1] = (uint32_t)tp.y;
+                }
+                const uint64_t mf = __ballot(hit && !leaf && fits);
+                top += 2u * (uint32_t)__popcll(mf);
+                // no room (only a full stack's last item, see `take`): the lanes walk that subtree
+                for (uint64_t over = mi & ~mf; over; over &= over - 1ull) {
+                    const int src = __ffsll((long long)over) - 1;
+                    const int32_t stop = __builtin_amdgcn_readlane(f2i(hi.w), src);
+                    int32_t cur = valid ? __builtin_amdgcn_readlane(tp.x, src) : stop;
+                    int64_t steps = 0;
+                    while (__ballot(cur != stop) != 0ull) {
+                        if (++steps > limit) {
+                            if (lane == 0) atomicOr(ovf, 16u);
+                            break;
+                        }
+                        if (fill > kGroupStage - 256u) flush();
+                        bool h = false;
+                        int32_t j = 0;
+                        if (cur != stop) {
+                            const int32_t x = cur >> 1;
+                            const NodeRec* r = (cur & 1) ? &d.leaf[x] : &d.inode[x];
+                            const float4 a = r->lo, b = r->hi;
+                            const bool o = box_overlap(qb, a, b);
+                            ++visits;
+                            if ((cur & 1) || !o) {
+                                h = (cur & 1) && o && x > after && (!BATCH || x <= last);
+                                j = x;
+                                cur = f2i(b.w);
+                            } else {
+                                cur = d.itopo[x].x;
+                            }
+                        }
+                        emit(h, j);
+                    }
+                }
+            }
+            if (ml) {
+                if (hit && leaf) cand[ncand + (uint32_t)__popcll(ml & lanes_below())] = (uint32_t)nd;
+                ncand += (uint32_t)__popcll(ml);
+            }
+            if (ncand >= 64u || (top == 0u && ncand > 0u)) {
+                test_leaves(min(ncand, 64u));
+                const uint32_t rest = ncand > 64u ? ncand - 64u : 0u;
+                const uint32_t v = (uint32_t)lane < rest ? cand[64 + lane] : 0u;
+                if ((uint32_t)lane < rest) cand[lane] = v;
+                ncand = rest;
+                if (top == 0u && ncand > 0u) {  // the last round's overhang
+                    test_leaves(ncand);
+                    ncand = 0;
+                }
+            }
+        }
+        flush();
+    }
+    add_visits(d, visits);
+}
+
+// Workgroups of k_group_cd, one group per wave: the same number for each XCD's share.
+static unsigned group_grid(int32_t n) {
+    const unsigned share = (((unsigned)n + 63u) / 64u + kXcds - 1) / kXcds;
+    return kXcds * ((share + kWaves - 1) / kWaves);
+}
+
 // Queries of a traversal: the leaves before the last one (self-CD) or the other object's leaves.
 static int64_t query_count(const DevState& d, int32_t n) { return d.inter ? d.nq : n - 1; }
+
+// Self-CD over boxes made from the vertices.
+static bool group_ok(const DevState& d) { return !d.inter && !d.pbox; }
 
 void launch_pure_cd(DevState& d, int32_t n, hipStream_t s) {
     reset_step_counters(d, s);
     const int64_t nq = query_count(d, n);
-    if (nq > 0)
+    if (group_ok(d) && nq > 0)
+        hipLaunchKernelGGL(k_group_cd<false>, dim3(group_grid(n)), dim3(kBlock), 0, s, n, d, nullptr, nullptr);
+    else if (nq > 0)
         hipLaunchKernelGGL(k_traverse<false>, dim3(grid_for(nq)), dim3(kBlock), 0, s, n, d, null_sink(), null_sink());
 }
 
 // ---------------------------------------------------------------- batched scenes
 // Self-CD over many scenes in one tree: the sort keys carry the scene id above the 30 Morton
-// bits, so every scene is one subtree and its leaves are contiguous. Query x of the scene whose
-// last leaf is b walks the leaves (x, b] only: from lca[x + 1] to that subtree's escape
-// lca[b + 1]. Persistent: each wave takes 64 queries at a time from a global counter until
-// all are taken (uneven scenes and uneven per-query work balance themselves).
-__global__ void __launch_bounds__(kBlock) k_batch_cd(int32_t n, DevState d, const uint64_t* __restrict__ keys,
-                                                     const int32_t* __restrict__ scene_last, uint32_t* queue) {
-    __shared__ StagesBP st;
-    stages_init(st);
-    const Out out = make_out(st, d);
-    const int lane = lane_id();
-    uint32_t v = 0;
-    for (;;) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(queue, 64u);
-        base = __shfl(base, 0);
-        if (base >= (uint32_t)n) break;  // wave-uniform exit: the queue is drained
-        const int32_t x = (int32_t)(base + lane);
-        if (x < n) {
-            const int32_t last = scene_last[(int32_t)(keys[x] >> 30)];
-            if (x < last) {
-                const float4 lo = d.leaf[x].lo, hi = d.leaf[x].hi;
-                v += stackless<false>(d, out, x, rec_box(lo, hi), f2i(hi.w), d.leaf_lca[last + 1]);
-            }
-        }
-    }
-    out.pair_final();
-    add_visits(d, v);
-}
-
-// Counters are cleared with kernels (no memset nodes) so that the sequence can be captured in
-// a graph; `grid` workgroups stay resident and drain the query queue.
-void launch_batch_cd(DevState& d, int32_t n, const uint64_t* keys, const int32_t* scene_last, uint32_t* queue,
-                     unsigned grid, hipStream_t s) {
+// bits, so every scene is one subtree and its leaves are contiguous; query x of the scene whose
+// last leaf is b is paired with the leaves (x, b] only. At most `grid` workgroups, each taking
+// groups of its XCD's share in turn. Counters are cleared with a kernel (no memset nodes) so that
+// the sequence can be captured in a graph.
+void launch_batch_cd(DevState& d, int32_t n, const uint64_t* keys, const int32_t* scene_last, unsigned grid,
+                     hipStream_t s) {
     reset_step_counters(d, s);
-    fill_u32(queue, 1, 0u, s);
-    if (n >= 2) hipLaunchKernelGGL(k_batch_cd, dim3(grid), dim3(kBlock), 0, s, n, d, keys, scene_last, queue);
+    const unsigned g = std::min(group_grid(n), kXcds * std::max(grid / kXcds, 1u));
+    if (n >= 2) hipLaunchKernelGGL(k_group_cd<true>, dim3(g), dim3(kBlock), 0, s, n, d, keys, scene_last);
 }
 
 // ---------------------------------------------------------------- ordering
@@ -1297,7 +1550,7 @@ __device__ inline uint32_t desc_test(const DevState& d, const Out& out, lds_int2
     out.pair_push(emit, make_int2(q, nd));
     int4 tp = make_int4(0, 0, 0, 0);
     if (int_hit) tp = d.itopo[nd];
-    const int32_t lc = (tp.x << 1) | (tp.w & 1), rc = (tp.y << 1) | ((tp.w >> 1) & 1);
+    const int32_t lc = tp.x, rc = tp.y;
     const bool ok_l = desc_push(stk, top, int_hit, q, lc);
     const bool ok_r = desc_push(stk, top, int_hit, q, rc);
     if (int_hit && !(ok_l && ok_r)) {  // no room: walk what did not fit here (one call site)
@@ -1427,7 +1680,7 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
             const bool desc = internal && hit;
             int4 tp = make_int4(0, 0, 0, 0);
             if (desc) tp = d.itopo[nd[u]];
-            const int32_t lc = (tp.x << 1) | (tp.w & 1), rc = (tp.y << 1) | ((tp.w >> 1) & 1);
+            const int32_t lc = tp.x, rc = tp.y;
             const bool ok_l = desc_push(stk, stop, desc, q[u], lc);
             const bool ok_r = desc_push(stk, stop, desc, q[u], rc);
             if (desc && !(ok_l && ok_r)) {  // no room on the stack: this lane walks the subtree

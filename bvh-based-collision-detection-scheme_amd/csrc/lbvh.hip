@@ -557,7 +557,8 @@ __global__ void __launch_bounds__(kBlock) k_write_internal(int32_t n, const int3
     d.int_rc[id] = rc;
     d.int_par[id] = par;
     d.int_mark[id] = mark;
-    d.itopo[id] = make_int4(lc, rc, par, (int32_t)mark);
+    d.itopo[id] = make_int4((lc << 1) | (lleaf ? 1 : 0), (rc << 1) | (rleaf ? 1 : 0), par * 2 + ((mark & 4u) ? 1 : 0),
+                            s_b[k]);
     d.int_rx[id] = s_a[k];
     d.int_ry[id] = s_b[k];
     d.inode[id].lo.w = i2f(s_a[k]);
@@ -748,7 +749,7 @@ __global__ void __launch_bounds__(kBlock) k_rp_starts(int32_t n, DevState d) {
             for (; q >= 0 && depth < kDepthCap - 1; q = d.int_par[q]) ++depth;
             if (q >= 0) atomicOr(d.rp_tdeep, 1u);
             const int4 tp = d.itopo[x];
-            e = make_int4(x, tp.x, tp.y, depth | ((tp.w & 1) << 16) | ((tp.w & 2) << 17));
+            e = make_int4(x, tp.x >> 1, tp.y >> 1, depth | ((tp.x & 1) << 16) | ((tp.y & 1) << 18));
         }
     }
     const uint32_t slot = wave_append(d.rp_tcount, top);
@@ -778,9 +779,9 @@ __global__ void __launch_bounds__(kBlock) k_rp_walk(int32_t n, DevState d) {
     int32_t q = p;
     for (int32_t i = 0; i < len && d.int_rx[q] == x; ++i) {
         const int4 tp = d.itopo[q];
-        const int32_t rs = ((tp.w & 2) ? tp.y : d.int_rx[tp.y]) - cs;
+        const int32_t rs = ((tp.y & 1) ? tp.y >> 1 : d.int_rx[tp.y >> 1]) - cs;
         d.rp_ent[q - r + a] = make_int2(q, rp_pack(own, rs, len - 1 - i));
-        q = tp.z;
+        q = tp.z >> 1;
     }
 }
 
@@ -833,9 +834,9 @@ __global__ void __launch_bounds__(kBlock) k_rp_chunk_sort(DevState d) {
             int32_t dest = -1;
             // rp_tpos holds positions only when the top tree has a list (seg_end > 0); deep
             // top trees merged by climbing never write it
-            if (seg_end > 0 && tp.z >= 0 && d.rp_tpos[tp.z] < seg_end) {
-                const int4 pe = d.rp_tlist[d.rp_tpos[tp.z]];
-                dest = (tp.w & 4) ? pe.z : pe.y;
+            if (seg_end > 0 && tp.z >= 0 && d.rp_tpos[tp.z >> 1] < seg_end) {
+                const int4 pe = d.rp_tlist[d.rp_tpos[tp.z >> 1]];
+                dest = (tp.z & 1) ? pe.z : pe.y;
             }
             d.rp_ent[pos + roots] = make_int2(dest, 0);
         }
@@ -987,7 +988,7 @@ __global__ void __launch_bounds__(kTopBlock) k_rp_top_segments(DevState d, int32
     for (int32_t lev = 0; lev <= top; ++lev) {
         const int32_t b0 = ls[lev], b1 = lev > 0 ? ls[lev - 1] : m;
         for (int32_t i = b0 + (int32_t)threadIdx.x; i < b1; i += kTopBlock) {
-            const int32_t par = d.itopo[d.rp_tlist[i].x].z;  // the parent of a top node is a top node
+            const int32_t par = d.itopo[d.rp_tlist[i].x].z >> 1;  // the parent of a top node is a top node
             const int32_t pi = par >= 0 ? d.rp_tpos[par] : -1;
             int32_t sid = -1;
             if (ts[i] <= kTopLds) sid = (pi < 0 || ts[pi] > kTopLds) ? (int32_t)atomicAdd(&nseg, 1u) : sg[pi];
@@ -1274,12 +1275,12 @@ __device__ inline void refit_top_climb(const DevState& d, int32_t m) {
         store_box(&d.inode[e.x], b);
         for (int32_t q = e.x;;) {
             const int4 tq = d.itopo[q];
-            const int32_t u = tq.z;
+            const int32_t u = tq.z >> 1;
             if (u < 0) break;
             const int4 tu = d.itopo[u];
-            const bool right = (tq.w & 4) != 0;  // q is u's right child
-            const int32_t sib = right ? tu.x : tu.y;
-            const int sk = (right ? (tu.w & 1) : (tu.w & 2)) ? 1 : 0;
+            const bool right = (tq.z & 1) != 0;  // q is u's right child
+            const int32_t se = right ? tu.x : tu.y, sib = se >> 1;
+            const int sk = se & 1;
             if (sk == 0 && rp_is_top(d, sib)) {
                 if (__hip_atomic_fetch_add(&flag[u], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) break;
                 flag[u] = 0;

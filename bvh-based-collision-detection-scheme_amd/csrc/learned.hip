@@ -321,7 +321,7 @@ int learned_forward_noalloc(LearnedState* L, int device, const float* feats, int
 //    stride 68: writes and reads free of bank conflicts).
 // Each workgroup leaves its sums in `part` (kGradStride words), which k_train_finish adds up in a
 // fixed order: repeated runs give the same bits. Bound by MFMA issue and the launch itself:
-// 49,061 rows take 0.03 ms. (One thread per row, adding each of its 5313 gradients to the
+// 49,061 rows take 0.042 ms. (One thread per row, adding each of its 5313 gradients to the
 // workgroup's LDS sums, took 19.5 ms: all 64 lanes added to one LDS word at a time.)
 constexpr int kTrainBlock = 256;
 constexpr int kTrainWaves = kTrainBlock / 64;

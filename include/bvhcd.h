@@ -313,7 +313,7 @@ int  bvhcd_batch_destroy(bvhcd_batch* b);
 int  bvhcd_batch_set_topology(bvhcd_batch* b, const int32_t* faces, int where);
 /* xyz: concatenated per-scene vertices; host memory may be reused when the call returns. */
 int  bvhcd_batch_update_vertices(bvhcd_batch* b, const float* xyz, int where);
-/* One frame for every scene: bvh_op BUILD or REFIT, then the persistent self-CD traversal,
+/* One frame for every scene: bvh_op BUILD or REFIT, then the self-CD traversal,
    the narrow phase and the per-scene grouping of the hits. use_graph = 1: the frame is captured
    in a hipGraph on first use (one graph per bvh_op) and replayed afterwards. */
 int  bvhcd_batch_step(bvhcd_batch* b, int bvh_op, int use_graph);
@@ -344,7 +344,7 @@ int  bvhcd_autotune_set(int kernel, int64_t n, uint32_t grid, uint32_t unroll);
    for the batched traversal (CudaDevice::evalOptimalBlockSize, CudaDevice.cu:60-83, picks a
    block size per kernel; bvhcd_autotune_set keeps 256). */
 int  bvhcd_autotune_set_block(int kernel, int64_t n, uint32_t grid, uint32_t unroll, uint32_t block);
-/* The persistent batched traversal; drops the captured frame graphs (re-captured on next use). */
+/* The batched traversal; drops the captured frame graphs (re-captured on next use). */
 int  bvhcd_batch_autotune(bvhcd_batch* b);
 /* Text table of every timed candidate (kernel, size class, grid, ms, chosen); returns its
    length (copies at most cap - 1 bytes plus a terminator). */

@@ -670,3 +670,45 @@ def test_full_spheres_sequence_digests(pkg, oracle):
         restr += ctx.stats()["last_bvh_op"] == pkg.BVH_RESTRUCTURE
     print(f"[gpu] spheres restructure frames: {restr}", flush=True)
     ctx.close()
+
+
+def _soup(kind, T, rng):
+    """Faces and vertices of T triangles: `soup` spread with jumps between far clusters, `stack` all on
+    one spot (every box overlaps every other), `mesh` a strip sharing vertices, `bad` a soup with
+    infinities, NaN and one triangle of NaN alone."""
+    if kind == "mesh":
+        x = np.arange(T + 2)
+        v = np.stack([x * 0.1, (x % 2) * 0.1, 0.02 * np.sin(x)], 1)
+        return np.stack([x[:-2], x[1:-1], x[2:]], 1).astype(np.int32), v.astype(np.float32)
+    c = rng.integers(0, 3, (T, 1)) * 40.0 + rng.random((T, 3)) * (T ** (1 / 3)) * 0.5
+    if kind == "stack":
+        c[:] = 0.0
+    v = (c[:, None] + rng.random((T, 3, 3))).reshape(-1, 3).astype(np.float32)
+    if kind == "bad":
+        v[3 * (T // 2):3 * (T // 2) + 3] = np.nan
+        v[0, 1], v[-1, 2], v[3 * (T // 3), 0] = np.inf, -np.inf, np.nan
+    return np.arange(3 * T, dtype=np.int32).reshape(-1, 3), v
+
+
+@pytest.mark.parametrize("skip_adjacent", [False, True])
+@pytest.mark.parametrize("kind,T", [("soup", 1), ("soup", 2), ("mesh", 63), ("mesh", 64), ("soup", 65), ("mesh", 511),
+                                    ("soup", 513), ("bad", 700), ("mesh", 20011), ("soup", 50021), ("stack", 4097)])
+def test_pure_traversal_equals_front_walk(pkg, oracle, kind, T, skip_adjacent):
+    """The traversal of 64 queries at a time against the queries' own walks (GENERATE) on the same
+    trees: sizes around a wave's 64 queries and a workgroup's 256, clusters that make runs of queries
+    jump, every box overlapping every other (the node stack at its limit), infinities and NaN."""
+    print(f"[gpu] pure traversal against walks: {kind} {T} skip {skip_adjacent}", flush=True)
+    faces, v = _soup(kind, T, np.random.default_rng(T))
+    cap = T * T // 2 + 1024 if kind == "stack" else 64 * T + 4096
+    ctx = pkg.CollisionContext(T, len(v), int_front_cap=cap, ext_front_cap=cap, pair_cap=cap,
+                               skip_adjacent=skip_adjacent)
+    ctx.set_topology(faces, len(v))
+    moved = (v + np.random.default_rng(1).normal(0, 0.02, v.shape)).astype(np.float32)
+    for xyz, op in ((v, pkg.BVH_BUILD), (moved, pkg.BVH_REFIT)):
+        ctx.update_vertices(xyz)
+        ctx.step(op, pkg.FRONT_PURE_BVH_CD)
+        got = {f: oracle.pair_set(ctx.pairs(f)) for f in (False, True)}
+        ctx.step(pkg.BVH_NONE, pkg.FRONT_GENERATE)
+        for f in (False, True):
+            np.testing.assert_array_equal(got[f], oracle.pair_set(ctx.pairs(f)), err_msg=f"{op} filtered {f}")
+    ctx.close()
