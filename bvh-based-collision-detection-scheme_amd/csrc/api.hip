@@ -28,6 +28,12 @@ constexpr int kLog = 8;   // device log words per frame
 // check.
 constexpr double kLearnedCapacityShare = 0.75;
 constexpr int kLearnedMaxBackoff = 3;
+// Host vertices and host read-outs of up to these sizes go through pinned buffers of the context: the
+// upload is then one queued copy and the read-out a kernel writing host memory, where a copy of
+// pageable memory costs a round trip each (2,560 triangles, vertices in and pairs out: 226 -> 132 us
+// a frame with the totals read the same way). Larger ones gain nothing: the copy itself dominates.
+constexpr size_t kStageBytes = 1u << 20;
+constexpr int64_t kHostPairs = 1 << 16;
 }  // namespace
 
 struct bvhcd_ctx {
@@ -70,6 +76,10 @@ struct bvhcd_ctx {
     double rebuild_ms = -1.0;    // ms of the last rebuild frame (BUILD + GENERATE)
     bool rebuild_timed = false;  // the last step was a rebuild whose time is still to be read
     bool totals_pending = false; // pair totals of the last step not summed yet (done on demand)
+    bool hres_valid = false;     // d.hres holds the last step's totals (reset by every change)
+    float* stage[2] = {nullptr, nullptr};  // pinned: host uploads of up to kStageBytes
+    hipEvent_t staged[2] = {nullptr, nullptr};  // the copy out of each stage is done
+    int2* hpairs = nullptr;      // pinned: read-outs of up to kHostPairs pairs
     bool step_zeroed = false;    // this step's refit zeroed the step counters for its KEEP
 };
 
@@ -314,6 +324,25 @@ void ensure_totals(bvhcd_ctx* c) {
     c->totals_pending = false;
 }
 
+// The last step's totals and overflow flags in d.hres: one launch and one synchronisation, nothing
+// when they are there already.
+int read_totals(bvhcd_ctx* c) {
+    if (c->hres_valid) return BVHCD_OK;
+    launch_pair_totals(c->d, c->stream, c->cfg.narrow_phase != 0);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->totals_pending = false;
+    c->hres_valid = true;
+    return BVHCD_OK;
+}
+
+// Pinned buffer, made on first use and freed with the context (null: no memory for it).
+template <class T>
+T* pinned(T*& p, size_t n) {
+    void* q = nullptr;
+    if (!p && hipHostMalloc(&q, n * sizeof(T), hipHostMallocDefault) == hipSuccess) p = static_cast<T*>(q);
+    return p;
+}
+
 void log_frame(bvhcd_ctx* c, int bvh_op, int front_op) {
     if (!timing_on(c)) return;
     ensure_totals(c);
@@ -362,6 +391,17 @@ void frame_bytes(double T, double V, int bvh_op, int front_op, double visits, do
     double tot = 0;
     for (int i = 0; i < 7; ++i) tot += out[i];
     out[S_TOTAL] = tot;
+}
+
+// Host vertices of this size go through the pinned stages (bvhcd_update_vertices).
+bool staged_upload(const bvhcd_ctx* c) { return sizeof(float) * 3 * (size_t)c->V <= kStageBytes; }
+// Once kernels that read an own vertex buffer are enqueued, the next upload into that buffer on the
+// copy stream must wait for them, also when a later part of the step fails. (Staged uploads are
+// ordered by the context stream, and the size class only changes with the topology, whose call waits
+// for the stream.)
+void mark_consumed(bvhcd_ctx* c) {
+    if (!staged_upload(c) && (c->d.verts == c->own_verts || c->d.verts == c->own_verts2))
+        (void)hipEventRecord(c->consumed[c->d.verts == c->own_verts2 ? 1 : 0], c->stream);
 }
 
 // ---------------------------------------------------------------- BVH maintenance
@@ -580,6 +620,7 @@ int run_front(bvhcd_ctx* c, int& front_op) {
     // segment counters (without a narrow phase they stay zero)
     if (c->cfg.narrow_phase) launch_narrow(d, s, true);
     c->totals_pending = true;
+    c->hres_valid = false;
     end(c, S_NARROW);
     return BVHCD_OK;
 }
@@ -627,19 +668,13 @@ int do_step(bvhcd_ctx* c, int bvh_op, int front_op) {
     begin(c, S_TOTAL);
     bool topo = false;
     c->step_zeroed = false;
-    // Once kernels that read an own vertex buffer are enqueued, the next host upload into that
-    // buffer must wait for them, also when a later part of the step fails.
-    auto mark_consumed = [c]() {
-        if (c->d.verts == c->own_verts || c->d.verts == c->own_verts2)
-            (void)hipEventRecord(c->consumed[c->d.verts == c->own_verts2 ? 1 : 0], c->stream);
-    };
     int st = run_bvh(c, bvh_op, topo);
-    if (st) { mark_consumed(); return st; }
+    if (st) { mark_consumed(c); return st; }
     if (topo) c->front_valid = false;
     st = run_front(c, front_op);
     c->step_zeroed = false;
     if (!st && c->cfg.auto_grow) st = grow_and_retry(c, front_op);
-    mark_consumed();
+    mark_consumed(c);
     if (st) return st;
     end(c, S_TOTAL);
     c->last_bvh = bvh_op;
@@ -696,10 +731,7 @@ void plain_schedule(int sched, int64_t f, int bc, int fc, int& bvh_op, int& fron
     }
 }
 
-int check_overflow(bvhcd_ctx* c) {
-    uint32_t ovf = 0;
-    HIPCHK(c, hipMemcpyAsync(&ovf, c->d.ctr + C_OVF, sizeof(ovf), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+int overflow_status(bvhcd_ctx* c, uint32_t ovf) {
     if (ovf) {
         char buf[160];
         if (ovf & 16u) return fail(c, BVHCD_E_DEVICE, "traversal step bound exceeded (corrupted tree)");
@@ -708,6 +740,12 @@ int check_overflow(bvhcd_ctx* c) {
         return fail(c, BVHCD_E_CAPACITY, buf);
     }
     return BVHCD_OK;
+}
+int check_overflow(bvhcd_ctx* c) {
+    uint32_t ovf = 0;
+    HIPCHK(c, hipMemcpyAsync(&ovf, c->d.ctr + C_OVF, sizeof(ovf), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return overflow_status(c, ovf);
 }
 
 void timing_free(bvhcd_ctx* c) {
@@ -734,7 +772,15 @@ void release_upload(bvhcd_ctx* c) {
         if (c->copied[b]) (void)hipEventDestroy(c->copied[b]);
         if (c->consumed[b]) (void)hipEventDestroy(c->consumed[b]);
         c->copied[b] = c->consumed[b] = nullptr;
+        if (c->staged[b]) (void)hipEventDestroy(c->staged[b]);
+        if (c->stage[b]) (void)hipHostFree(c->stage[b]);
+        c->staged[b] = nullptr;
+        c->stage[b] = nullptr;
     }
+    if (c->hpairs) (void)hipHostFree(c->hpairs);
+    if (c->d.hres) (void)hipHostFree(c->d.hres);
+    c->hpairs = nullptr;
+    c->d.hres = nullptr;
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
     c->copy_stream = nullptr;
 }
@@ -775,6 +821,7 @@ int bvhcd_create(const bvhcd_config* cfg, bvhcd_ctx** out) {
         ok &= hipEventCreateWithFlags(&c->consumed[b], hipEventDisableTiming) == hipSuccess;
         ok &= ok && hipEventRecord(c->consumed[b], c->stream) == hipSuccess;
     }
+    ok = ok && pinned(c->d.hres, H_SCENES);
     if (!ok) {
         release_upload(c);
         free_all(c);
@@ -828,6 +875,7 @@ int bvhcd_set_topology(bvhcd_ctx* c, const int32_t* faces, int64_t T, int64_t V,
     c->T = T;
     c->V = V;
     c->built = c->front_valid = c->restr_pending = c->learned_frame = c->repair_pending = false;
+    c->hres_valid = false;
     c->keep_base = -1.0;
     c->keep_excess = 0.0;
     c->rebuild_ms = -1.0;
@@ -858,11 +906,23 @@ int bvhcd_update_vertices(bvhcd_ctx* c, const float* xyz, int64_t V, int where) 
         HIPCHK(c, hipMemcpyAsync(c->d.verts, xyz, sizeof(float) * 3 * V, hipMemcpyDeviceToDevice, c->stream));
         return BVHCD_OK;
     }
-    // Host memory: the upload goes on the copy stream into the buffer the latest step did not
-    // read (once the step before it, which did, is done), so it overlaps the steps still
-    // running; the call returns when the copy is complete (the caller may reuse xyz).
+    // Small host uploads: into a pinned stage, then one copy on the context stream, which the call does
+    // not wait for (xyz may be reused at once; a stage is written again once its last copy is done).
     const int b = c->vbuf ^ 1;
     float* dst = b ? c->own_verts2 : c->own_verts;
+    if (staged_upload(c) && pinned(c->stage[b], std::min<size_t>(3 * (size_t)c->d.maxV, kStageBytes / sizeof(float)))) {
+        if (!c->staged[b]) HIPCHK(c, hipEventCreateWithFlags(&c->staged[b], hipEventDisableTiming));
+        else HIPCHK(c, hipEventSynchronize(c->staged[b]));
+        std::memcpy(c->stage[b], xyz, sizeof(float) * 3 * V);
+        HIPCHK(c, hipMemcpyAsync(dst, c->stage[b], sizeof(float) * 3 * V, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, hipEventRecord(c->staged[b], c->stream));
+        c->vbuf = b;
+        c->d.verts = dst;
+        return BVHCD_OK;
+    }
+    // Larger ones: the upload goes on the copy stream into the buffer the latest step did not
+    // read (once the step before it, which did, is done), so it overlaps the steps still
+    // running; the call returns when the copy is complete (the caller may reuse xyz).
     HIPCHK(c, hipStreamWaitEvent(c->copy_stream, c->consumed[b], 0));
     HIPCHK(c, hipMemcpyAsync(dst, xyz, sizeof(float) * 3 * V, hipMemcpyHostToDevice, c->copy_stream));
     HIPCHK(c, hipEventRecord(c->copied[b], c->copy_stream));
@@ -974,25 +1034,42 @@ int bvhcd_step_scheduled(bvhcd_ctx* c) {
 
 int bvhcd_get_pairs(bvhcd_ctx* c, int32_t* out, int64_t cap, int64_t* num, int where, int filtered) {
     if (!c || !num) return BVHCD_E_INVALID;
-    ensure_totals(c);
-    uint32_t cnt = 0;
-    HIPCHK(c, hipMemcpyAsync(&cnt, c->d.ctr + (filtered ? C_NP : C_BP), sizeof(cnt), hipMemcpyDeviceToHost, c->stream));
-    int st = check_overflow(c);
-    *num = cnt;
+    const int kind = filtered ? 1 : 0;
+    // into a device buffer: totals and pairs in one launch, one synchronisation for both
+    const bool fused = where == BVHCD_MEM_DEVICE && out && cap > 0 && !c->hres_valid;
+    if (fused)
+        launch_totals_and_gather(c->d, kind, reinterpret_cast<int2*>(out), cap, c->cfg.narrow_phase != 0, c->stream);
+    if (fused) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        c->totals_pending = false;
+        c->hres_valid = true;
+    }
+    int st = read_totals(c);
     if (st) return st;
+    const volatile uint32_t* res = c->d.hres;
+    const uint32_t cnt = res[kind ? H_NP : H_BP];
+    *num = cnt;
+    st = overflow_status(c, res[H_OVF]);
+    if (st || fused) return st;
     if (out && cap > 0) {
         const int64_t k = std::min<int64_t>(cap, cnt);
         if (k > 0) {
             // segments, then the implicit shared-vertex pairs, gathered (leaf ids mapped to
-            // triangle ids) straight into a device buffer, or through the read-out buffer to the
-            // host in pieces of its size (implicit pairs are not stored, so the total can exceed it)
+            // triangle ids) straight into a device buffer, or through a pinned or the read-out buffer
+            // to the host, in pieces of its size (implicit pairs are not stored, so the total can
+            // exceed it)
             if (where == BVHCD_MEM_DEVICE) {
-                launch_pair_gather(c->d, filtered ? 1 : 0, reinterpret_cast<int2*>(out), 0, k, c->stream);
+                launch_pair_gather(c->d, kind, reinterpret_cast<int2*>(out), 0, k, c->stream);
+            } else if (k <= kHostPairs && pinned(c->hpairs, kHostPairs)) {
+                launch_pair_gather(c->d, kind, c->hpairs, 0, k, c->stream);
+                HIPCHK(c, hipStreamSynchronize(c->stream));
+                std::memcpy(out, c->hpairs, sizeof(int2) * k);
+                return BVHCD_OK;
             } else {
                 const int64_t piece = std::max<int64_t>(1, c->d.pair_cap);
                 for (int64_t first = 0; first < k; first += piece) {
                     const int64_t m = std::min<int64_t>(piece, k - first);
-                    launch_pair_gather(c->d, filtered ? 1 : 0, c->d.pair_tmp, first, m, c->stream);
+                    launch_pair_gather(c->d, kind, c->d.pair_tmp, first, m, c->stream);
                     HIPCHK(c, hipMemcpyAsync(out + 2 * first, c->d.pair_tmp, sizeof(int2) * m, hipMemcpyDeviceToHost,
                                              c->stream));
                     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1348,6 +1425,7 @@ int bvhcd_autotune(bvhcd_ctx* c) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     // leave a consistent result: the current front's pairs and their narrow phase
+    c->hres_valid = false;
     launch_keep(d, n, c->stream);
     if (c->cfg.narrow_phase) launch_narrow(d, c->stream);
     else clear_np(d, c->stream);
@@ -1407,6 +1485,7 @@ int bvhcd_restructure(bvhcd_ctx* c, const int32_t* roots, int64_t k) {
     c->tcap = tcap;
     if (st) return st;
     c->restr_pending = false;
+    c->hres_valid = false;
     return check_overflow(c);
 }
 
@@ -1482,6 +1561,7 @@ DevState inter_view(bvhcd_inter* x) {
     v.pair_seg_cap = o.pair_seg_cap;
     v.pcnt = o.pcnt;
     v.ctr = o.ctr;
+    v.hres = x->rigid->d.hres;  // the second object's own: it reports no pairs itself
     v.skip_adj = 0;
     v.inter = 1;
     v.fchunk[0] = v.fchunk[1] = nullptr;  // inter fronts are sorted by query after production
@@ -1510,14 +1590,17 @@ void inter_keep_view(bvhcd_inter* x, const DevState& v) {
     o.front_version = v.front_version;
 }
 
+int inter_overflow_status(bvhcd_inter* x, uint32_t ovf) {
+    if (ovf & 16u) return ifail(x, BVHCD_E_DEVICE, "traversal step bound exceeded (corrupted tree)");
+    if (ovf) return ifail(x, BVHCD_E_CAPACITY, "inter front or pair capacity exceeded");
+    return BVHCD_OK;
+}
 int inter_check_overflow(bvhcd_inter* x) {
     uint32_t ovf = 0;
     hipStream_t s = x->def->stream;
     IHIPCHK(x, hipMemcpyAsync(&ovf, x->own.ctr + C_OVF, sizeof(ovf), hipMemcpyDeviceToHost, s));
     IHIPCHK(x, hipStreamSynchronize(s));
-    if (ovf & 16u) return ifail(x, BVHCD_E_DEVICE, "traversal step bound exceeded (corrupted tree)");
-    if (ovf) return ifail(x, BVHCD_E_CAPACITY, "inter front or pair capacity exceeded");
-    return BVHCD_OK;
+    return inter_overflow_status(x, ovf);
 }
 
 }  // namespace
@@ -1653,8 +1736,7 @@ int bvhcd_inter_step(bvhcd_inter* x, int rigid_op, int front_op) {
     inter_keep_view(x, v);
     x->last_front = front_op;
     // the next host upload into the querying object's vertex buffer waits for these kernels
-    if (rg->d.verts == rg->own_verts || rg->d.verts == rg->own_verts2)
-        IHIPCHK(x, hipEventRecord(rg->consumed[rg->d.verts == rg->own_verts2 ? 1 : 0], s));
+    mark_consumed(rg);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ifail(x, BVHCD_E_DEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
     return BVHCD_OK;
@@ -1663,15 +1745,21 @@ int bvhcd_inter_step(bvhcd_inter* x, int rigid_op, int front_op) {
 int bvhcd_inter_get_pairs(bvhcd_inter* x, int32_t* out, int64_t cap, int64_t* num, int where, int filtered) {
     if (!x || !num) return BVHCD_E_INVALID;
     hipStream_t s = x->def->stream;
-    uint32_t cnt = 0;
-    IHIPCHK(x, hipMemcpyAsync(&cnt, x->own.ctr + (filtered ? C_NP : C_BP), sizeof(cnt), hipMemcpyDeviceToHost, s));
-    const int st = inter_check_overflow(x);
+    IHIPCHK(x, hipStreamSynchronize(s));  // the step left its totals in pinned host memory
+    const volatile uint32_t* res = x->rigid->d.hres;
+    const uint32_t cnt = x->last_front < 0 ? 0u : res[filtered ? H_NP : H_BP];
+    const int st = x->last_front < 0 ? BVHCD_OK : inter_overflow_status(x, res[H_OVF]);
     *num = cnt;
     if (st || !out || cap <= 0 || cnt == 0) return st;
     DevState v = inter_view(x);
     const int64_t k = std::min<int64_t>(cap, cnt);
     if (where == BVHCD_MEM_DEVICE) {
         launch_pair_gather(v, filtered ? 1 : 0, reinterpret_cast<int2*>(out), 0, k, s);
+    } else if (k <= kHostPairs && pinned(x->rigid->hpairs, kHostPairs)) {
+        launch_pair_gather(v, filtered ? 1 : 0, x->rigid->hpairs, 0, k, s);
+        IHIPCHK(x, hipStreamSynchronize(s));
+        std::memcpy(out, x->rigid->hpairs, sizeof(int2) * k);
+        return BVHCD_OK;
     } else {
         launch_pair_gather(v, filtered ? 1 : 0, v.pair_tmp, 0, k, s);
         IHIPCHK(x, hipMemcpyAsync(out, v.pair_tmp, sizeof(int2) * k, hipMemcpyDeviceToHost, s));

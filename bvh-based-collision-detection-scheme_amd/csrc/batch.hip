@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(kBlock) k_group_count(DevState d, int32_t S, c
     for (int32_t i = threadIdx.x; i < S; i += kBlock) tbl[(int64_t)i * gridDim.x + blockIdx.x] = cnt[i];
 }
 
-// soff[s] = first slot of scene s, soff[S] = hits.
+// soff[s] = first slot of scene s, soff[S] = hits; the same in the host words.
 __global__ void __launch_bounds__(kBlock) k_group_scatter(DevState d, int32_t S, const int32_t* __restrict__ tri_scene,
                                                           const int64_t* __restrict__ toff,
                                                           const uint32_t* __restrict__ tbl,
@@ -249,8 +249,11 @@ __global__ void __launch_bounds__(kBlock) k_group_scatter(DevState d, int32_t S,
     for (int32_t i = threadIdx.x; i < S; i += kBlock) next[i] = tbl[(int64_t)i * gridDim.x + blockIdx.x];
     const uint32_t m = seg_prefix(d.pcnt + kPairSegs * kCntStride, (uint32_t)d.pair_seg_cap, pre);  // holds a barrier
     if (blockIdx.x == 0) {
-        for (int32_t i = threadIdx.x; i < S; i += kBlock) soff[i] = tbl[(int64_t)i * gridDim.x];
-        if (threadIdx.x == 0) soff[S] = m;
+        for (int32_t i = threadIdx.x; i <= S; i += kBlock) {
+            const uint32_t v = i < S ? tbl[(int64_t)i * gridDim.x] : m;
+            soff[i] = v;
+            d.hres[H_SCENES + i] = v;
+        }
     }
     const HitRange r = hit_range(m);
     for (uint32_t k0 = r.begin + (threadIdx.x & ~63u); k0 < r.end; k0 += kBlock) {  // wave-uniform
@@ -344,13 +347,15 @@ void record_frame(bvhcd_batch* b, int bvh_op, unsigned grid) {
                        b->scur, b->grouped);
 }
 
+const volatile uint32_t* host_words(const bvhcd_batch* b) { return b->d.hres; }
+
 unsigned batch_grid(bvhcd_batch* b) { return shape_grid(tuned_shape(TK_BATCH_CD, b->T)); }
 
+// Waits for the last frame and reports its overflow flags. The frame left its totals, flags and (up to
+// kGroupScenes scenes) the scenes' first slots in pinned host words: nothing is copied.
 int check_batch_overflow(bvhcd_batch* b) {
-    uint32_t ovf = 0;
-    if (hipMemcpyAsync(&ovf, b->d.ctr + C_OVF, sizeof(ovf), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
-        hipStreamSynchronize(b->stream) != hipSuccess)
-        return bfail(b, BVHCD_E_DEVICE, "device error");
+    if (hipStreamSynchronize(b->stream) != hipSuccess) return bfail(b, BVHCD_E_DEVICE, "device error");
+    const uint32_t ovf = host_words(b)[H_OVF];
     if (ovf & 16u) return bfail(b, BVHCD_E_DEVICE, "traversal step bound exceeded");
     if (ovf) return bfail(b, BVHCD_E_CAPACITY, "pair capacity exceeded");
     return BVHCD_OK;
@@ -471,10 +476,15 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     ok &= balloc(b, b->keys, T);
     ok &= balloc(b, b->keys_tmp, T);
     ok &= balloc(b, b->scnt, S + 1);
+    void* words = nullptr;
+    ok = ok && hipHostMalloc(&words, sizeof(uint32_t) * (H_SCENES + std::min(S, kGroupScenes) + 1),
+                             hipHostMallocDefault) == hipSuccess;
+    d.hres = static_cast<uint32_t*>(words);
     ok &= balloc(b, b->scur, S + 1);
     ok &= balloc(b, b->gtbl, (size_t)gtbl_n);
     if (!ok) {
         for (void* p : b->allocs) (void)hipFree(p);
+        if (d.hres) (void)hipHostFree(d.hres);
         if (b->own_stream) (void)hipStreamDestroy(b->stream);
         delete b;
         return BVHCD_E_OOM;
@@ -499,6 +509,7 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     }
     if (!okc) {
         for (void* p : b->allocs) (void)hipFree(p);
+        if (d.hres) (void)hipHostFree(d.hres);
         if (b->own_stream) (void)hipStreamDestroy(b->stream);
         delete b;
         return BVHCD_E_DEVICE;
@@ -512,6 +523,7 @@ int bvhcd_batch_destroy(bvhcd_batch* b) {
     (void)hipStreamSynchronize(b->stream);
     drop_graphs(b);
     for (void* p : b->allocs) (void)hipFree(p);
+    if (b->d.hres) (void)hipHostFree(b->d.hres);
     if (b->own_stream) (void)hipStreamDestroy(b->stream);
     delete b;
     return BVHCD_OK;
@@ -590,14 +602,17 @@ int bvhcd_batch_pair_counts(bvhcd_batch* b, int64_t* counts) {
     if (!b->built) return bfail(b, BVHCD_E_NOT_BUILT, "no step yet");
     int st = check_batch_overflow(b);
     if (st) return st;
+    if (b->S <= kGroupScenes) {
+        const volatile uint32_t* off = host_words(b) + H_SCENES;
+        for (int32_t s = 0; s < b->S; ++s) counts[s] = (int64_t)(off[s + 1] - off[s]);
+        return BVHCD_OK;
+    }
     std::vector<uint32_t> off(b->S + 1);
     if (hipMemcpyAsync(off.data(), b->scnt, sizeof(uint32_t) * (b->S + 1), hipMemcpyDeviceToHost, b->stream) !=
             hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)
         return bfail(b, BVHCD_E_DEVICE, "device error");
-    uint32_t total = 0;
-    if (hipMemcpy(&total, b->d.ctr + C_NP, sizeof(total), hipMemcpyDeviceToHost) != hipSuccess)
-        return bfail(b, BVHCD_E_DEVICE, "device error");
+    const uint32_t total = host_words(b)[H_NP];
     for (int32_t s = 0; s < b->S; ++s) counts[s] = (int64_t)((s + 1 < b->S ? off[s + 1] : total) - off[s]);
     return BVHCD_OK;
 }
@@ -611,8 +626,10 @@ int bvhcd_batch_get_pairs(bvhcd_batch* b, int32_t scene, int32_t* out, int64_t c
     if (!out) return BVHCD_OK;
     if (cap < *n) return bfail(b, BVHCD_E_CAPACITY, "output buffer too small");
     uint32_t off = 0;
-    if (hipMemcpy(&off, b->scnt + scene, sizeof(off), hipMemcpyDeviceToHost) != hipSuccess ||
-        (*n > 0 && hipMemcpy(out, b->grouped + off, sizeof(int2) * (size_t)*n, hipMemcpyDeviceToHost) != hipSuccess))
+    if (b->S <= kGroupScenes) off = host_words(b)[H_SCENES + scene];
+    else if (hipMemcpy(&off, b->scnt + scene, sizeof(off), hipMemcpyDeviceToHost) != hipSuccess)
+        return bfail(b, BVHCD_E_DEVICE, "pair copy failed");
+    if ((*n > 0 && hipMemcpy(out, b->grouped + off, sizeof(int2) * (size_t)*n, hipMemcpyDeviceToHost) != hipSuccess))
         return bfail(b, BVHCD_E_DEVICE, "pair copy failed");
     return BVHCD_OK;
 }

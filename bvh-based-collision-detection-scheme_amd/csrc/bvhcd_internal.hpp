@@ -274,6 +274,9 @@ struct DevState {
     uint32_t* pcnt = nullptr;       // [2][kPairSegs * kCntStride]: bp, np segment counts
     // counters block: see Counter enum
     uint32_t* ctr = nullptr;        // 32 words
+    // pinned host words the totals kernels leave a step's results in (HostWord), for the host to read
+    // after one synchronisation and without a copy; null: not wanted
+    uint32_t* hres = nullptr;
     // Queries of the front kernels: the tree's own leaves for self-CD (qleaf = leaf, qprim =
     // prim_idx, each query walking only the leaves after it). An inter-object view (inter = 1)
     // points them at another object's sorted leaves instead, its nq queries each walking the
@@ -313,6 +316,11 @@ enum Counter : int {
     C_WAVE_TOTAL = 27, // wave-ordered production: entries of the list being gathered
     C_WAVE_CHUNKS = 28,// wave-ordered production: chunk records of the list being gathered
     C_NUM = 32
+};
+enum HostWord : int {
+    H_BP = 0, H_NP = 1,  // C_BP, C_NP
+    H_OVF = 2,           // C_OVF
+    H_SCENES = 4         // batched scenes: first slot of every scene, then the number of hits
 };
 enum Counter64 : int {
     C64_VISITS = 0,    // node tests of the last step

@@ -2071,7 +2071,7 @@ void launch_narrow(DevState& d, hipStream_t s, bool counters_zeroed) {
 // took, so an overflowing list reports what it needed) and their largest segment: ctr[C_BP],
 // ctr[C_NP], ctr[C_BP_SEGMAX], ctr[C_NP_SEGMAX]. Implicit (shared-vertex) pairs are added to
 // both totals; with a narrow phase they are hits.
-__global__ void k_pair_totals(DevState d, int narrow) {
+__device__ inline void pair_totals(const DevState& d, int narrow) {  // two waves, one per list
     const int kind = threadIdx.x >> 6, g = lane_id();
     const uint32_t* cnt = d.pcnt + kind * kPairSegs * kCntStride;
     uint32_t v = cnt[g * kCntStride] + (g == 0 ? cnt[kDroppedWord] : 0u), m = cnt[g * kCntStride];
@@ -2082,10 +2082,16 @@ __global__ void k_pair_totals(DevState d, int narrow) {
     if (g == 0) {
         const uint32_t impl = d.ctr[C_IMPLICIT];
         if (kind == 1) d.ctr[C_IMPL_NP] = narrow ? impl : 0u;
-        d.ctr[kind ? C_NP : C_BP] = v + (kind == 0 || narrow ? impl : 0u);
+        const uint32_t total = v + (kind == 0 || narrow ? impl : 0u);
+        d.ctr[kind ? C_NP : C_BP] = total;
         d.ctr[kind ? C_NP_SEGMAX : C_BP_SEGMAX] = m;
+        if (d.hres) {
+            d.hres[kind ? H_NP : H_BP] = total;
+            if (kind == 0) d.hres[H_OVF] = d.ctr[C_OVF];
+        }
     }
 }
+__global__ void k_pair_totals(DevState d, int narrow) { pair_totals(d, narrow); }
 void launch_pair_totals(DevState& d, hipStream_t s, bool narrow) {
     hipLaunchKernelGGL(k_pair_totals, dim3(1), dim3(128), 0, s, d, narrow ? 1 : 0);
 }
@@ -2109,19 +2115,30 @@ __device__ inline int2 list_pair(const DevState& d, int kind, const uint32_t* pr
     return a < b ? make_int2(a, b) : make_int2(b, a);
 }
 
-// Contiguous copy of pairs [first, first + count) of a list into dst.
+// Contiguous copy of pairs [first, first + count) of a list into dst. TOTALS: the totals too, by the
+// first workgroup's first two waves, and no copy after an overflow.
+template <bool TOTALS>
 __global__ void __launch_bounds__(kBlock) k_pair_gather(DevState d, int kind, int2* __restrict__ dst, uint64_t first,
-                                                        uint64_t count) {
+                                                        uint64_t count, int narrow) {
     __shared__ uint32_t pre[kPairSegs + 1];
     const uint32_t listed = seg_prefix(d.pcnt + kind * kPairSegs * kCntStride, (uint32_t)d.pair_seg_cap, pre);
-    const uint64_t total = (uint64_t)listed + d.ctr[kind ? C_IMPL_NP : C_IMPLICIT];
+    const uint32_t impl = !TOTALS ? d.ctr[kind ? C_IMPL_NP : C_IMPLICIT] : kind == 0 || narrow ? d.ctr[C_IMPLICIT] : 0u;
+    if (TOTALS) {
+        if (blockIdx.x == 0 && threadIdx.x < 128) pair_totals(d, narrow);
+        if (d.ctr[C_OVF]) return;
+    }
+    const uint64_t total = (uint64_t)listed + impl;
     const uint64_t end = min(first + count, total);
     for (uint64_t k = first + blockIdx.x * blockDim.x + threadIdx.x; k < end; k += gridDim.x * blockDim.x)
         dst[k - first] = list_pair(d, kind, pre, listed, (uint32_t)k);
 }
 void launch_pair_gather(DevState& d, int kind, int2* dst, int64_t first, int64_t count, hipStream_t s) {
-    hipLaunchKernelGGL(k_pair_gather, dim3(2048), dim3(kBlock), 0, s, d, kind, dst, (uint64_t)first,
-                       (uint64_t)count);
+    hipLaunchKernelGGL(k_pair_gather<false>, dim3(std::min(grid_for(count), 2048u)), dim3(kBlock), 0, s, d, kind, dst,
+                       (uint64_t)first, (uint64_t)count, 0);
+}
+void launch_totals_and_gather(DevState& d, int kind, int2* dst, int64_t cap, bool narrow, hipStream_t s) {
+    hipLaunchKernelGGL(k_pair_gather<true>, dim3(std::min(grid_for(cap), 2048u)), dim3(kBlock), 0, s, d, kind, dst,
+                       (uint64_t)0, (uint64_t)cap, narrow ? 1 : 0);
 }
 
 // ---------------------------------------------------------------- pair-set digest

@@ -85,6 +85,9 @@ void launch_narrow(DevState& d, hipStream_t s, bool counters_zeroed = false);  /
 void launch_pair_totals(DevState& d, hipStream_t s, bool narrow);
 void clear_np(DevState& d, hipStream_t s);
 void launch_pair_gather(DevState& d, int kind, int2* dst, int64_t first, int64_t count, hipStream_t s);
+// The totals and the copy of the first cap pairs (fewer if there are not so many, none if a list
+// overflowed) in one launch.
+void launch_totals_and_gather(DevState& d, int kind, int2* dst, int64_t cap, bool narrow, hipStream_t s);
 void launch_digest(DevState& d, int filtered, hipStream_t s);
 void launch_restr_decision(DevState& d, int32_t n, hipStream_t s);    // counts into ctr[C_RT_*]
 
