@@ -32,7 +32,8 @@ inline unsigned make_shape(unsigned grid, unsigned unroll, unsigned waves = 4) {
 inline unsigned shape_grid(unsigned sh) { return sh & 0xFFFFFFu; }
 inline unsigned shape_unroll(unsigned sh) { return ((sh >> 24) & 15u) ? ((sh >> 24) & 15u) : 1u; }
 inline unsigned shape_waves(unsigned sh) { return (sh >> 28) ? (sh >> 28) : 4u; }
-unsigned tuned_shape(int kernel, int64_t n);
+// The shape set for the size class of n, else the default for `queries` (0: n).
+unsigned tuned_shape(int kernel, int64_t n, int64_t queries = 0);
 void set_tuned_shape(int kernel, int64_t n, unsigned sh);
 void record_tuning(int kernel, int64_t n, unsigned sh, float ms);
 std::string tuning_report();
