@@ -1096,9 +1096,9 @@ void launch_refit_prep(DevState& d, int32_t n, hipStream_t s) {
     const int32_t nc = refit_chunks(n);
     fill_i32(d.rp_cstart, nc + 1, n, s);
     fill_u32(d.rp_tcount, 1, 0u, s);
-    hipLaunchKernelGGL(k_rp_starts, dim3(grid_for(n)), dim3(kBlock), 0, s, n, d);
     fill_u32(d.rp_tdone, 1, 0u, s);
-    fill_u32(d.rp_tdeep, 1, 0u, s);
+    fill_u32(d.rp_tdeep, 1, 0u, s);  // set by k_rp_starts: cleared before it
+    hipLaunchKernelGGL(k_rp_starts, dim3(grid_for(n)), dim3(kBlock), 0, s, n, d);
     fill_i32(d.rp_tsz, n, 0, s);  // climb flags of deep top trees (prep scratch otherwise)
     hipLaunchKernelGGL(k_rp_top_sort, dim3(1), dim3(kTopBlock), 0, s, d);
     hipLaunchKernelGGL(k_rp_top_segments, dim3(1), dim3(kTopBlock), 0, s, d, refit_tcb_boxes(n));

@@ -712,3 +712,29 @@ def test_pure_traversal_equals_front_walk(pkg, oracle, kind, T, skip_adjacent):
         for f in (False, True):
             np.testing.assert_array_equal(got[f], oracle.pair_set(ctx.pairs(f)), err_msg=f"{op} filtered {f}")
     ctx.close()
+
+
+@pytest.mark.parametrize("T,chain", [(4096, 3000), (24000, 18000)])
+def test_refit_deep_chain_of_different_boxes(pkg, oracle, T, chain):
+    """A chain of equal Morton codes deeper than the refit's level bins, its triangles' boxes all
+    different (so a node merged before its child shows), below and above the size of a top tree
+    that one workgroup holds in LDS: boxes equal the oracle's refit after a build and a refit."""
+    print(f"[gpu] refit deep chain {chain} of {T}", flush=True)
+    rng = np.random.default_rng(5)
+    c = rng.random((T, 1, 3))
+    c[:chain] = 0.3 + c[:chain] * 1e-5  # well inside one Morton cell
+    v = (c + rng.random((T, 3, 3)) * 1e-6).reshape(-1, 3).astype(np.float32)
+    f = np.arange(3 * T, dtype=np.int32).reshape(T, 3)
+    ctx = pkg.CollisionContext(T, 3 * T, narrow_phase=False, pair_cap=64 * T)
+    ctx.set_topology(f, 3 * T)
+    topo = None
+    for k in range(2):
+        ctx.update_vertices(v)
+        ctx.step(pkg.BVH_BUILD if k == 0 else pkg.BVH_REFIT, pkg.FRONT_PURE_BVH_CD)
+        b = ctx.export_bvh()
+        topo = topo or oracle.build_topology(b["codes"])
+        leaf = oracle.tri_boxes(f, v)[b["prim_idx"]]
+        np.testing.assert_array_equal(b["leaf_box"], leaf)
+        np.testing.assert_array_equal(b["int_box"], oracle.refit_boxes(topo, leaf))
+        v = (v + rng.normal(0, 1e-7, v.shape)).astype(np.float32)
+    ctx.close()
