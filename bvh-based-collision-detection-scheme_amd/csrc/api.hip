@@ -142,11 +142,16 @@ bool alloc_lists(bvhcd_ctx* c, int64_t ci, int64_t ce, int64_t cp) {
             ok = ok && lalloc(d.fnode[k][b], (size_t)d.front_cap[k]);
             ok = ok && lalloc(d.fquery[k][b], (size_t)d.front_cap[k]);
         }
-    // digit table of the largest sort (front ordering) and the scan block sums
+    // tile words of the largest sort (front ordering) and of the largest scan (per-node counts, waves or
+    // partition tiles)
     const int64_t max_sort = std::max<int64_t>(T, std::max(d.front_cap[0], d.front_cap[1]));
-    d.sort_hist_n = (size_t)(256 * ((max_sort + 4095) / 4096));
-    d.scan_tmp_n = (size_t)((std::max<int64_t>((int64_t)d.sort_hist_n, T + 2) + 4095) / 4096 + 1);
-    ok = ok && lalloc(d.sort_hist, d.sort_hist_n) && lalloc(d.scan_tmp, d.scan_tmp_n);
+    const int64_t max_scan = std::max<int64_t>({T + 2, d.wave_cap, d.front_cap[1] / kAdjTile + 2});
+    d.scan_tiles = (size_t)((max_scan + 4095) / 4096);
+    ok = ok && lalloc(d.sort_state, sort_state_words(max_sort)) && lalloc(d.sort_ctl, sort_ctl_words()) &&
+         lalloc(d.scan_state, d.scan_tiles) && lalloc(d.scan_ctl, 2) &&
+         hipMemsetAsync(d.sort_ctl, 0, sort_ctl_words() * sizeof(uint32_t), c->stream) == hipSuccess &&
+         hipMemsetAsync(d.scan_state, 0, d.scan_tiles * sizeof(uint64_t), c->stream) == hipSuccess &&
+         hipMemsetAsync(d.scan_ctl, 0, 2 * sizeof(uint32_t), c->stream) == hipSuccess;
     ok = ok && lalloc(d.bp, (size_t)d.pair_cap) && lalloc(d.np, (size_t)d.pair_cap) &&
          lalloc(d.pair_tmp, (size_t)d.pair_cap);
     ok = ok && lalloc(d.adj_cnt, (size_t)(d.front_cap[1] / kAdjTile + 2)) &&

@@ -410,10 +410,8 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     if (cfg->pair_cap <= 0) cp = std::min<int64_t>(cp, (int64_t)(0.5 * (double)free_b / 24.0));
     d.pair_seg_cap = std::max<int64_t>((std::max<int64_t>(cp, 1) + kPairSegs - 1) / kPairSegs, 1);
     d.pair_cap = d.pair_seg_cap * kPairSegs;
-    const int64_t tiles = (T + 4095) / 4096;
-    d.sort_hist_n = (size_t)(256 * tiles);
     const int64_t gtbl_n = S <= kGroupScenes ? (int64_t)S * group_blocks(S) : 0;
-    d.scan_tmp_n = (size_t)((std::max<int64_t>({(int64_t)d.sort_hist_n, T + 2, gtbl_n}) + 4095) / 4096 + 1);
+    d.scan_tiles = (size_t)((std::max<int64_t>({T + 2, gtbl_n, (int64_t)S + 1}) + 4095) / 4096);
     bool ok = true;
     ok &= balloc(b, d.faces, 3 * T);
     ok &= balloc(b, d.verts, 3 * V);
@@ -460,8 +458,10 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     ok &= balloc(b, d.depths, T + 1);
     ok &= balloc(b, d.offsets, T + 1);
     ok &= balloc(b, d.tkmap, T);
-    ok &= balloc(b, d.sort_hist, d.sort_hist_n);
-    ok &= balloc(b, d.scan_tmp, d.scan_tmp_n);
+    ok &= balloc(b, d.sort_state, sort_state_words(T));
+    ok &= balloc(b, d.sort_ctl, sort_ctl_words());
+    ok &= balloc(b, d.scan_state, d.scan_tiles);
+    ok &= balloc(b, d.scan_ctl, 2);
     ok &= balloc(b, d.ctr, 32);
     ok &= balloc(b, d.bp, d.pair_cap);
     ok &= balloc(b, d.np, d.pair_cap);
@@ -501,6 +501,9 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
                hipMemcpyAsync(b->voff_dev, b->voff.data(), sizeof(int64_t) * (S + 1), hipMemcpyHostToDevice,
                               b->stream) == hipSuccess &&
                hipMemsetAsync(d.ctr, 0, 32 * sizeof(uint32_t), b->stream) == hipSuccess &&
+               hipMemsetAsync(d.sort_ctl, 0, sort_ctl_words() * sizeof(uint32_t), b->stream) == hipSuccess &&
+               hipMemsetAsync(d.scan_state, 0, d.scan_tiles * sizeof(uint64_t), b->stream) == hipSuccess &&
+               hipMemsetAsync(d.scan_ctl, 0, 2 * sizeof(uint32_t), b->stream) == hipSuccess &&
                hipMemsetAsync(d.pcnt, 0, 2 * kPairSegs * kCntStride * sizeof(uint32_t), b->stream) == hipSuccess;
     if (okc) {
         hipLaunchKernelGGL(k_tri_scene, dim3(std::min<unsigned>(grid_for(T), 4096)), dim3(kBlock), 0, b->stream, T, S,

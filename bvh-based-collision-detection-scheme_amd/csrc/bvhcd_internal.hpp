@@ -206,10 +206,11 @@ struct DevState {
     uint32_t* offsets = nullptr;    // T+1
     int32_t* tkmap = nullptr;       // T split id -> preorder id
     // scan / sort scratch
-    uint32_t* scan_tmp = nullptr;   // block sums
-    size_t scan_tmp_n = 0;
-    uint32_t* sort_hist = nullptr;  // digit histograms
-    size_t sort_hist_n = 0;
+    uint64_t* scan_state = nullptr; // scan_tiles: one word per tile of a scan, zero between scans
+    uint32_t* scan_ctl = nullptr;   // 2: tile counter, tiles done, zero between scans
+    size_t scan_tiles = 0;
+    uint64_t* sort_state = nullptr; // sort_state_words(): tile words of two passes
+    uint32_t* sort_ctl = nullptr;   // sort_ctl_words(): digit counts, counters, zero between sorts
     float* scene_box = nullptr;     // 6 floats (+ pad)
     uint32_t* scene_box_u = nullptr;// ordered-int reduction scratch, 6 words
     // fronts: SoA (node id, query leaf), double buffered per kind (0 internal, 1 external)

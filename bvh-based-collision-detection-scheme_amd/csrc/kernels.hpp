@@ -11,6 +11,10 @@ void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 void fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t s);
 void launch_scene_box(DevState& d, int32_t T, hipStream_t s);
 void launch_codes(DevState& d, int32_t T, uint32_t* codes, int32_t* vals, hipStream_t s);
+// Scratch: scan_tiles words of d.scan_state for (n + 4095) / 4096 tiles, sort_state_words(n) of
+// d.sort_state for sorts of up to n keys; d.scan_* and d.sort_ctl are zero before the first use.
+size_t sort_state_words(int64_t n);
+size_t sort_ctl_words();
 void launch_exscan(DevState& d, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, hipStream_t s);
 void radix_sort_u32(DevState& d, uint32_t* keys, int32_t* vals, uint32_t* tkeys, int32_t* tvals, int64_t n, int nbits,
                     hipStream_t s);

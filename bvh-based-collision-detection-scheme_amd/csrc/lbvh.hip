@@ -15,12 +15,13 @@
 //    searches over the sorted codes (nearest delta >= d on the left, nearest delta > d on
 //    the right), so emission is one independent thread per node: no atomics, no climbing,
 //    no memory-ordering hazards.
-//  * Sorting is an LSD radix sort with 8-bit digits over an LDS-staged tile of 4096 keys:
-//    per-tile digit counts, a device-wide exclusive scan of the digit-major count table,
-//    then a stable wave64 multisplit ranking in LDS and coalesced scatter.
+//  * Sorting is an LSD radix sort with 8-bit digits, one launch per digit: tiles rank their keys
+//    with a stable wave64 multisplit in LDS, hand their digit counts on along the chain of tiles
+//    and scatter coalesced.
 //  * Refit is level-synchronous over treelet-aligned chunks: each workgroup merges its
 //    treelets' nodes one depth level per barrier in LDS (no atomics), then the top tree above
 //    the treelets is merged in LDS by one workgroup per segment of at most 4096 nodes.
+#include <algorithm>
 #include <type_traits>
 
 #include "bvhcd_internal.hpp"
@@ -100,6 +101,22 @@ void launch_codes(DevState& d, int32_t T, uint32_t* codes, int32_t* vals, hipStr
                        vals);
 }
 
+// ======================================================================= chained tiles
+// The scan and the sort's digit passes run as one launch each: tiles hand their running sums on to
+// the following ones through a word per tile (and digit), a 64-bit (flag, value) pair written and
+// read in one access: kTileSum = the tile's own sum, kTileRun = the sum of all tiles up to it. A
+// workgroup takes its tile from a counter, so every tile it waits for belongs to a workgroup that is
+// already running, and those publish their own sum before they wait for anything: every wait ends.
+// (A reduce, a scan of the tile sums and a second read took three launches per scan and five per
+// digit pass; on small scenes the launches were most of the time.)
+constexpr uint64_t kTileSum = 1ull << 32, kTileRun = 2ull << 32;
+__device__ inline void tile_store(uint64_t* p, uint64_t flag, uint32_t v) {
+    __hip_atomic_store(p, flag | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline uint64_t tile_load(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ======================================================================= exclusive scan (u32)
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;  // 4096
@@ -126,148 +143,174 @@ __device__ inline uint32_t block_exscan(uint32_t v, uint32_t& excl) {
     return total;
 }
 
-__global__ void __launch_bounds__(kBlock) k_scan_sums(const uint32_t* __restrict__ in, int64_t n, uint32_t* sums) {
-    const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    uint32_t s = 0;
-    for (int i = 0; i < kScanItems; ++i) {
-        int64_t j = base + (int64_t)i * kBlock + threadIdx.x;
-        if (j < n) s += in[j];
-    }
-    uint32_t ex;
-    uint32_t tot = block_exscan(s, ex);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-
-// Single-block exclusive scan of m block sums (in place); optional total.
-__global__ void __launch_bounds__(kBlock) k_scan_single(uint32_t* sums, int64_t m, uint32_t* total_out) {
-    uint32_t carry = 0;
-    for (int64_t base = 0; base < m; base += kBlock) {
-        int64_t j = base + threadIdx.x;
-        uint32_t v = j < m ? sums[j] : 0u;
-        uint32_t ex;
-        uint32_t tot = block_exscan(v, ex);
-        if (j < m) sums[j] = carry + ex;
-        carry += tot;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && total_out) *total_out = carry;
-}
-
 // `in` may equal `out` (in-place scan): every thread reads its items before the barrier in
-// block_exscan and writes them after it.
-__global__ void __launch_bounds__(kBlock) k_scan_apply(const uint32_t* in, int64_t n, const uint32_t* __restrict__ sums,
-                                                       uint32_t* out) {
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
+// block_exscan and writes them after it. Wave 0 looks back over 64 tiles at a time. ctl[0] = tile
+// counter, ctl[1] = tiles done; the workgroup that finishes last clears them and the tile words for
+// the next scan. 180k values 14 -> 5 us, 41k 13 -> 5 us, 2.1M 25 -> 11 us.
+__global__ void __launch_bounds__(kBlock) k_scan(const uint32_t* in, int64_t n, uint32_t* out, uint32_t* total_out,
+                                                 uint64_t* state, uint32_t* ctl) {
+    __shared__ uint32_t s_tile, s_before, s_last;
+    if (threadIdx.x == 0) s_tile = atomicAdd(&ctl[0], 1u);
+    __syncthreads();
+    const uint32_t tile = s_tile;
+    const int64_t base = (int64_t)tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
     uint32_t v[kScanItems];
     uint32_t s = 0;
+#pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
-        int64_t j = base + i;
-        v[i] = j < n ? in[j] : 0u;
+        v[i] = base + i < n ? in[base + i] : 0u;
         s += v[i];
     }
     uint32_t ex;
-    block_exscan(s, ex);
-    uint32_t run = sums[blockIdx.x] + ex;
+    const uint32_t tot = block_exscan(s, ex);
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        uint32_t before = 0;
+        if (lane == 0) tile_store(&state[tile], tile == 0 ? kTileRun : kTileSum, tot);
+        for (int64_t t = (int64_t)tile - 1; t >= 0;) {  // tiles t, t - 1, ... one per lane
+            const uint64_t x = t - lane >= 0 ? tile_load(&state[t - lane]) : kTileRun;
+            const uint64_t run = __ballot((x & kTileRun) != 0), none = __ballot((x >> 32) == 0);
+            const int stop = run ? __ffsll((long long)run) - 1 : 63;  // the last tile to add
+            if (none & ((2ull << stop) - 1ull)) {  // one of them has not published yet
+                __builtin_amdgcn_s_sleep(1);
+                continue;
+            }
+            uint32_t y = lane <= stop ? (uint32_t)x : 0u;
+            for (int off = 32; off > 0; off >>= 1) y += __shfl_xor(y, off);
+            before += y;
+            if (run) break;
+            t -= 64;
+        }
+        if (lane == 0) {
+            if (tile > 0) tile_store(&state[tile], kTileRun, before + tot);
+            s_before = before;
+            if (total_out && tile == gridDim.x - 1) *total_out = before + tot;
+        }
+    }
+    __syncthreads();
+    uint32_t run = s_before + ex;
+#pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
-        int64_t j = base + i;
-        if (j < n) out[j] = run;
+        if (base + i < n) out[base + i] = run;
         run += v[i];
+    }
+    if (threadIdx.x == 0) s_last = atomicAdd(&ctl[1], 1u) == gridDim.x - 1 ? 1u : 0u;
+    __syncthreads();
+    if (s_last) {
+        for (uint32_t t = threadIdx.x; t < gridDim.x; t += kBlock) tile_store(&state[t], 0ull, 0u);
+        if (threadIdx.x < 2) ctl[threadIdx.x] = 0u;
     }
 }
 
 // out[0..n-1] = exclusive scan of in[0..n-1]; if total != nullptr, *total = sum (device).
 void launch_exscan(DevState& d, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, hipStream_t s) {
     if (n <= 0) return;
-    const int64_t blocks = (n + kScanTile - 1) / kScanTile;
-    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)blocks), dim3(kBlock), 0, s, in, n, d.scan_tmp);
-    hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kBlock), 0, s, d.scan_tmp, blocks, total);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)blocks), dim3(kBlock), 0, s, in, n, d.scan_tmp, out);
+    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+    hipLaunchKernelGGL(k_scan, dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n, out, total, d.scan_state, d.scan_ctl);
 }
 
 // ======================================================================= radix sort
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kBlock * kSortItems;  // 4096 keys per tile
+// Stable LSD sort, 8-bit digits. One kernel counts the digits of every pass over the unsorted keys
+// (they do not depend on the order); each pass is then one launch over chained tiles: a tile ranks
+// its keys, hands its digit counts on, and scatters.
 constexpr int kRadix = 256;
+constexpr int kSortMaxPasses = 8;
+constexpr int kSortCtl = kSortMaxPasses * kRadix + kSortMaxPasses + 1;  // counts, tile counters, tiles done
+constexpr int kSortLook = 8;  // tiles a digit's thread looks back over at a time
 
-// Digit counts of one 4096-key tile. Each wave takes 64 keys at a time and groups equal digits
-// with a wave64 multisplit (8 ballots), so one LDS atomic per distinct digit per wave replaces
-// one per key: partially sorted input (later passes, front node ids) has long runs of equal
-// digits that would otherwise serialise on the same LDS word.
-template <class K>
-__global__ void __launch_bounds__(kBlock) k_sort_hist(const K* __restrict__ keys, int64_t n, const uint32_t* dn,
-                                                      int shift, uint32_t* __restrict__ hist, int64_t tiles) {
-    __shared__ uint32_t h[kRadix];
-    if (dn) n = min(n, (int64_t)*dn);
-    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-    if (base >= n) {  // block-uniform: an empty tile contributes zero counts
-        hist[(int64_t)tid * tiles + blockIdx.x] = 0;
-        return;
-    }
-    h[tid] = 0;
-    __syncthreads();
-    const uint64_t below = (1ull << lane) - 1ull;
-    constexpr int kPerWave = kSortTile / (kBlock / 64);
-    for (int r = 0; r < kPerWave / 64; ++r) {
-        const int64_t j = base + w * kPerWave + r * 64 + lane;
-        const bool ok = j < n;
-        const uint32_t dig = ok ? (uint32_t)(keys[j] >> shift) & 0xFFu : 0u;
-        uint64_t peers = __ballot(ok);
+// Lanes holding the same digit as this one (wave64 multisplit, 8 ballots).
+__device__ inline uint64_t digit_peers(bool ok, uint32_t dig) {
+    uint64_t peers = __ballot(ok);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const uint64_t m = __ballot(ok && ((dig >> b) & 1u));
-            peers &= ((dig >> b) & 1u) ? m : ~m;
-        }
-        if (ok && (peers & below) == 0) atomicAdd(&h[dig], (uint32_t)__popcll(peers));
+    for (int b = 0; b < 8; ++b) {
+        const uint64_t m = __ballot(ok && ((dig >> b) & 1u));
+        peers &= ((dig >> b) & 1u) ? m : ~m;
     }
-    __syncthreads();
-    hist[(int64_t)tid * tiles + blockIdx.x] = h[tid];
+    return peers;
 }
 
-// Stable scatter of one 4096-key tile. Wave w owns the tile's items [1024 w, 1024 w + 1024),
+// Digit counts of all passes into ctl (cleared by the last sort). One LDS atomic per distinct digit
+// per wave: sorted stretches have long runs of equal digits that would otherwise serialise on one
+// LDS word. Also clears the first pass's tile words.
+template <class K>
+__global__ void __launch_bounds__(kBlock) k_sort_count(const K* __restrict__ keys, int64_t n, const uint32_t* dn,
+                                                       int passes, int tile_items, uint32_t* __restrict__ ctl,
+                                                       uint64_t* __restrict__ state) {
+    __shared__ uint32_t h[kSortMaxPasses * kRadix];
+    if (dn) n = min(n, (int64_t)*dn);
+    const int64_t words = (n + tile_items - 1) / tile_items * kRadix;
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < words; i += (int64_t)gridDim.x * kBlock)
+        state[i] = 0ull;
+    if (blockIdx.x * (int64_t)kBlock >= n) return;  // block-uniform
+    for (int i = threadIdx.x; i < passes * kRadix; i += kBlock) h[i] = 0;
+    __syncthreads();
+    const uint64_t below = (1ull << lane_id()) - 1ull;
+    for (int64_t j0 = blockIdx.x * (int64_t)kBlock + (threadIdx.x & ~63); j0 < n; j0 += (int64_t)gridDim.x * kBlock) {
+        const bool ok = j0 + lane_id() < n;  // wave-uniform trip count
+        const K key = ok ? keys[j0 + lane_id()] : (K)0;
+        for (int p = 0; p < passes; ++p) {
+            const uint32_t dig = (uint32_t)(key >> (8 * p)) & 0xFFu;
+            const uint64_t peers = digit_peers(ok, dig);
+            if (ok && (peers & below) == 0) atomicAdd(&h[p * kRadix + dig], (uint32_t)__popcll(peers));
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < passes * kRadix; i += kBlock)
+        if (h[i]) atomicAdd(&ctl[i], h[i]);
+}
+
+// One digit pass over tiles of 256 * ITEMS keys. Wave w owns the tile's items [64 ITEMS w, 64 ITEMS (w + 1)),
 // taken 64 at a time in index order; a wave64 multisplit (8 ballots) gives each item its rank
 // among the wave's earlier items with the same digit, using only the wave's own LDS counters
 // (no block barrier inside the loop). One block-level pass then turns the per-wave digit counts
 // into offsets, so an item's tile position is
 //   tile_start[digit] + (same-digit items of earlier waves) + (its rank inside the wave),
-// i.e. the stable order by index. Keys stay in registers between the two steps.
-template <class K>
-__global__ void __launch_bounds__(kBlock) k_sort_scatter(const K* __restrict__ keys, const int32_t* __restrict__ vals,
-                                                         int64_t n, const uint32_t* dn, int shift,
-                                                         const uint32_t* __restrict__ hist, int64_t tiles,
-                                                         K* __restrict__ okeys, int32_t* __restrict__ ovals) {
+// i.e. the stable order by index. Thread t looks back for digit t, kSortLook tiles at a time. Keys and
+// values stay in registers meanwhile. state_next (the next pass's tile words) is cleared row by row;
+// `last` = last pass: the workgroup finishing last clears ctl for the next sort.
+template <class K, int ITEMS>
+__global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys, const int32_t* __restrict__ vals,
+                                                      int64_t n, const uint32_t* dn, int pass, int last,
+                                                      uint32_t* __restrict__ ctl, uint64_t* __restrict__ state,
+                                                      uint64_t* __restrict__ state_next, K* __restrict__ okeys,
+                                                      int32_t* __restrict__ ovals) {
     constexpr int kWavesS = kBlock / 64;
-    constexpr int kPerWave = kSortTile / kWavesS;   // 1024
-    constexpr int kRounds = kPerWave / 64;          // 16
+    constexpr int kTile = kBlock * ITEMS;
+    constexpr int kPerWave = 64 * ITEMS;
     __shared__ uint32_t wcnt[kWavesS][kRadix];      // per-wave digit counts, then offsets
     __shared__ uint32_t tile_start[kRadix];
     __shared__ uint32_t gofs[kRadix];
-    __shared__ K skeys[kSortTile];
-    __shared__ int32_t svals[kSortTile];
-    __shared__ uint8_t sdig[kSortTile];
+    __shared__ K skeys[kTile];
+    __shared__ int32_t svals[kTile];
+    __shared__ uint8_t sdig[kTile];
+    __shared__ uint32_t s_tile, s_last;
 
-    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6, shift = 8 * pass;
     if (dn) n = min(n, (int64_t)*dn);
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-    if (base >= n) return;  // whole block uniform: before any barrier
-    const int valid = (int)((n - base) < kSortTile ? (n - base) : kSortTile);
-
+    const uint32_t tiles = (uint32_t)((n + kTile - 1) / kTile);
+    if (blockIdx.x >= tiles) return;  // whole block: as many workgroups stay as there are tiles
+    if (tid == 0) s_tile = atomicAdd(&ctl[kSortMaxPasses * kRadix + pass], 1u);
     for (int k = lane; k < kRadix; k += 64) wcnt[w][k] = 0;
-    K key[kRounds];
-    uint32_t rk[kRounds];
+    __syncthreads();
+    const uint32_t tile = s_tile;
+    const int64_t base = (int64_t)tile * kTile;
+    const int valid = (int)((n - base) < kTile ? (n - base) : kTile);
+
+    K key[ITEMS];
+    int32_t val[ITEMS];
+    uint32_t rk[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int j = w * kPerWave + r * 64 + lane;
+        key[r] = j < valid ? keys[base + j] : (K)0;
+        val[r] = j < valid ? vals[base + j] : 0;
+    }
     const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-        const int j = w * kPerWave + r * 64 + lane;
-        const bool ok = j < valid;
-        key[r] = ok ? keys[base + j] : (K)0;
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool ok = w * kPerWave + r * 64 + lane < valid;
         const uint32_t dig = (uint32_t)(key[r] >> shift) & 0xFFu;
-        uint64_t peers = __ballot(ok);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const uint64_t m = __ballot(ok && ((dig >> b) & 1u));
-            peers &= ((dig >> b) & 1u) ? m : ~m;
-        }
+        const uint64_t peers = digit_peers(ok, dig);
         const uint32_t before = ok ? wcnt[w][dig] : 0u;
         rk[r] = before + (uint32_t)__popcll(peers & below);
         // the lowest lane of each peer group advances the wave's count (its read above was
@@ -276,7 +319,7 @@ __global__ void __launch_bounds__(kBlock) k_sort_scatter(const K* __restrict__ k
         __builtin_amdgcn_wave_barrier();  // keep the next round's reads after this write
     }
     __syncthreads();
-    {   // digit tid: offsets of each wave's group, then the tile-wide exclusive scan
+    {   // digit tid: offsets of each wave's group, the tile-wide scan, the earlier tiles' keys
         uint32_t acc = 0;
 #pragma unroll
         for (int ww = 0; ww < kWavesS; ++ww) {
@@ -284,26 +327,53 @@ __global__ void __launch_bounds__(kBlock) k_sort_scatter(const K* __restrict__ k
             wcnt[ww][tid] = acc;
             acc += c;
         }
-        uint32_t ex;
-        block_exscan(acc, ex);   // contains a barrier; every thread reaches it
+        uint64_t* own = state + (int64_t)tile * kRadix + tid;
+        tile_store(own, tile == 0 ? kTileRun : kTileSum, acc);
+        state_next[(int64_t)tile * kRadix + tid] = 0ull;
+        uint32_t ex, first;
+        block_exscan(acc, ex);   // contain barriers; every thread reaches them
+        block_exscan(ctl[pass * kRadix + tid], first);
+        uint32_t before = 0;
+        bool open = tile > 0;
+        for (int64_t t = (int64_t)tile - 1; open;) {
+            uint64_t x[kSortLook];
+#pragma unroll
+            for (int u = 0; u < kSortLook; ++u)
+                x[u] = t - u >= 0 ? tile_load(state + (t - u) * kRadix + tid) : kTileRun;
+            bool moved = false;
+#pragma unroll
+            for (int u = 0; u < kSortLook; ++u) {
+                if (!open || (x[u] >> 32) == 0 || (u > 0 && !moved)) {
+                    moved = false;  // not published yet: look again from here
+                    continue;
+                }
+                before += (uint32_t)x[u];
+                moved = true;
+                --t;
+                if (x[u] & kTileRun) open = false;
+            }
+            if (open && !moved) __builtin_amdgcn_s_sleep(1);
+        }
+        if (tile > 0) tile_store(own, kTileRun, before + acc);
         tile_start[tid] = ex;
-        gofs[tid] = hist[(int64_t)tid * tiles + blockIdx.x];
+        gofs[tid] = first + before;
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const int j = w * kPerWave + r * 64 + lane;
         if (j < valid) {
             const uint32_t dig = (uint32_t)(key[r] >> shift) & 0xFFu;
             const uint32_t pos = tile_start[dig] + wcnt[w][dig] + rk[r];
             skeys[pos] = key[r];
-            svals[pos] = vals[base + j];
+            svals[pos] = val[r];
             sdig[pos] = (uint8_t)dig;
         }
     }
     __syncthreads();
     // coalesced write-out in tile-sorted order
-    for (int i = 0; i < kSortItems; ++i) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
         const int j = i * kBlock + tid;
         if (j < valid) {
             const uint32_t dg = sdig[j];
@@ -312,31 +382,48 @@ __global__ void __launch_bounds__(kBlock) k_sort_scatter(const K* __restrict__ k
             ovals[o] = svals[j];
         }
     }
+    if (!last) return;
+    if (tid == 0) s_last = atomicAdd(&ctl[kSortCtl - 1], 1u) == tiles - 1 ? 1u : 0u;
+    __syncthreads();
+    if (s_last)
+        for (int i = tid; i < kSortCtl; i += kBlock) ctl[i] = 0u;
 }
+
+// Tiles of 1024 keys up to this many keys (256 workgroups), of 4096 above.
+constexpr int64_t kSortSmall = 1 << 18;
+size_t sort_state_words(int64_t n) {
+    const int64_t tiles = n <= kSortSmall ? (n + 1023) / 1024 : std::max<int64_t>((n + 4095) / 4096, kSortSmall / 1024);
+    return (size_t)(2 * kRadix * std::max<int64_t>(tiles, 1));
+}
+size_t sort_ctl_words() { return kSortCtl; }
 
 // Stable LSD sort of (keys, vals) over bits [0, nbits), ping-ponging between the given
 // buffers. n is the element count, or (dn != nullptr) its upper bound with the actual count
 // read on the device. Returns true when the result sits in (tkeys, tvals) (odd pass count).
+template <class K, int ITEMS>
+static bool sort_passes(DevState& d, K* keys, int32_t* vals, K* tkeys, int32_t* tvals, int64_t n, const uint32_t* dn,
+                        int passes, hipStream_t s) {
+    constexpr int kTile = kBlock * ITEMS;
+    const unsigned tiles = (unsigned)((n + kTile - 1) / kTile);
+    uint64_t* state[2] = {d.sort_state, d.sort_state + (size_t)kRadix * tiles};
+    hipLaunchKernelGGL(k_sort_count<K>, dim3(std::min(grid_for(n), 512u)), dim3(kBlock), 0, s, keys, n, dn, passes,
+                       kTile, d.sort_ctl, state[0]);
+    for (int p = 0; p < passes; ++p) {
+        hipLaunchKernelGGL((k_sort_pass<K, ITEMS>), dim3(tiles), dim3(kBlock), 0, s, keys, vals, n, dn, p,
+                           p == passes - 1 ? 1 : 0, d.sort_ctl, state[p & 1], state[(p + 1) & 1], tkeys, tvals);
+        std::swap(keys, tkeys);
+        std::swap(vals, tvals);
+    }
+    return passes & 1;
+}
 template <class K>
 bool radix_sort_passes(DevState& d, K* keys, int32_t* vals, K* tkeys, int32_t* tvals, int64_t n, const uint32_t* dn,
                        int nbits, hipStream_t s) {
     if (n <= 1 && !dn) return false;
     if (n < 1) return false;
-    const int64_t tiles = (n + kSortTile - 1) / kSortTile;
     const int passes = (nbits + 7) / 8;
-    K* ik = keys; int32_t* iv = vals;
-    K* ok = tkeys; int32_t* ov = tvals;
-    for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p;
-        hipLaunchKernelGGL(k_sort_hist<K>, dim3((unsigned)tiles), dim3(kBlock), 0, s, ik, n, dn, shift, d.sort_hist,
-                           tiles);
-        launch_exscan(d, d.sort_hist, d.sort_hist, (int64_t)kRadix * tiles, nullptr, s);
-        hipLaunchKernelGGL(k_sort_scatter<K>, dim3((unsigned)tiles), dim3(kBlock), 0, s, ik, iv, n, dn, shift,
-                           d.sort_hist, tiles, ok, ov);
-        std::swap(ik, ok);
-        std::swap(iv, ov);
-    }
-    return passes & 1;
+    return n <= kSortSmall ? sort_passes<K, 4>(d, keys, vals, tkeys, tvals, n, dn, passes, s)
+                           : sort_passes<K, 16>(d, keys, vals, tkeys, tvals, n, dn, passes, s);
 }
 
 // Result always ends in (keys, vals).

@@ -738,3 +738,31 @@ def test_refit_deep_chain_of_different_boxes(pkg, oracle, T, chain):
         np.testing.assert_array_equal(b["int_box"], oracle.refit_boxes(topo, leaf))
         v = (v + rng.normal(0, 1e-7, v.shape)).astype(np.float32)
     ctx.close()
+
+
+@pytest.mark.parametrize("T", [255, 1024, 1025, 4096, 4097, 65537, 262144, 262145, 300001])
+def test_sort_and_scan_tile_edges(pkg, oracle, T):
+    """Builds at the edges of the sort's 1024- and 4096-key tiles, of its switch between them (262,144
+    keys) and of the scan's 4096-value tiles: codes, order and topology equal the oracle's, twice in
+    a row (the second build starts from the scratch the first one left)."""
+    print(f"[gpu] sort and scan at {T} triangles", flush=True)
+    rng = np.random.default_rng(T)
+    c = rng.random((T, 1, 3))
+    c[: T // 4] = 0.25 + c[: T // 4] / 2048  # many equal codes: the order within them is the triangles'
+    v = (c + rng.random((T, 3, 3)) * 1e-6).reshape(-1, 3).astype(np.float32)
+    f = np.arange(3 * T, dtype=np.int32).reshape(T, 3)
+    ctx = pkg.CollisionContext(T, 3 * T, narrow_phase=False)
+    ctx.set_topology(f, 3 * T)
+    box = oracle.scene_box(f, v)
+    codes = oracle.morton_codes(f, v, box)
+    order = np.argsort(codes, kind="stable")
+    topo = oracle.build_topology(codes[order])
+    for _ in range(2):
+        ctx.update_vertices(v)
+        ctx.step(pkg.BVH_BUILD, pkg.FRONT_PURE_BVH_CD)
+        b = ctx.export_bvh()
+        np.testing.assert_array_equal(b["codes"], codes[order])
+        np.testing.assert_array_equal(b["prim_idx"], order)
+        for k in ("int_lc", "int_rc", "int_rx", "int_ry", "leaf_par", "leaf_lca"):
+            np.testing.assert_array_equal(b[k], topo[k], err_msg=k)
+    ctx.close()
