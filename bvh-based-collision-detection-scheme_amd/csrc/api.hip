@@ -145,7 +145,7 @@ bool alloc_lists(bvhcd_ctx* c, int64_t ci, int64_t ce, int64_t cp) {
     // tile words of the largest sort (front ordering) and of the largest scan (per-node counts, waves or
     // partition tiles)
     const int64_t max_sort = std::max<int64_t>(T, std::max(d.front_cap[0], d.front_cap[1]));
-    const int64_t max_scan = std::max<int64_t>({T + 2, d.wave_cap, d.front_cap[1] / kAdjTile + 2});
+    const int64_t max_scan = std::max<int64_t>({T + 2, d.wave_cap, d.front_cap[1] / kAdjTile + 2, sort_scan_values(max_sort)});
     d.scan_tiles = (size_t)((max_scan + 4095) / 4096);
     ok = ok && lalloc(d.sort_state, sort_state_words(max_sort)) && lalloc(d.sort_ctl, sort_ctl_words()) &&
          lalloc(d.scan_state, d.scan_tiles) && lalloc(d.scan_ctl, 2) &&

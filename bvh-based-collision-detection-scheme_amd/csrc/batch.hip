@@ -411,7 +411,7 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     d.pair_seg_cap = std::max<int64_t>((std::max<int64_t>(cp, 1) + kPairSegs - 1) / kPairSegs, 1);
     d.pair_cap = d.pair_seg_cap * kPairSegs;
     const int64_t gtbl_n = S <= kGroupScenes ? (int64_t)S * group_blocks(S) : 0;
-    d.scan_tiles = (size_t)((std::max<int64_t>({T + 2, gtbl_n, (int64_t)S + 1}) + 4095) / 4096);
+    d.scan_tiles = (size_t)((std::max<int64_t>({T + 2, gtbl_n, (int64_t)S + 1, sort_scan_values(T)}) + 4095) / 4096);
     bool ok = true;
     ok &= balloc(b, d.faces, 3 * T);
     ok &= balloc(b, d.verts, 3 * V);

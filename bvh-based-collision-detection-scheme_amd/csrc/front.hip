@@ -1274,8 +1274,14 @@ static void order_front(DevState& d, int kind, int32_t nb, uint32_t* cnt, uint32
 // A freshly generated internal front is radix-sorted instead (3 passes of 8 bits, then the bucket
 // starts by binary search): there every query's front holds the few nodes with the largest
 // subtrees, and the counting sort's atomics on those nodes' counters contend even when each wave
-// takes its equal keys together (measured on the folded 2M-triangle cloth, 45 M entries: counting
-// 4.7 ms, radix 1.9 ms; the other fronts: counting 1.0-1.4 ms, radix 1.2-1.9 ms).
+// takes its equal keys together (measured on the folded 2M-triangle cloth, 46.8 M entries: counting
+// 4.7 ms, radix 1.3 ms). So is a generated external front of a large scene: in query order hardly
+// any neighbours share a leaf, so the counting sort makes two random atomics per entry (2M cloth,
+// 35 M entries: 1.6 ms against 1.0 ms; GENERATE of 522k triangles 2.09 -> 1.97 ms, of 130k 0.53 against
+// 0.56 ms). Fronts made by UPDATE are nearly in node order already, where the counting sort is the
+// faster one for both kinds (UPDATE of the 2M cloth 3.18 ms, 3.51 with internal and 3.78 with both by
+// radix).
+constexpr int32_t kRadixExtMin = 1 << 18;
 static void radix_order_front(DevState& d, int kind, int32_t nb, uint32_t* beg, hipStream_t s) {
     const int c = d.fcur[kind], o = c ^ 1;
     const bool in_tmp = radix_sort_u32_dev(d, d.fnode[kind][c], d.fquery[kind][c], d.fnode[kind][o], d.fquery[kind][o],
@@ -1292,7 +1298,8 @@ static void radix_order_front(DevState& d, int kind, int32_t nb, uint32_t* beg, 
 void launch_order_fronts(DevState& d, int32_t n, hipStream_t s, bool generated) {
     if (generated) radix_order_front(d, 0, n - 1, d.intbeg, s);
     else order_front(d, 0, n - 1, d.intcnt, d.intbeg, false, s);
-    order_front(d, 1, n, d.extcnt, d.extbeg, false, s);
+    if (generated && n >= kRadixExtMin) radix_order_front(d, 1, n, d.extbeg, s);
+    else order_front(d, 1, n, d.extcnt, d.extbeg, false, s);
 }
 
 // Without node ordering, the front comes out ordered by query without a global sort: the

@@ -15,6 +15,7 @@ void launch_codes(DevState& d, int32_t T, uint32_t* codes, int32_t* vals, hipStr
 // d.sort_state for sorts of up to n keys; d.scan_* and d.sort_ctl are zero before the first use.
 size_t sort_state_words(int64_t n);
 size_t sort_ctl_words();
+int64_t sort_scan_values(int64_t n);  // values that a sort of up to n keys scans
 void launch_exscan(DevState& d, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, hipStream_t s);
 void radix_sort_u32(DevState& d, uint32_t* keys, int32_t* vals, uint32_t* tkeys, int32_t* tvals, int64_t n, int nbits,
                     hipStream_t s);

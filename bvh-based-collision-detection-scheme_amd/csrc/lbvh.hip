@@ -147,9 +147,13 @@ __device__ inline uint32_t block_exscan(uint32_t v, uint32_t& excl) {
 // block_exscan and writes them after it. Wave 0 looks back over 64 tiles at a time. ctl[0] = tile
 // counter, ctl[1] = tiles done; the workgroup that finishes last clears them and the tile words for
 // the next scan. 180k values 14 -> 5 us, 41k 13 -> 5 us, 2.1M 25 -> 11 us.
+// dn (null: n values): a sort's count table, 256 values per tile of tile_items of the *dn keys.
 __global__ void __launch_bounds__(kBlock) k_scan(const uint32_t* in, int64_t n, uint32_t* out, uint32_t* total_out,
-                                                 uint64_t* state, uint32_t* ctl) {
+                                                 const uint32_t* dn, int tile_items, uint64_t* state, uint32_t* ctl) {
     __shared__ uint32_t s_tile, s_before, s_last;
+    if (dn) n = min(n, ((int64_t)*dn + tile_items - 1) / tile_items * 256);
+    const uint32_t tiles = (uint32_t)((n + kScanTile - 1) / kScanTile);
+    if (blockIdx.x >= tiles) return;  // whole block: as many workgroups stay as there are tiles
     if (threadIdx.x == 0) s_tile = atomicAdd(&ctl[0], 1u);
     __syncthreads();
     const uint32_t tile = s_tile;
@@ -184,7 +188,7 @@ __global__ void __launch_bounds__(kBlock) k_scan(const uint32_t* in, int64_t n, 
         if (lane == 0) {
             if (tile > 0) tile_store(&state[tile], kTileRun, before + tot);
             s_before = before;
-            if (total_out && tile == gridDim.x - 1) *total_out = before + tot;
+            if (total_out && tile == tiles - 1) *total_out = before + tot;
         }
     }
     __syncthreads();
@@ -194,29 +198,39 @@ __global__ void __launch_bounds__(kBlock) k_scan(const uint32_t* in, int64_t n, 
         if (base + i < n) out[base + i] = run;
         run += v[i];
     }
-    if (threadIdx.x == 0) s_last = atomicAdd(&ctl[1], 1u) == gridDim.x - 1 ? 1u : 0u;
+    if (threadIdx.x == 0) s_last = atomicAdd(&ctl[1], 1u) == tiles - 1 ? 1u : 0u;
     __syncthreads();
     if (s_last) {
-        for (uint32_t t = threadIdx.x; t < gridDim.x; t += kBlock) tile_store(&state[t], 0ull, 0u);
+        for (uint32_t t = threadIdx.x; t < tiles; t += kBlock) tile_store(&state[t], 0ull, 0u);
         if (threadIdx.x < 2) ctl[threadIdx.x] = 0u;
     }
 }
 
+static void scan_values(DevState& d, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total,
+                        const uint32_t* dn, int tile_items, hipStream_t s) {
+    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+    hipLaunchKernelGGL(k_scan, dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n, out, total, dn, tile_items,
+                       d.scan_state, d.scan_ctl);
+}
 // out[0..n-1] = exclusive scan of in[0..n-1]; if total != nullptr, *total = sum (device).
 void launch_exscan(DevState& d, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, hipStream_t s) {
-    if (n <= 0) return;
-    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-    hipLaunchKernelGGL(k_scan, dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n, out, total, d.scan_state, d.scan_ctl);
+    if (n > 0) scan_values(d, in, out, n, total, nullptr, 1, s);
 }
 
 // ======================================================================= radix sort
-// Stable LSD sort, 8-bit digits. One kernel counts the digits of every pass over the unsorted keys
-// (they do not depend on the order); each pass is then one launch over chained tiles: a tile ranks
-// its keys, hands its digit counts on, and scatters.
+// Stable LSD sort, 8-bit digits, in one of two ways:
+//  * chained (up to kSortChained keys): one kernel counts the digits of every pass over the unsorted
+//    keys (they do not depend on the order); each pass is then one launch over chained tiles: a tile
+//    ranks its keys, hands its digit counts on, and scatters;
+//  * tabled: per pass a table of digit counts per tile, its scan, and the scatter. The chain passes
+//    about 30 tiles per us whatever their number (one counter hands the tiles out), which a pass of
+//    many tiles waits for: 46.8M keys take 0.50 ms a pass chained (with the count's share) and 0.38 ms
+//    tabled, 8.4M keys 0.08 ms chained.
 constexpr int kRadix = 256;
+constexpr int64_t kSortChained = 1 << 25;
 constexpr int kSortMaxPasses = 8;
 constexpr int kSortCtl = kSortMaxPasses * kRadix + kSortMaxPasses + 1;  // counts, tile counters, tiles done
-constexpr int kSortLook = 8;  // tiles a digit's thread looks back over at a time
+constexpr int kSortLook = 16;  // tiles a digit's thread looks back over at a time
 
 // Lanes holding the same digit as this one (wave64 multisplit, 8 ballots).
 __device__ inline uint64_t digit_peers(bool ok, uint32_t dig) {
@@ -245,18 +259,60 @@ __global__ void __launch_bounds__(kBlock) k_sort_count(const K* __restrict__ key
     for (int i = threadIdx.x; i < passes * kRadix; i += kBlock) h[i] = 0;
     __syncthreads();
     const uint64_t below = (1ull << lane_id()) - 1ull;
-    for (int64_t j0 = blockIdx.x * (int64_t)kBlock + (threadIdx.x & ~63); j0 < n; j0 += (int64_t)gridDim.x * kBlock) {
-        const bool ok = j0 + lane_id() < n;  // wave-uniform trip count
-        const K key = ok ? keys[j0 + lane_id()] : (K)0;
-        for (int p = 0; p < passes; ++p) {
-            const uint32_t dig = (uint32_t)(key >> (8 * p)) & 0xFFu;
-            const uint64_t peers = digit_peers(ok, dig);
-            if (ok && (peers & below) == 0) atomicAdd(&h[p * kRadix + dig], (uint32_t)__popcll(peers));
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t j0 = blockIdx.x * (int64_t)kBlock + (threadIdx.x & ~63); j0 < n; j0 += 4 * stride) {
+        K key[4];  // wave-uniform trip count; four loads in flight
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t j = j0 + u * stride + lane_id();
+            key[u] = j < n ? keys[j] : (K)0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool ok = j0 + u * stride + lane_id() < n;
+            for (int p = 0; p < passes; ++p) {
+                const uint32_t dig = (uint32_t)(key[u] >> (8 * p)) & 0xFFu;
+                const uint64_t peers = digit_peers(ok, dig);
+                if (ok && (peers & below) == 0) atomicAdd(&h[p * kRadix + dig], (uint32_t)__popcll(peers));
+            }
         }
     }
     __syncthreads();
     for (int i = threadIdx.x; i < passes * kRadix; i += kBlock)
         if (h[i]) atomicAdd(&ctl[i], h[i]);
+}
+
+// Tiles of a tabled pass: of the actual count where that is on the device only (dn).
+__device__ inline uint32_t table_tiles(int64_t n, const uint32_t* dn, int tile_items) {
+    if (dn) n = min(n, (int64_t)*dn);
+    return (uint32_t)((n + tile_items - 1) / tile_items);
+}
+// Digit counts per tile of a tabled pass: table[digit][tile].
+template <class K, int ITEMS>
+__global__ void __launch_bounds__(kBlock) k_sort_table(const K* __restrict__ keys, int64_t n, const uint32_t* dn,
+                                                       int shift, uint32_t* __restrict__ table) {
+    __shared__ uint32_t h[kRadix];
+    if (dn) n = min(n, (int64_t)*dn);
+    const int64_t base = (int64_t)blockIdx.x * kBlock * ITEMS;
+    if (base >= n) return;  // block-uniform
+    h[threadIdx.x] = 0;
+    K key[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int64_t j = base + r * kBlock + threadIdx.x;
+        key[r] = j < n ? keys[j] : (K)0;
+    }
+    __syncthreads();
+    const uint64_t below = (1ull << lane_id()) - 1ull;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool ok = base + r * kBlock + threadIdx.x < n;
+        const uint32_t dig = (uint32_t)(key[r] >> shift) & 0xFFu;
+        const uint64_t peers = digit_peers(ok, dig);
+        if (ok && (peers & below) == 0) atomicAdd(&h[dig], (uint32_t)__popcll(peers));
+    }
+    __syncthreads();
+    table[(int64_t)threadIdx.x * table_tiles(n, nullptr, kBlock * ITEMS) + blockIdx.x] = h[threadIdx.x];
 }
 
 // One digit pass over tiles of 256 * ITEMS keys. Wave w owns the tile's items [64 ITEMS w, 64 ITEMS (w + 1)),
@@ -265,10 +321,10 @@ __global__ void __launch_bounds__(kBlock) k_sort_count(const K* __restrict__ key
 // (no block barrier inside the loop). One block-level pass then turns the per-wave digit counts
 // into offsets, so an item's tile position is
 //   tile_start[digit] + (same-digit items of earlier waves) + (its rank inside the wave),
-// i.e. the stable order by index. Thread t looks back for digit t, kSortLook tiles at a time. Keys and
-// values stay in registers meanwhile. state_next (the next pass's tile words) is cleared row by row;
+// i.e. the stable order by index. Chained: thread t looks back for digit t, kSortLook tiles at a time;
+// tabled: its place comes from the scanned table (in ctl). Keys and values stay in registers meanwhile. state_next (the next pass's tile words) is cleared row by row;
 // `last` = last pass: the workgroup finishing last clears ctl for the next sort.
-template <class K, int ITEMS>
+template <class K, int ITEMS, bool CHAINED>
 __global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys, const int32_t* __restrict__ vals,
                                                       int64_t n, const uint32_t* dn, int pass, int last,
                                                       uint32_t* __restrict__ ctl, uint64_t* __restrict__ state,
@@ -282,17 +338,16 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys
     __shared__ uint32_t gofs[kRadix];
     __shared__ K skeys[kTile];
     __shared__ int32_t svals[kTile];
-    __shared__ uint8_t sdig[kTile];
     __shared__ uint32_t s_tile, s_last;
 
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6, shift = 8 * pass;
     if (dn) n = min(n, (int64_t)*dn);
     const uint32_t tiles = (uint32_t)((n + kTile - 1) / kTile);
     if (blockIdx.x >= tiles) return;  // whole block: as many workgroups stay as there are tiles
-    if (tid == 0) s_tile = atomicAdd(&ctl[kSortMaxPasses * kRadix + pass], 1u);
+    if (CHAINED && tid == 0) s_tile = atomicAdd(&ctl[kSortMaxPasses * kRadix + pass], 1u);
     for (int k = lane; k < kRadix; k += 64) wcnt[w][k] = 0;
-    __syncthreads();
-    const uint32_t tile = s_tile;
+    if (CHAINED) __syncthreads();
+    const uint32_t tile = CHAINED ? s_tile : blockIdx.x;
     const int64_t base = (int64_t)tile * kTile;
     const int valid = (int)((n - base) < kTile ? (n - base) : kTile);
 
@@ -327,36 +382,44 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys
             wcnt[ww][tid] = acc;
             acc += c;
         }
-        uint64_t* own = state + (int64_t)tile * kRadix + tid;
-        tile_store(own, tile == 0 ? kTileRun : kTileSum, acc);
-        state_next[(int64_t)tile * kRadix + tid] = 0ull;
-        uint32_t ex, first;
-        block_exscan(acc, ex);   // contain barriers; every thread reaches them
-        block_exscan(ctl[pass * kRadix + tid], first);
-        uint32_t before = 0;
-        bool open = tile > 0;
-        for (int64_t t = (int64_t)tile - 1; open;) {
-            uint64_t x[kSortLook];
-#pragma unroll
-            for (int u = 0; u < kSortLook; ++u)
-                x[u] = t - u >= 0 ? tile_load(state + (t - u) * kRadix + tid) : kTileRun;
-            bool moved = false;
-#pragma unroll
-            for (int u = 0; u < kSortLook; ++u) {
-                if (!open || (x[u] >> 32) == 0 || (u > 0 && !moved)) {
-                    moved = false;  // not published yet: look again from here
-                    continue;
-                }
-                before += (uint32_t)x[u];
-                moved = true;
-                --t;
-                if (x[u] & kTileRun) open = false;
-            }
-            if (open && !moved) __builtin_amdgcn_s_sleep(1);
+        if (!CHAINED) {
+            uint32_t ex;
+            block_exscan(acc, ex);
+            tile_start[tid] = ex;
+            gofs[tid] = ctl[(int64_t)tid * tiles + tile];
         }
-        if (tile > 0) tile_store(own, kTileRun, before + acc);
-        tile_start[tid] = ex;
-        gofs[tid] = first + before;
+        uint64_t* own = state + (int64_t)tile * kRadix + tid;
+        if (CHAINED) {
+            tile_store(own, tile == 0 ? kTileRun : kTileSum, acc);
+            state_next[(int64_t)tile * kRadix + tid] = 0ull;
+            uint32_t ex, first;
+            block_exscan(acc, ex);   // contain barriers; every thread reaches them
+            block_exscan(ctl[pass * kRadix + tid], first);
+            uint32_t before = 0;
+            bool open = tile > 0;
+            for (int64_t t = (int64_t)tile - 1; open;) {
+                uint64_t x[kSortLook];
+#pragma unroll
+                for (int u = 0; u < kSortLook; ++u)
+                    x[u] = t - u >= 0 ? tile_load(state + (t - u) * kRadix + tid) : kTileRun;
+                bool moved = false;
+#pragma unroll
+                for (int u = 0; u < kSortLook; ++u) {
+                    if (!open || (x[u] >> 32) == 0 || (u > 0 && !moved)) {
+                        moved = false;  // not published yet: look again from here
+                        continue;
+                    }
+                    before += (uint32_t)x[u];
+                    moved = true;
+                    --t;
+                    if (x[u] & kTileRun) open = false;
+                }
+                if (open && !moved) __builtin_amdgcn_s_sleep(1);
+            }
+            if (tile > 0) tile_store(own, kTileRun, before + acc);
+            tile_start[tid] = ex;
+            gofs[tid] = first + before;
+        }
     }
     __syncthreads();
 #pragma unroll
@@ -367,7 +430,6 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys
             const uint32_t pos = tile_start[dig] + wcnt[w][dig] + rk[r];
             skeys[pos] = key[r];
             svals[pos] = val[r];
-            sdig[pos] = (uint8_t)dig;
         }
     }
     __syncthreads();
@@ -376,13 +438,14 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys
     for (int i = 0; i < ITEMS; ++i) {
         const int j = i * kBlock + tid;
         if (j < valid) {
-            const uint32_t dg = sdig[j];
+            const K k = skeys[j];
+            const uint32_t dg = (uint32_t)(k >> shift) & 0xFFu;
             const int64_t o = (int64_t)gofs[dg] + (j - (int64_t)tile_start[dg]);
-            okeys[o] = skeys[j];
+            okeys[o] = k;
             ovals[o] = svals[j];
         }
     }
-    if (!last) return;
+    if (!CHAINED || !last) return;
     if (tid == 0) s_last = atomicAdd(&ctl[kSortCtl - 1], 1u) == tiles - 1 ? 1u : 0u;
     __syncthreads();
     if (s_last)
@@ -396,6 +459,7 @@ size_t sort_state_words(int64_t n) {
     return (size_t)(2 * kRadix * std::max<int64_t>(tiles, 1));
 }
 size_t sort_ctl_words() { return kSortCtl; }
+int64_t sort_scan_values(int64_t n) { return n > kSortChained ? (n + 4095) / 4096 * kRadix : 0; }
 
 // Stable LSD sort of (keys, vals) over bits [0, nbits), ping-ponging between the given
 // buffers. n is the element count, or (dn != nullptr) its upper bound with the actual count
@@ -405,11 +469,23 @@ static bool sort_passes(DevState& d, K* keys, int32_t* vals, K* tkeys, int32_t* 
                         int passes, hipStream_t s) {
     constexpr int kTile = kBlock * ITEMS;
     const unsigned tiles = (unsigned)((n + kTile - 1) / kTile);
+    if (n > kSortChained) {
+        uint32_t* table = reinterpret_cast<uint32_t*>(d.sort_state);
+        for (int p = 0; p < passes; ++p) {
+            hipLaunchKernelGGL((k_sort_table<K, ITEMS>), dim3(tiles), dim3(kBlock), 0, s, keys, n, dn, 8 * p, table);
+            scan_values(d, table, table, (int64_t)kRadix * tiles, nullptr, dn, kTile, s);
+            hipLaunchKernelGGL((k_sort_pass<K, ITEMS, false>), dim3(tiles), dim3(kBlock), 0, s, keys, vals, n, dn, p, 0,
+                               table, nullptr, nullptr, tkeys, tvals);
+            std::swap(keys, tkeys);
+            std::swap(vals, tvals);
+        }
+        return passes & 1;
+    }
     uint64_t* state[2] = {d.sort_state, d.sort_state + (size_t)kRadix * tiles};
-    hipLaunchKernelGGL(k_sort_count<K>, dim3(std::min(grid_for(n), 512u)), dim3(kBlock), 0, s, keys, n, dn, passes,
+    hipLaunchKernelGGL(k_sort_count<K>, dim3(std::min(grid_for(n), 1024u)), dim3(kBlock), 0, s, keys, n, dn, passes,
                        kTile, d.sort_ctl, state[0]);
     for (int p = 0; p < passes; ++p) {
-        hipLaunchKernelGGL((k_sort_pass<K, ITEMS>), dim3(tiles), dim3(kBlock), 0, s, keys, vals, n, dn, p,
+        hipLaunchKernelGGL((k_sort_pass<K, ITEMS, true>), dim3(tiles), dim3(kBlock), 0, s, keys, vals, n, dn, p,
                            p == passes - 1 ? 1 : 0, d.sort_ctl, state[p & 1], state[(p + 1) & 1], tkeys, tvals);
         std::swap(keys, tkeys);
         std::swap(vals, tvals);
