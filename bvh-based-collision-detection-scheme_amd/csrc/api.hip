@@ -143,9 +143,9 @@ bool alloc_lists(bvhcd_ctx* c, int64_t ci, int64_t ce, int64_t cp) {
             ok = ok && lalloc(d.fquery[k][b], (size_t)d.front_cap[k]);
         }
     // tile words of the largest sort (front ordering) and of the largest scan (per-node counts, waves or
-    // partition tiles)
+    // the sort's)
     const int64_t max_sort = std::max<int64_t>(T, std::max(d.front_cap[0], d.front_cap[1]));
-    const int64_t max_scan = std::max<int64_t>({T + 2, d.wave_cap, d.front_cap[1] / kAdjTile + 2, sort_scan_values(max_sort)});
+    const int64_t max_scan = std::max<int64_t>({T + 2, d.wave_cap, sort_scan_values(max_sort)});
     d.scan_tiles = (size_t)((max_scan + 4095) / 4096);
     ok = ok && lalloc(d.sort_state, sort_state_words(max_sort)) && lalloc(d.sort_ctl, sort_ctl_words()) &&
          lalloc(d.scan_state, d.scan_tiles) && lalloc(d.scan_ctl, 2) &&
@@ -154,8 +154,6 @@ bool alloc_lists(bvhcd_ctx* c, int64_t ci, int64_t ce, int64_t cp) {
          hipMemsetAsync(d.scan_ctl, 0, 2 * sizeof(uint32_t), c->stream) == hipSuccess;
     ok = ok && lalloc(d.bp, (size_t)d.pair_cap) && lalloc(d.np, (size_t)d.pair_cap) &&
          lalloc(d.pair_tmp, (size_t)d.pair_cap);
-    ok = ok && lalloc(d.adj_cnt, (size_t)(d.front_cap[1] / kAdjTile + 2)) &&
-         lalloc(d.adj_off, (size_t)(d.front_cap[1] / kAdjTile + 2));
     // wave-ordered GENERATE: one chunk record per staging flush (every flush but a wave's last
     // holds more than 128 entries; the last ones may all land in one segment)
     d.chunk_seg_cap = std::max(d.front_cap[0], d.front_cap[1]) / kPairSegs / 128 + d.wave_cap + 16;
@@ -228,7 +226,7 @@ int allocate(bvhcd_ctx* c) {
     ok &= dalloc(c, d.offsets, T + 1);
     ok &= dalloc(c, d.tkmap, T);
     ok &= dalloc(c, d.scene_box, 8);
-    ok &= dalloc(c, d.scene_box_u, 8);
+    ok &= dalloc(c, d.scene_part, 6 * kSceneParts);
     ok &= dalloc(c, d.fsize, 4);
     ok &= dalloc(c, d.intcnt, T + 1);
     ok &= dalloc(c, d.extcnt, T + 2);
@@ -414,10 +412,9 @@ int do_build(bvhcd_ctx* c) {
     DevState& d = c->d;
     const int32_t n = (int32_t)c->T;
     hipStream_t s = c->stream;
-    launch_scene_box(d, n, s);
-    launch_codes(d, n, d.codes, d.prim_idx, s);
+    launch_box_and_codes(d, n, d.codes, d.prim_idx, s);
     radix_sort_u32(d, d.codes, d.prim_idx, d.keys_tmp, d.vals_tmp, n, 30, s);
-    launch_prim_map(d, n, s);
+    launch_leaf_setup(d, n, s);
     if (n >= 2) {
         launch_emit_full(d, n, s);
     } else {
@@ -579,7 +576,9 @@ int run_front(bvhcd_ctx* c, int& front_op) {
     // more per rebuild.)
     const bool order = !is_learned(c->cfg.scheduler);  // node order, else query order
     const bool quality = c->cfg.enable_restructure != 0 && order;
-    if (front_op != BVHCD_FRONT_KEEP && front_op != BVHCD_FRONT_PURE_BVH_CD) d.front_version++;
+    // (REORDER only moves internal entries: the external front's partition and its counts stay valid)
+    if (front_op != BVHCD_FRONT_KEEP && front_op != BVHCD_FRONT_PURE_BVH_CD && front_op != BVHCD_FRONT_REORDER)
+        d.front_version++;
     switch (front_op) {
         case BVHCD_FRONT_PURE_BVH_CD:
             begin(c, S_FRONT);

@@ -323,7 +323,7 @@ void record_frame(bvhcd_batch* b, int bvh_op, unsigned grid) {
         if (radix_sort_u64_dev(d, b->keys, d.prim_idx, b->keys_tmp, d.vals_tmp, n, bits, s))
             hipLaunchKernelGGL(k_copy_sorted, dim3(std::min<unsigned>(grid_for(n), 8192)), dim3(kBlock), 0, s,
                                (int64_t)n, b->keys_tmp, d.vals_tmp, b->keys, d.prim_idx);
-        launch_prim_map(d, n, s);
+        launch_leaf_setup(d, n, s);
         launch_emit_full64(d, b->keys, n, s);
         launch_refit_prep(d, n, s);
     }

@@ -212,7 +212,7 @@ struct DevState {
     uint64_t* sort_state = nullptr; // sort_state_words(): tile words of two passes
     uint32_t* sort_ctl = nullptr;   // sort_ctl_words(): digit counts, counters, zero between sorts
     float* scene_box = nullptr;     // 6 floats (+ pad)
-    uint32_t* scene_box_u = nullptr;// ordered-int reduction scratch, 6 words
+    float* scene_part = nullptr;    // kSceneParts boxes: the workgroups' parts of the scene box
     // fronts: SoA (node id, query leaf), double buffered per kind (0 internal, 1 external)
     uint32_t* fnode[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [kind][buf]
     int32_t* fquery[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
@@ -220,8 +220,6 @@ struct DevState {
     int fcur[2] = {0, 0};           // current buffer per kind
     int64_t front_version = 0;      // host-side: bumped whenever a step changes the front's contents
     int64_t adj_version = -1;       // host-side: front version of the last shared-vertex partition
-    uint32_t* adj_cnt = nullptr;    // partition scratch: shared-vertex entries per tile, then offsets
-    uint32_t* adj_off = nullptr;
     uint32_t* fsize = nullptr;      // [kind*2 + buf] sizes (4 words)
     uint32_t* fcnt = nullptr;       // [kind][kPairSegs * kCntStride] segment counters of a front
                                     // being produced (front_cap is kPairSegs equal segments)
@@ -310,12 +308,13 @@ enum Counter : int {
     C_FREQ_I = 13,     // capacity the last produced internal / external front needed
     C_FREQ_E = 14,
     // words 16..23 hold 64-bit counters (see Counter64)
-    C_ADJ = 24,        // shared-vertex entries heading the current external front (last partition)
     C_NO_IMPLICIT = 25,// the last refit cannot vouch for shared-vertex pairs: a vertex coordinate
                        // above 1e8 in magnitude (or NaN / inf), or boxes given by the caller
     C_BADFACE = 26,    // set_topology: a face vertex id outside its vertex range
     C_WAVE_TOTAL = 27, // wave-ordered production: entries of the list being gathered
     C_WAVE_CHUNKS = 28,// wave-ordered production: chunk records of the list being gathered
+    C_ADJ = 30,        // shared-vertex entries heading the current external front (last partition); the
+                       // next word counts the others meanwhile (both taken by one 64-bit add)
     C_NUM = 32
 };
 enum HostWord : int {
@@ -363,9 +362,9 @@ __device__ inline bool leaves_share_vertex(const DevState& d, int32_t a, int32_t
     return faces_share_vertex(d.lfaces, a, b);
 }
 
+constexpr int kSceneParts = 1024;
 // Launch helpers
 constexpr int kBlock = 256;
-constexpr uint32_t kAdjTile = 16 * kBlock;  // external-front entries per shared-vertex partition block
 inline unsigned grid_for(int64_t n, int block = kBlock) {
     int64_t g = (n + block - 1) / block;
     if (g < 1) g = 1;

@@ -1727,83 +1727,82 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
 }
 
 // ---------------------------------------------------------------- shared-vertex partition
-// Reorders the current external front, stably, into [entries whose two triangles share a vertex |
-// the rest] and records the head length in C_ADJ. Two passes over tiles of kAdjTile entries
-// (count, exclusive scan, scatter into the spare buffer), run by KEEP once per front version.
-
-__global__ void __launch_bounds__(kBlock) k_adj_count(DevState d, FrontIn in, uint32_t* __restrict__ cnt) {
-    __shared__ uint32_t wsum[kWaves];
+// Reorders the current external front into [entries whose two triangles share a vertex | the rest]
+// and leaves the head's length in C_ADJ; run by KEEP once per front version. One pass: a workgroup
+// flags its tile (flags in registers), takes the tile's places with one atomic, the head's from the
+// front's start and the rest's from its end, and reads the entries again to place them. A tile keeps
+// its order; tiles follow one another about as they are dispatched. Bound by the faces gathered per
+// entry (both triangles'), once: 2M cloth, 35M entries 0.30 -> 0.28 ms against counting, a scan and a
+// scatter that tested every entry twice; 41k triangles 40 -> 19 us.
+template <int ITEMS>
+__global__ void __launch_bounds__(kBlock) k_adj_partition(DevState d, FrontIn in, uint32_t* __restrict__ dst_node,
+                                                          int32_t* __restrict__ dst_query, uint32_t* dst_size) {
+    static_assert(ITEMS * kWaves <= kBlock, "one thread per round and wave in the scan");
+    __shared__ uint32_t cnt[ITEMS * kWaves];  // flagged entries before each round's wave
+    __shared__ uint32_t base_head, base_rest;
     const uint32_t ne = min(*in.size[1], in.cap[1]);
-    const uint32_t b0 = blockIdx.x * kAdjTile;
-    uint32_t c = 0;
-    for (uint32_t i = b0 + threadIdx.x; i < min(b0 + kAdjTile, ne); i += kBlock)
-        c += leaves_share_vertex(d, in.query[1][i], (int32_t)in.node[1][i]) ? 1u : 0u;
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off);
-    if (lane_id() == 0) wsum[threadIdx.x >> 6] = c;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int w = 0; w < kWaves; ++w) t += wsum[w];
-        cnt[blockIdx.x] = t;
-    }
-}
-
-__global__ void __launch_bounds__(kBlock) k_adj_scatter(DevState d, FrontIn in, const uint32_t* __restrict__ off,
-                                                        uint32_t* __restrict__ dst_node, int32_t* __restrict__ dst_query,
-                                                        uint32_t* dst_size) {
-    __shared__ uint32_t wa[kWaves], wv[kWaves];
-    const uint32_t ne = min(*in.size[1], in.cap[1]);
-    const uint32_t total_adj = d.ctr[C_ADJ];
-    const uint32_t b0 = blockIdx.x * kAdjTile;
-    const int w = threadIdx.x >> 6;
-    uint32_t run_a = off[blockIdx.x], run_n = total_adj + (b0 - off[blockIdx.x]);
-    for (uint32_t t0 = b0; t0 < min(b0 + kAdjTile, ne); t0 += kBlock) {
-        const uint32_t i = t0 + threadIdx.x;
-        const bool valid = i < ne;
-        uint32_t node = 0;
-        int32_t query = 0;
-        if (valid) {
-            node = in.node[1][i];
-            query = in.query[1][i];
-        }
-        const bool adj = valid && leaves_share_vertex(d, query, (int32_t)node);
-        const uint64_t ma = __ballot(adj), mv = __ballot(valid);
-        if (lane_id() == 0) {
-            wa[w] = (uint32_t)__popcll(ma);
-            wv[w] = (uint32_t)__popcll(mv);
-        }
-        __syncthreads();
-        uint32_t before_a = 0, before_v = 0, tile_a = 0, tile_v = 0;
-        for (int k = 0; k < kWaves; ++k) {
-            if (k < w) {
-                before_a += wa[k];
-                before_v += wv[k];
-            }
-            tile_a += wa[k];
-            tile_v += wv[k];
-        }
-        if (valid) {
-            const uint64_t below = lanes_below();
-            const uint32_t o = adj ? run_a + before_a + (uint32_t)__popcll(ma & below)
-                                   : run_n + (before_v - before_a) + (uint32_t)__popcll(mv & ~ma & below);
-            dst_node[o] = node;
-            dst_query[o] = query;
-        }
-        run_a += tile_a;
-        run_n += tile_v - tile_a;
-        __syncthreads();
-    }
     if (blockIdx.x == 0 && threadIdx.x == 0) *dst_size = ne;
+    const uint64_t b0 = (uint64_t)blockIdx.x * (kBlock * ITEMS);
+    if (b0 >= ne) return;  // block-uniform
+    const uint32_t left = (uint32_t)min<uint64_t>(ne - b0, kBlock * ITEMS);  // the tile's entries
+    const uint32_t* node = in.node[1] + b0;
+    const int32_t* query = in.query[1] + b0;
+    const int w = threadIdx.x >> 6;
+    uint64_t flags = 0;
+#pragma unroll 4
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t i = r * kBlock + threadIdx.x;
+        const bool adj = i < left && leaves_share_vertex(d, query[i], (int32_t)node[i]);
+        flags |= adj ? 1ull << r : 0ull;
+        const uint64_t m = __ballot(adj);
+        if (lane_id() == 0) cnt[r * kWaves + w] = (uint32_t)__popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // exclusive scan of the counts
+        uint32_t carry = 0;
+        for (int g = 0; g < ITEMS * kWaves; g += 64) {
+            const uint32_t v = cnt[g + threadIdx.x];
+            uint32_t x = v;
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t y = __shfl_up(x, off);
+                if ((int)threadIdx.x >= off) x += y;
+            }
+            cnt[g + threadIdx.x] = carry + x - v;
+            carry += __shfl(x, 63);
+        }
+        if (threadIdx.x == 0) {
+            const unsigned long long old =
+                atomicAdd(reinterpret_cast<unsigned long long*>(d.ctr + C_ADJ),
+                          (unsigned long long)carry | (unsigned long long)(left - carry) << 32);
+            base_head = (uint32_t)old;
+            base_rest = ne - (uint32_t)(old >> 32) - (left - carry);
+        }
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t i = r * kBlock + threadIdx.x;
+        const bool adj = (flags >> r) & 1ull;
+        const uint64_t m = __ballot(adj);
+        if (i >= left) continue;
+        const uint32_t before = cnt[r * kWaves + w] + (uint32_t)__popcll(m & lanes_below());  // flagged ones
+        const uint32_t o = adj ? base_head + before : base_rest + (i - before);
+        dst_node[o] = node[i];
+        dst_query[o] = query[i];
+    }
 }
 
 void launch_adj_partition(DevState& d, int32_t n, hipStream_t s) {
     const FrontIn in = cur_front(d);
-    const unsigned tiles = (unsigned)std::max<int64_t>(1, (d.front_cap[1] + kAdjTile - 1) / kAdjTile);
-    hipLaunchKernelGGL(k_adj_count, dim3(tiles), dim3(kBlock), 0, s, d, in, d.adj_cnt);
-    launch_exscan(d, d.adj_cnt, d.adj_off, tiles, d.ctr + C_ADJ, s);
     const int nb = d.fcur[1] ^ 1;
-    hipLaunchKernelGGL(k_adj_scatter, dim3(tiles), dim3(kBlock), 0, s, d, in, d.adj_off, d.fnode[1][nb],
-                       d.fquery[1][nb], d.fsize + 2 + nb);
+    fill_u32(d.ctr + C_ADJ, 2, 0u, s);
+    // tiles of 16384 entries on large scenes: the tiles' atomics follow one another
+    if (n > (1 << 19))
+        hipLaunchKernelGGL(k_adj_partition<64>, dim3(grid_for(d.front_cap[1], 64 * kBlock)), dim3(kBlock), 0, s, d, in,
+                           d.fnode[1][nb], d.fquery[1][nb], d.fsize + 2 + nb);
+    else
+        hipLaunchKernelGGL(k_adj_partition<16>, dim3(grid_for(d.front_cap[1], 16 * kBlock)), dim3(kBlock), 0, s, d, in,
+                           d.fnode[1][nb], d.fquery[1][nb], d.fsize + 2 + nb);
     d.fcur[1] = nb;
     d.adj_version = d.front_version;
 }

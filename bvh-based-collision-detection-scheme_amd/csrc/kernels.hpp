@@ -10,7 +10,7 @@ namespace bvhcd {
 void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 void fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t s);
 void launch_scene_box(DevState& d, int32_t T, hipStream_t s);
-void launch_codes(DevState& d, int32_t T, uint32_t* codes, int32_t* vals, hipStream_t s);
+void launch_box_and_codes(DevState& d, int32_t T, uint32_t* codes, int32_t* vals, hipStream_t s);
 // Scratch: scan_tiles words of d.scan_state for (n + 4095) / 4096 tiles, sort_state_words(n) of
 // d.sort_state for sorts of up to n keys; d.scan_* and d.sort_ctl are zero before the first use.
 size_t sort_state_words(int64_t n);
@@ -66,7 +66,8 @@ constexpr int32_t kRefitTopLds = 4096;
 constexpr int32_t kRefitTopGrid = 64;
 // Capacity (boxes) of the hand-over array between the chunk refit and the top-tree merge.
 inline int64_t refit_tcb_boxes(int64_t T) { return 2 * (int64_t)kRefitTopLds + T / 128; }
-void launch_prim_map(DevState& d, int32_t n, hipStream_t s);
+// After every sort, before the emission and the refit preparation (it sets their start values).
+void launch_leaf_setup(DevState& d, int32_t n, hipStream_t s);
 
 // front.hip
 void launch_pure_cd(DevState& d, int32_t n, hipStream_t s);

@@ -60,7 +60,7 @@ int restructure_subtrees(DevState& d, int32_t n, hipStream_t s, bool prepare_fro
     radix_sort_u64(d, d.r_keys, d.vals_tmp, d.r_keys2, d.prim_map, n, bits, s);
     hipLaunchKernelGGL(k_restr_unpack, dim3(grid_for(n)), dim3(kBlock), 0, s, n, d.r_keys, d.codes);
     hipMemcpyAsync(d.prim_idx, d.vals_tmp, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, s);
-    launch_prim_map(d, n, s);
+    launch_leaf_setup(d, n, s);
     launch_emit_runs(d, n, d.rt_of_leaf, d.r_leaf_lo, d.r_leaf_hi, d.r_split_lo, d.r_split_hi, d.r_base, d.r_keep_par,
                      d.r_keep_mark, s);
     launch_refit_prep(d, n, s);
