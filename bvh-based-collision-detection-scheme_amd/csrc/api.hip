@@ -191,6 +191,7 @@ int allocate(bvhcd_ctx* c) {
     ok &= dalloc(c, d.int_rx, T);
     ok &= dalloc(c, d.int_ry, T);
     ok &= dalloc(c, d.itopo, T);
+    ok &= dalloc(c, d.top_cut, 65);
     ok &= dalloc(c, d.tri_finite, T);
     ok &= dalloc(c, d.lfaces, 3 * T);
     ok &= dalloc(c, d.sa_ref, T);
@@ -272,7 +273,7 @@ int allocate(bvhcd_ctx* c) {
     ok &= dalloc(c, d.rtasks, d.rtask_cap);
     ok &= dalloc(c, d.pcnt, 2 * kPairSegs * kCntStride);
     ok &= dalloc(c, d.fcnt, 2 * kPairSegs * kCntStride);
-    d.wave_cap = (int64_t)grid_for(std::max<int64_t>(T - 1, 1)) * (kBlock / 64);
+    d.wave_cap = max_walk_waves(std::max<int64_t>(T - 1, 1));
     for (int k = 0; k < 2; ++k) ok &= dalloc(c, d.wave_tot[k], (size_t)d.wave_cap);
     ok &= dalloc(c, d.wave_base, (size_t)d.wave_cap);
     ok &= dalloc(c, d.wave_nch, (size_t)d.wave_cap);

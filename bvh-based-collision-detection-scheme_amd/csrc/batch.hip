@@ -427,6 +427,7 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     ok &= balloc(b, d.int_rx, T);
     ok &= balloc(b, d.int_ry, T);
     ok &= balloc(b, d.itopo, T);
+    ok &= balloc(b, d.top_cut, 65);
     ok &= balloc(b, d.tri_finite, T);
     ok &= balloc(b, d.lfaces, 3 * T);
     ok &= balloc(b, d.rp_cstart, (size_t)refit_chunks((int32_t)T) + 1);

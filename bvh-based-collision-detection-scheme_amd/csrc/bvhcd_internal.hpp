@@ -156,6 +156,7 @@ struct DevState {
     uint32_t* int_mark = nullptr;
     int32_t* int_rx = nullptr;
     int32_t* int_ry = nullptr;
+    uint32_t* top_cut = nullptr;    // 65: encoded nodes that cover the tree near its root, [64] = how many
     int4* itopo = nullptr;          // T-1: children and parent as (id << 1 | bit), last leaf: x, y = left,
                                     // right child with bit 0 = leaf (the encoding of escapes), z = parent
                                     // with bit 0 = this node is its right child (negative: root), w = rangey

@@ -465,7 +465,7 @@ static void record_chunks(DevState& d, FrontSink& sk, int kind) {
 // each with its offset in the segments, so the next kernel finds the entries in one load); then one
 // workgroup per producing wave w loads its chunks straight from the segments (chunk c holds the
 // wave's entries c.z .. c.z + count - 1) and orders the run by query with a counting sort in LDS
-// on q - 64 w (the wave's queries are 64 w .. 64 w + 63), writing it once at the scan of the
+// on q - per w (the wave's queries are per w .. per w + per - 1), writing it once at the scan of the
 // wave totals. The order within a query is not kept (fronts are multisets). A run longer than
 // kWaveRunLds entries, or one past the capacity, is written in production order (clamped to the
 // capacity; the overflow bit is set and the front stays a dense prefix). The size becomes the
@@ -492,13 +492,13 @@ __global__ void __launch_bounds__(kBlock) k_chunk_list(DevState d, int kind) {
 }
 constexpr uint32_t kWaveRunLds = 4096;
 constexpr int kOrderBlock = 512;  // LDS allows 4 workgroups per CU: 8 waves each fill it
-__global__ void __launch_bounds__(kOrderBlock) k_wave_order(DevState d, int kind, uint32_t waves,
+__global__ void __launch_bounds__(kOrderBlock) k_wave_order(DevState d, int kind, uint32_t waves, uint32_t per,
                                                        const uint32_t* __restrict__ src_node,
                                                        const int32_t* __restrict__ src_query,
                                                        uint32_t* __restrict__ dst_node,
                                                        int32_t* __restrict__ dst_query, uint32_t* dst_size) {
     __shared__ uint32_t lnode[kWaveRunLds];
-    __shared__ uint32_t lkey[kWaveRunLds];  // (q - 64 w) << 16 | rank among the run's entries of q
+    __shared__ uint32_t lkey[kWaveRunLds];  // (q - per w) << 16 | rank among the run's entries of q
     __shared__ uint32_t cnt[64];
     const uint32_t w = blockIdx.x;
     const uint32_t cap = (uint32_t)min(d.front_cap[kind], (int64_t)0xFFFFFFFF);
@@ -530,7 +530,7 @@ __global__ void __launch_bounds__(kOrderBlock) k_wave_order(DevState d, int kind
     }
     if (threadIdx.x < 64) cnt[threadIdx.x] = 0u;
     __syncthreads();
-    const int32_t q0 = (int32_t)(w * 64u);
+    const int32_t q0 = (int32_t)(w * per);
     for (uint32_t c = c0 + wid; c < c1; c += kOrderBlock / 64) {
         const uint4 ch = d.clist[c];
         const int64_t src = (int64_t)((uint64_t)ch.x | (uint64_t)ch.y << 32);
@@ -574,14 +574,14 @@ __global__ void __launch_bounds__(kOrderBlock) k_wave_order(DevState d, int kind
     }
 }
 
-static void front_finish_waves(DevState& d, int kind, int64_t waves, hipStream_t s) {
+static void front_finish_waves(DevState& d, int kind, int64_t waves, uint32_t per, hipStream_t s) {
     const int c = d.fcur[kind], nb = c ^ 1;  // the production is in the spare buffer's segments
     launch_exscan(d, d.wave_tot[kind], d.wave_base, waves, d.ctr + C_WAVE_TOTAL, s);
     fill_u32(d.wave_nch, waves, 0u, s);
     hipLaunchKernelGGL(k_chunk_count, dim3(512), dim3(kBlock), 0, s, d, kind);
     launch_exscan(d, d.wave_nch, d.wave_cbase, waves, d.ctr + C_WAVE_CHUNKS, s);
     hipLaunchKernelGGL(k_chunk_list, dim3(512), dim3(kBlock), 0, s, d, kind);
-    hipLaunchKernelGGL(k_wave_order, dim3((unsigned)waves), dim3(kOrderBlock), 0, s, d, kind, (uint32_t)waves,
+    hipLaunchKernelGGL(k_wave_order, dim3((unsigned)waves), dim3(kOrderBlock), 0, s, d, kind, (uint32_t)waves, per,
                        d.fnode[kind][nb], d.fquery[kind][nb], d.fnode[kind][c], d.fquery[kind][c],
                        d.fsize + 2 * kind + c);
 }
@@ -683,20 +683,20 @@ __device__ inline int kth_set_lane(uint64_t m, uint32_t k) {
 // lanes sharing the work: a query's walk from `cur` to `stop` is, at an overlapping internal
 // node nd, nd's subtree followed by the walk from nd's escape to `stop`. So a lane at such a node
 // can hand the second part to an idle lane (its own walk then stops at nd's escape) — the walks
-// of 64 queries end at very different times (the longest is ~1.8x the mean on the folded 2M
+// of a wave's `per` queries end at very different times (the longest is ~1.8x the mean on the folded 2M
 // cloth), and without this the wave waits for its longest one. The nodes tested, the entries
-// and the pairs are those of the 64 queries' own walks; only their order changes.
+// and the pairs are those of the queries' own walks; only their order changes.
 template <bool FRONT>
-__global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, DevState d, FrontSink fi, FrontSink fe) {
+__global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, uint32_t per, DevState d, FrontSink fi, FrontSink fe) {
     __shared__ Stages st;
     stages_init(st);
     const Out out = make_out(st, fi, fe, d);
     const int lane = lane_id();
     const int32_t nq = d.inter ? d.nq : n - 1;
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t i = (int32_t)((blockIdx.x * kWaves + (threadIdx.x >> 6)) * per) + lane;
     // self-CD: query leaf i walks the leaves after it (from lca[i + 1], its record's escape);
     // inter-object: every query walks the whole tree from its root lca[0]
-    bool act = i < nq;
+    bool act = lane < (int)per && i < nq;
     int32_t qi = i, cur = -1, stop = -1, spine = -1;  // spine: bottom of the spine being descended
     Box qb{};
     if (act) {
@@ -781,16 +781,17 @@ __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, DevState d, Fron
 }
 
 // ---------------------------------------------------------------- pairs of 64 queries at a time
-// The overlapping leaf pairs (q, j > q) of a whole tree, without a front. A wave takes 64 queries
-// (neighbouring sorted leaves) together and works in two steps:
-//  * nodes: the tree from its root, 64 nodes per round off a per-wave LDS stack, each lane testing
+// The overlapping leaf pairs (q, j > q) of a whole tree, without a front. A wave takes `size` (up to 64)
+// queries (neighbouring sorted leaves) together and works in two steps:
+//  * nodes: the tree from a cut of up to 64 nodes near its root, 64 nodes per round off a per-wave LDS stack, each lane testing
 //    one node against the boxes of the 64 queries and dropping subtrees that hold no leaf after the
 //    first query. A run of neighbouring leaves can jump (Morton order), and one box around a jump
 //    covers everything between: the run is cut at its three widest jumps and a node is tested
 //    against the four pieces' boxes (2M-triangle folded cloth: 481 nodes per wave instead of 793,
 //    the worst wave 2281 instead of 59425);
-//  * leaves: each leaf reached (170 per wave there) is loaded once for the wave (scalar load) and
-//    tested by every lane against its own query; hits go to the wave's LDS list.
+//  * leaves: each leaf reached (170 per wave there) is tested by every lane against its own query, its
+//    box kept in LDS (STAGED) or loaded once more for the wave through the scalar cache; hits go to
+//    the wave's LDS list.
 // Every node test serves 64 queries and every leaf record is fetched once per wave, where a walk
 // or a front entry per query fetches two 32-byte records per test. A pair is found exactly when the
 // leaves' boxes overlap, as in a query's own walk: a node's box holds its leaves' boxes and a piece's
@@ -799,19 +800,24 @@ __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, DevState d, Fron
 // skip_adj: pairs of triangles that share a vertex are removed when the LDS list is flushed (64 pairs
 // per step; the query's vertex ids come from its lane).
 // Bound by instruction issue (61 % of the VALU and 63 % of the scalar slots busy; half the node
-// rounds run with few nodes). Folded cloths: 180k triangles 185 -> 145 us (against the queries' own
+// rounds run with few nodes). Folded cloths: 180k triangles 185 -> 111 us (against the queries' own
 // walks sharing a wave's lanes), 64 scenes of 2.6M triangles 1.04 -> 0.56 ms (against a walk per
 // lane). KEEP's test of a front stays where there is one: 0.56 ms against 0.60 ms here on the 2M
 // cloth, and 12 us against 43 us on 2,560 triangles, where the tree's depth in rounds is what counts.
 constexpr uint32_t kGroupStack = 512;  // encoded nodes per wave (2 KB)
-constexpr uint32_t kGroupStage = 512;  // staged pairs per wave (4 KB): flushes of 257..512 pairs
 constexpr int kGroupPieces = 4;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef BVHCD_LDS f32x4 lds_f32x4;
+template <bool STAGED>
 struct GroupLds {
+    static constexpr uint32_t kStage = STAGED ? 256 : 512;  // staged pairs per wave
+    f32x4 box[kWaves][STAGED ? 128 : 1][2];  // of the leaves reached: (lo, leaf id), (hi, -)
+    uint32_t cand[kWaves][STAGED ? 1 : 128]; // or their ids alone
     uint32_t stack[kWaves][kGroupStack];
-    uint32_t cand[kWaves][128];        // leaves reached, tested 64 at a time
-    int2 pairs[kWaves][kGroupStage];
+    int2 pairs[kWaves][kStage];
     uint32_t fill[kWaves][2];          // [1]: segment rotor (stage_flush)
 };
+typedef const __attribute__((address_space(4))) float4 const_float4;  // loaded through the scalar cache
 __device__ inline float lane_f(float v, int lane) {
     return i2f(__builtin_amdgcn_readlane(f2i(v), lane));
 }
@@ -819,15 +825,22 @@ __device__ inline uint32_t wave_max(uint32_t v) {
     for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
     return v;
 }
-typedef const __attribute__((address_space(4))) float4 const_float4;  // loaded through the scalar cache
+__device__ inline void wave_lds_order() {  // LDS operations of one wave complete in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
-template <bool BATCH>
-__global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
+template <bool BATCH, bool STAGED>
+__global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, DevState d,
                                                      const uint64_t* __restrict__ keys,
                                                      const int32_t* __restrict__ scene_last) {
-    __shared__ GroupLds lds;
+    constexpr uint32_t kGroupStage = GroupLds<STAGED>::kStage;
+    constexpr int kAtOnce = STAGED ? 2 : 4;  // leaves loaded together
+    __shared__ GroupLds<STAGED> lds;
     const int w = threadIdx.x >> 6, lane = lane_id();
     lds_u32* const stk = (lds_u32*)lds.stack[w];
+    lds_f32x4* const box = (lds_f32x4*)lds.box[w];
     lds_u32* const cand = (lds_u32*)lds.cand[w];
     lds_int2* const sb = (lds_int2*)lds.pairs[w];
     lds_u32* const sf = (lds_u32*)lds.fill[w];
@@ -836,13 +849,13 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
     uint32_t* const ovf = &d.ctr[C_OVF];
     const bool drop_adj = d.skip_adj != 0;
     // each XCD takes one contiguous eighth of the groups; the grid is a multiple of the XCDs
-    const uint32_t groups = ((uint32_t)n + 63u) / 64u, share = (groups + kXcds - 1) / kXcds;
+    const uint32_t groups = ((uint32_t)n + size - 1u) / size, share = (groups + kXcds - 1) / kXcds;
     const uint32_t xcd = blockIdx.x % kXcds, end_gi = min((xcd + 1) * share, groups);
     uint32_t visits = 0;
     for (uint32_t gi = xcd * share + (blockIdx.x / kXcds) * kWaves + w; gi < end_gi;  // wave-uniform
          gi += gridDim.x / kXcds * kWaves) {
-        const int32_t g0 = (int32_t)(gi * 64u), q = g0 + lane;
-        const bool valid = q < n;
+        const int32_t g0 = (int32_t)(gi * size), q = g0 + lane;
+        const bool valid = (uint32_t)lane < size && q < n;
         Box qb = empty_box();
         int32_t after = INT32_MAX, last = n - 1;  // this lane's leaves: (after, last]
         int32_t f0 = 0, f1 = 0, f2 = 0;           // its triangle's vertices
@@ -859,11 +872,11 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
         }
         // the wave's last leaf (scenes follow one another in leaf order)
         const int32_t glast =
-            BATCH ? __builtin_amdgcn_readlane(last, min(63, n - 1 - g0)) : n - 1;
+            BATCH ? __builtin_amdgcn_readlane(last, min((int32_t)size - 1, n - 1 - g0)) : n - 1;
         // cut the 64 queries at their widest jumps between box centres
         const float cx = qb.mnx + qb.mxx, cy = qb.mny + qb.mxy, cz = qb.mnz + qb.mxz;
         const float gap = fabsf(__shfl_down(cx, 1) - cx) + fabsf(__shfl_down(cy, 1) - cy) + fabsf(__shfl_down(cz, 1) - cz);
-        uint32_t key = lane < 63 && q + 1 < n ? (((uint32_t)f2i(gap) & 0x7FFFFFC0u) | (uint32_t)lane) : 0u;
+        uint32_t key = lane + 1 < (int)size && q + 1 < n ? (((uint32_t)f2i(gap) & 0x7FFFFFC0u) | (uint32_t)lane) : 0u;
         uint64_t heads = 1ull;  // first lanes of the pieces
 #pragma unroll
         for (int c = 1; c < kGroupPieces; ++c) {
@@ -937,27 +950,35 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
             }
             fill += (uint32_t)__popcll(m);
         };
-        // tests the first k (<= 64) of the leaves reached, four loaded at a time
+        // tests the first k (<= 64) of the leaves reached, kAtOnce loaded together (what lies past the
+        // k-th is some leaf and is not counted)
         auto test_leaves = [&](uint32_t k) {
-            const int32_t cv = (int32_t)cand[min((uint32_t)lane, k - 1u)];
-            for (uint32_t c = 0; c < k; c += 4) {
-                if (fill > kGroupStage - 256u) flush();
-                float4 lo[4], hi[4];
-                int32_t j[4];
+            const int32_t cv = STAGED ? 0 : (int32_t)cand[min((uint32_t)lane, k - 1u)];
+            for (uint32_t c = 0; c < k; c += kAtOnce) {
+                if (fill > kGroupStage - 64u * kAtOnce) flush();
+                float4 lo[kAtOnce], hi[kAtOnce];
+                int32_t j[kAtOnce];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    j[u] = __builtin_amdgcn_readlane(cv, (int)(c + u));
-                    const_float4* r = (const_float4*)(uintptr_t)&d.leaf[j[u]];
-                    lo[u] = make_float4(r[0].x, r[0].y, r[0].z, r[0].w);
-                    hi[u] = make_float4(r[1].x, r[1].y, r[1].z, r[1].w);
+                for (int u = 0; u < kAtOnce; ++u) {
+                    if (STAGED) {  // broadcast reads
+                        const f32x4 a = box[2 * (c + u)], b = box[2 * (c + u) + 1];
+                        lo[u] = make_float4(a.x, a.y, a.z, 0.f);
+                        hi[u] = make_float4(b.x, b.y, b.z, 0.f);
+                        j[u] = f2i(a.w);
+                    } else {
+                        j[u] = __builtin_amdgcn_readlane(cv, (int)(c + u));
+                        const_float4* r = (const_float4*)(uintptr_t)&d.leaf[j[u]];
+                        lo[u] = make_float4(r[0].x, r[0].y, r[0].z, 0.f);
+                        hi[u] = make_float4(r[1].x, r[1].y, r[1].z, 0.f);
+                    }
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
+                for (int u = 0; u < kAtOnce; ++u)
                     emit(c + u < k && j[u] > after && (!BATCH || j[u] <= last) && box_overlap(qb, lo[u], hi[u]), j[u]);
             }
         };
-        uint32_t top = 1, ncand = 0;  // wave-uniform
-        if (lane == 0) stk[0] = (uint32_t)d.leaf_lca[0];
+        uint32_t top = d.top_cut[64], ncand = 0;  // wave-uniform
+        stk[lane] = d.top_cut[lane];
         // every node enters the stack at most once; the bound only guards against a corrupted tree
         // (flag 16, reported as a device error, instead of a hang)
         const int64_t limit = 2 * d.maxT + 16;
@@ -972,11 +993,11 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
             const int32_t e = act ? (int32_t)stk[top + lane] : 0, nd = e >> 1;
             const bool leaf = e & 1;
             bool hit = false;
-            float4 hi = make_float4(0.f, 0.f, 0.f, 0.f);
+            float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
             int4 tp = make_int4(0, 0, 0, 0);
             if (act) {
                 const NodeRec* r = leaf ? &d.leaf[nd] : &d.inode[nd];
-                const float4 lo = r->lo;
+                lo = r->lo;
                 hi = r->hi;
                 if (!leaf) tp = d.itopo[nd];
                 ++visits;
@@ -1007,7 +1028,7 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
                             if (lane == 0) atomicOr(ovf, 16u);
                             break;
                         }
-                        if (fill > kGroupStage - 256u) flush();
+                        if (fill > kGroupStage - 64u) flush();
                         bool h = false;
                         int32_t j = 0;
                         if (cur != stop) {
@@ -1029,14 +1050,31 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
                 }
             }
             if (ml) {
-                if (hit && leaf) cand[ncand + (uint32_t)__popcll(ml & lanes_below())] = (uint32_t)nd;
+                if (hit && leaf) {
+                    const uint32_t slot = ncand + (uint32_t)__popcll(ml & lanes_below());
+                    if (STAGED) {
+                        box[2 * slot] = f32x4{lo.x, lo.y, lo.z, i2f(nd)};
+                        box[2 * slot + 1] = f32x4{hi.x, hi.y, hi.z, 0.f};
+                    } else {
+                        cand[slot] = (uint32_t)nd;
+                    }
+                }
                 ncand += (uint32_t)__popcll(ml);
+                wave_lds_order();
             }
             if (ncand >= 64u || (top == 0u && ncand > 0u)) {
                 test_leaves(min(ncand, 64u));
                 const uint32_t rest = ncand > 64u ? ncand - 64u : 0u;
-                const uint32_t v = (uint32_t)lane < rest ? cand[64 + lane] : 0u;
-                if ((uint32_t)lane < rest) cand[lane] = v;
+                if ((uint32_t)lane < rest) {
+                    if (STAGED) {
+                        const f32x4 a = box[2 * (64 + lane)], b = box[2 * (64 + lane) + 1];
+                        box[2 * lane] = a;
+                        box[2 * lane + 1] = b;
+                    } else {
+                        cand[lane] = cand[64 + lane];
+                    }
+                }
+                wave_lds_order();
                 ncand = rest;
                 if (top == 0u && ncand > 0u) {  // the last round's overhang
                     test_leaves(ncand);
@@ -1049,14 +1087,45 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, DevState d,
     add_visits(d, visits);
 }
 
+// Queries per wave. Small scenes are bound by their heaviest wave, large ones by the node tests, which
+// 64 queries share: pure traversal, us, with 64 / 32 / 16 / 8: 2.6k 41 / 34 / 28 / 25, 41k 50 / 41 / 38 / 52,
+// 65k 114 / 95 / 78 / 80, 180k 134 / 111 / 125 / 178, 522k 345 / 350 / 457 / 641, 2.1M 693 / 877 / 1310.
+static uint32_t group_size(int32_t n) {
+    return n <= 4096 ? 8u : n <= 3 << 15 ? 16u : n <= 1 << 18 ? 32u : 64u;
+}
 // Workgroups of k_group_cd, one group per wave: the same number for each XCD's share.
 static unsigned group_grid(int32_t n) {
-    const unsigned share = (((unsigned)n + 63u) / 64u + kXcds - 1) / kXcds;
+    const unsigned g = group_size(n), share = (((unsigned)n + g - 1u) / g + kXcds - 1) / kXcds;
     return kXcds * ((share + kWaves - 1) / kWaves);
+}
+
+// The leaves' boxes staged in LDS up to kGroupStaged leaves: there few waves run and each waits for its
+// loads; on larger scenes the LDS would cost resident waves (staged / reloaded, us: 180k 131 / 146, 522k
+// 337 / 348, 1.2M 506 / 467, 8.4M 1997 / 1846).
+constexpr int32_t kGroupStaged = 1 << 19;
+template <bool BATCH>
+static void launch_group_cd(DevState& d, int32_t n, unsigned grid, const uint64_t* keys, const int32_t* scene_last,
+                            hipStream_t s) {
+    if (n <= kGroupStaged)
+        hipLaunchKernelGGL((k_group_cd<BATCH, true>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
+    else
+        hipLaunchKernelGGL((k_group_cd<BATCH, false>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
 }
 
 // Queries of a traversal: the leaves before the last one (self-CD) or the other object's leaves.
 static int64_t query_count(const DevState& d, int32_t n) { return d.inter ? d.nq : n - 1; }
+// Queries a wave of k_traverse starts with; its other lanes take parts of their walks over. With few
+// waves the longest wave is the kernel's time, with enough of them full waves do the least: GENERATE in
+// query order, us, with 64 / 32 / 16: 2.6k 128 / 103 / 87, 41k 154 / 135 / 123, 65k 349 / 250 / 197,
+// 180k 342 / 275 / 297, 522k 1276 / 960 / 898, 1.2M 1600 / 1493 / 1677, 2.1M 2189 / 2253 / 2742.
+uint32_t walk_queries(int64_t nq) { return nq <= 3 << 18 ? 16u : nq <= 3 << 19 ? 32u : 64u; }
+static unsigned walk_grid(int64_t nq) { return grid_for(nq, (int)(kWaves * walk_queries(nq))); }
+int64_t max_walk_waves(int64_t T) {
+    int64_t w = 1;
+    for (const int64_t nq : {T, std::min<int64_t>(T, 3 << 19), std::min<int64_t>(T, 3 << 18)})
+        w = std::max<int64_t>(w, (int64_t)walk_grid(nq) * kWaves);
+    return w;
+}
 
 // Self-CD over boxes made from the vertices.
 static bool group_ok(const DevState& d) { return !d.inter && !d.pbox; }
@@ -1065,9 +1134,11 @@ void launch_pure_cd(DevState& d, int32_t n, hipStream_t s) {
     reset_step_counters(d, s);
     const int64_t nq = query_count(d, n);
     if (group_ok(d) && nq > 0)
-        hipLaunchKernelGGL(k_group_cd<false>, dim3(group_grid(n)), dim3(kBlock), 0, s, n, d, nullptr, nullptr);
-    else if (nq > 0)
-        hipLaunchKernelGGL(k_traverse<false>, dim3(grid_for(nq)), dim3(kBlock), 0, s, n, d, null_sink(), null_sink());
+        launch_group_cd<false>(d, n, group_grid(n), nullptr, nullptr, s);
+    else if (nq > 0) {
+        hipLaunchKernelGGL(k_traverse<false>, dim3(walk_grid(nq)), dim3(kBlock), 0, s, n, walk_queries(nq), d,
+                           null_sink(), null_sink());
+    }
 }
 
 // ---------------------------------------------------------------- batched scenes
@@ -1080,7 +1151,7 @@ void launch_batch_cd(DevState& d, int32_t n, const uint64_t* keys, const int32_t
                      hipStream_t s) {
     reset_step_counters(d, s);
     const unsigned g = std::min(group_grid(n), kXcds * std::max(grid / kXcds, 1u));
-    if (n >= 2) hipLaunchKernelGGL(k_group_cd<true>, dim3(g), dim3(kBlock), 0, s, n, d, keys, scene_last);
+    if (n >= 2) launch_group_cd<true>(d, n, g, keys, scene_last, s);
 }
 
 // ---------------------------------------------------------------- ordering
@@ -1303,23 +1374,24 @@ void launch_order_fronts(DevState& d, int32_t n, hipStream_t s, bool generated) 
 }
 
 // Without node ordering, the front comes out ordered by query without a global sort: the
-// production is gathered in wave order (each wave's 64 consecutive queries keep their entries
+// production is gathered in wave order (each wave's consecutive queries keep their entries
 // together, the waves following in query order), then each wave's run is sorted by query.
 void launch_generate(DevState& d, int32_t n, hipStream_t s, bool order) {
     reset_step_counters(d, s);
     front_begin(d, s);
     FrontSink fi = next_sink(d, 0), fe = next_sink(d, 1);
     const int64_t nq = query_count(d, n);
-    const unsigned grid = nq > 0 ? grid_for(nq) : 0u;
+    const uint32_t per = walk_queries(nq);
+    const unsigned grid = nq > 0 ? walk_grid(nq) : 0u;
     const bool waves = !order && nq > 0 && wave_ordered_ok(d, (int64_t)grid * kWaves);
     if (waves) {
         record_chunks(d, fi, 0);
         record_chunks(d, fe, 1);
     }
-    if (nq > 0) hipLaunchKernelGGL(k_traverse<true>, dim3(grid), dim3(kBlock), 0, s, n, d, fi, fe);
+    if (nq > 0) hipLaunchKernelGGL(k_traverse<true>, dim3(grid), dim3(kBlock), 0, s, n, per, d, fi, fe);
     if (waves) {
-        front_finish_waves(d, 0, (int64_t)grid * kWaves, s);
-        front_finish_waves(d, 1, (int64_t)grid * kWaves, s);
+        front_finish_waves(d, 0, (int64_t)grid * kWaves, per, s);
+        front_finish_waves(d, 1, (int64_t)grid * kWaves, per, s);
     } else {
         front_finish(d, 0, false, s);
         front_finish(d, 1, false, s);

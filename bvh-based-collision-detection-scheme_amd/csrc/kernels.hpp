@@ -71,6 +71,7 @@ void launch_leaf_setup(DevState& d, int32_t n, hipStream_t s);
 
 // front.hip
 void launch_pure_cd(DevState& d, int32_t n, hipStream_t s);
+int64_t max_walk_waves(int64_t T);  // producing waves of a GENERATE over up to T queries
 // order = false keeps the emission order (entries of neighbouring queries together) and skips
 // the node-id sort and bucket offsets that only the front-quality heuristic reads.
 void launch_generate(DevState& d, int32_t n, hipStream_t s, bool order = true);  // traversal + ordering

@@ -1249,8 +1249,37 @@ __device__ inline void rp_top_segments(const DevState& d, int32_t tcb_cap) {
     }
 }
 
-// The chunk entries (one thread per leaf) and, by the first workgroup meanwhile, the top-tree list:
-// neither reads what the other writes.
+// Cut of the tree with at most 64 nodes, a level per step while all of a level's nodes can be
+// replaced by their children: where the pair traversal's waves start. One wave; a chain of equal
+// codes gains one node per step, so the steps are bounded.
+__device__ inline void rp_top_cut(const DevState& d) {
+    __shared__ int32_t node[64];
+    const int lane = threadIdx.x;
+    uint32_t cnt = 1;
+    if (lane == 0) node[0] = d.leaf_lca[0];
+    for (int step = 0; step < 8; ++step) {
+        __syncthreads();
+        const int32_t e = lane < (int)cnt ? node[lane] : 1;
+        const bool inner = lane < 64 && !(e & 1);
+        const uint64_t m = __ballot(inner);  // only the first wave's is used
+        __syncthreads();
+        if (lane < 64) {
+            const uint32_t more = (uint32_t)__popcll(m);
+            if (cnt + more <= 64u && inner) {
+                const int4 tp = d.itopo[e >> 1];
+                node[lane] = tp.x;
+                node[cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = tp.y;
+            }
+            if (cnt + more <= 64u) cnt += more;
+        }
+    }
+    __syncthreads();
+    if (lane < 64) d.top_cut[lane] = lane < (int)cnt ? (uint32_t)node[lane] : 1u;
+    if (lane == 0) d.top_cut[64] = cnt;
+}
+
+// The chunk entries (one thread per leaf) and, by the first two workgroups meanwhile, the top-tree
+// list and the cut near the root: none reads what another writes.
 __global__ void __launch_bounds__(kTopBlock) k_rp_lists(int32_t n, DevState d, int32_t tcb_cap) {
     if (blockIdx.x == 0) {
         rp_top_sort(d);
@@ -1258,7 +1287,11 @@ __global__ void __launch_bounds__(kTopBlock) k_rp_lists(int32_t n, DevState d, i
         rp_top_segments(d, tcb_cap);
         return;
     }
-    const int32_t x = (int32_t)(blockIdx.x - 1) * kTopBlock + (int32_t)threadIdx.x;
+    if (blockIdx.x == 1) {
+        rp_top_cut(d);
+        return;
+    }
+    const int32_t x = (int32_t)(blockIdx.x - 2) * kTopBlock + (int32_t)threadIdx.x;
     if (x < n) rp_walk(d, x);
 }
 
@@ -1269,7 +1302,7 @@ void launch_refit_prep(DevState& d, int32_t n, hipStream_t s) {
     if (n < 1) return;
     const int32_t nc = refit_chunks(n);  // start values: launch_leaf_setup
     hipLaunchKernelGGL(k_rp_starts, dim3(grid_for(n)), dim3(kBlock), 0, s, n, d);
-    hipLaunchKernelGGL(k_rp_lists, dim3(grid_for(n, kTopBlock) + 1), dim3(kTopBlock), 0, s, n, d, refit_tcb_boxes(n));
+    hipLaunchKernelGGL(k_rp_lists, dim3(grid_for(n, kTopBlock) + 2), dim3(kTopBlock), 0, s, n, d, refit_tcb_boxes(n));
     hipLaunchKernelGGL(k_rp_chunk_sort, dim3(nc), dim3(kBlock), 0, s, d);
 }
 
