@@ -204,7 +204,12 @@ __global__ void __launch_bounds__(kBlock) k_scan(const uint32_t* in, int64_t n, 
         if (base + i < n) out[base + i] = run;
         run += v[i];
     }
-    if (threadIdx.x == 0) s_last = atomicAdd(&ctl[1], 1u) == tiles - 1 ? 1u : 0u;
+    if (threadIdx.x == 0) {
+        // the tile's word must have arrived before the tile counts as done: the last workgroup's
+        // clearing must not be overtaken by it (this thread's wave wrote the word)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        s_last = atomicAdd(&ctl[1], 1u) == tiles - 1 ? 1u : 0u;
+    }
     __syncthreads();
     if (s_last) {
         for (uint32_t t = threadIdx.x; t < tiles; t += kBlock) tile_store(&state[t], 0ull, 0u);
