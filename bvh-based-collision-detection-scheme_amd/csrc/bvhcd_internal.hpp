@@ -14,6 +14,7 @@ namespace bvhcd {
 
 constexpr int kPairSegs = 64;   // pair-list segments (one append counter each)
 constexpr int kCntStride = 32;  // words between two segment counters (128 bytes)
+constexpr int kVisitWord = 4;   // words 4, 5 of a broad-phase segment's counter block: node tests
 constexpr int kDroppedWord = 2; // word of a list's counter block: entries no segment had room for
 
 // ------------------------------------------------------------------ node records (HBM layout)
@@ -329,9 +330,16 @@ enum Counter64 : int {
     C64_NUM = 4
 };
 __host__ __device__ inline uint64_t* ctr64(uint32_t* ctr) { return reinterpret_cast<uint64_t*>(ctr + 16); }
+// Node tests of the last step, in kPairSegs 64-bit words each in the cache line of a broad-phase
+// segment counter: one word for all took an atomic per workgroup at about 80 per us, 0.2 ms of a
+// 16384-workgroup KEEP.
+__device__ inline unsigned long long* visit_word(const DevState& d, uint32_t g) {
+    return reinterpret_cast<unsigned long long*>(d.pcnt + g * kCntStride + kVisitWord);
+}
 // Zeroes a step's output counters (pair-list segment counters, pair totals, overflow flags,
 // implicit pairs, node tests); lane g of one wave of 64 threads.
 __device__ inline void zero_step_counters(const DevState& d, int g) {
+    *visit_word(d, g) = 0ull;
     d.pcnt[g * kCntStride] = 0u;                // broad-phase segment counters
     d.pcnt[(kPairSegs + g) * kCntStride] = 0u;  // narrow-phase segment counters
     if (g == 0) {

@@ -377,18 +377,13 @@ __device__ uint32_t stackless(const DevState& d, const Out& out, int32_t qi, con
     return visits;
 }
 
-// Block-reduced visit count, one 64-bit atomic per block (blocks of up to 16 waves).
+// A wave's node tests, added to one of the kPairSegs visit words (beside the broad-phase segment
+// counters) which pair_totals sums.
 __device__ inline void add_visits(const DevState& d, uint32_t v) {
-    __shared__ uint64_t red[16];
     uint64_t x = v;
     for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off);
-    if (lane_id() == 0) red[threadIdx.x >> 6] = x;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t t = 0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
-        if (t) atomicAdd((unsigned long long*)&ctr64(d.ctr)[C64_VISITS], (unsigned long long)t);
-    }
+    const uint32_t b = blockIdx.x, slot = (b / kXcds * (blockDim.x >> 6) + (threadIdx.x >> 6) + b % kXcds * kXcds) % kPairSegs;
+    if (lane_id() == 0 && x) atomicAdd(visit_word(d, slot), (unsigned long long)x);
 }
 
 // ---------------------------------------------------------------- host-side front views
@@ -2172,6 +2167,11 @@ __device__ inline void pair_totals(const DevState& d, int narrow) {  // two wave
     for (int off = 32; off > 0; off >>= 1) {
         v += __shfl_down(v, off);
         m = max(m, __shfl_down(m, off));
+    }
+    if (kind == 0) {
+        uint64_t t = *visit_word(d, g);
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off);
+        if (g == 0) ctr64(d.ctr)[C64_VISITS] = t;
     }
     if (g == 0) {
         const uint32_t impl = d.ctr[C_IMPLICIT];
