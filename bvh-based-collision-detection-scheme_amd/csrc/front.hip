@@ -216,11 +216,14 @@ __device__ inline void stage_final(const Sink& sk, uint32_t* ovf, lds_int2* sbuf
 
 // Per-block staging storage for up to three lists; fill[list][wave] = {staged, rotor, recorded
 // entries of a wave-ordered production}.
-struct Stages {
-    int2 buf[3][kWaves][kStage3];
+template <uint32_t CAP>
+struct StagesT {
+    int2 buf[3][kWaves][CAP];
     uint32_t fill[3][kWaves][3];
 };
-__device__ inline void stages_init(Stages& st) {
+using Stages = StagesT<kStage3>;
+template <uint32_t CAP>
+__device__ inline void stages_init(StagesT<CAP>& st) {
     const int w = threadIdx.x >> 6;
     if (lane_id() < 3) {
         st.fill[lane_id()][w][0] = 0;
@@ -306,7 +309,8 @@ __device__ inline Out make_out(StagesBPT<W>& st, const DevState& d) {
     return o;
 }
 
-__device__ inline Out make_out(Stages& st, const FrontSink& fi, const FrontSink& fe, const DevState& d) {
+template <uint32_t CAP>
+__device__ inline Out make_out(StagesT<CAP>& st, const FrontSink& fi, const FrontSink& fe, const DevState& d) {
     Out o;
     o.fi = fi;
     o.fe = fe;
@@ -317,7 +321,7 @@ __device__ inline Out make_out(Stages& st, const FrontSink& fi, const FrontSink&
         o.sb[k] = (lds_int2*)st.buf[k][w];
         o.sf[k] = (lds_u32*)st.fill[k][w];
     }
-    o.scap = kStage3;
+    o.scap = CAP;
     o.lfaces = d.lfaces;
     o.skip_adj = d.skip_adj;
     return o;
@@ -1396,140 +1400,180 @@ void launch_generate(DevState& d, int32_t n, hipStream_t s, bool order) {
     d.front_by_query = order ? 0 : 1;
 }
 
+// ---------------------------------------------------------------- per-wave stacks of node tests
+constexpr uint32_t kDescStack = 512;
+template <int W, uint32_t CAP = kDescStack>
+struct DescStack {
+    int2 item[W][CAP];  // (query, node << 1 | leaf)
+    uint32_t top[W];
+};
+
+// Pushes (q, node enc) for the lanes with pred set; returns false for a lane whose item did not
+// fit (it must then test that node itself). Called by all active lanes of the wave.
+template <uint32_t CAP = kDescStack>
+__device__ inline bool desc_push(lds_int2* stk, lds_u32* top, bool pred, int32_t q, int32_t enc) {
+    const uint64_t m = __ballot(pred);
+    if (m == 0) return true;
+    const uint32_t t = *top;
+    const uint32_t rank = (uint32_t)__popcll(m & lanes_below());
+    const bool fits = t + rank < CAP;
+    if (pred && fits) {
+        stk[t + rank].x = q;
+        stk[t + rank].y = enc;
+    }
+    const uint32_t pushed = (uint32_t)__popcll(__ballot(pred && fits));
+    if (lane_id() == __ffsll((long long)__ballot(1)) - 1) *top = t + pushed;
+    return fits || !pred;
+}
+
+// Takes up to one item per active lane off the wave's stack; returns the number taken.
+__device__ inline uint32_t desc_pop(lds_int2* stk, lds_u32* top, bool& active, int32_t& q, int32_t& enc) {
+    const uint64_t m = __ballot(1);
+    const uint32_t t = *top, rank = (uint32_t)__popcll(m & lanes_below());
+    const uint32_t take = min(t, (uint32_t)__popcll(m));
+    active = rank < take;
+    if (active) {
+        q = stk[t - 1 - rank].x;
+        enc = stk[t - 1 - rank].y;
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (lane_id() == __ffsll((long long)m) - 1) *top = t - take;
+    __builtin_amdgcn_wave_barrier();
+    return take;
+}
+
 // ---------------------------------------------------------------- UPDATE (prune / sprout)
-// One entry per lane and loop iteration (grid-stride, so the wave's entries stay neighbours):
-// pruned and external entries are settled at once, an overlapping internal entry starts a sprout
-// walk (the stackless walk of its subtree, one node test per step, as in k_traverse), and the
-// wave steps its walks until all have ended, lanes without a walk taking over the tails of
-// others' (from an overlapping node's escape on): the wave no longer waits for its longest
-// sprout with the other lanes idle.
+// One entry per lane and loop iteration (grid-stride, so the wave's entries stay neighbours; the next
+// one's words are loaded meanwhile). Pruned entries climb by the parent words beside the node
+// records. An overlapping internal entry sprouts: its children go on the wave's LDS stack, from which
+// every lane tests one node per round (a node that does not overlap and every leaf is an entry of the
+// new front, an overlapping node pushes its children); rounds run while the stack fills the wave, the
+// rest waits for more entries. Bound by the latency of the loads that follow one another, so by their
+// number and the waves in flight. Against a walk per lane, parts of it handed to idle lanes, and
+// climbs by the spine arrays, us: 2.6k triangles 25 -> 18, 41k 78 -> 64, 65k boxes 60 -> 48,
+// 130k 89 -> 70, 2.1M 1710 -> 1340 (1860 with half as many waves).
+constexpr uint32_t kSproutStack = 256, kSproutStage = 192;  // 24 resident waves per CU
+__device__ inline uint32_t sprout_drain(const DevState& d, const Out& out, lds_int2* stk, lds_u32* top, uint32_t least) {
+    uint32_t visits = 0;
+    const int64_t limit = 64 * (2 * d.maxT + 16);
+    for (int64_t rounds = 0;; ++rounds) {
+        const uint32_t t = *top;
+        if (t < least || t == 0) break;
+        if (rounds > limit) {  // only a corrupted tree gets here (flag 16, a device error)
+            if (lane_id() == 0) {
+                atomicOr(&d.ctr[C_OVF], 16u);
+                *top = 0;
+            }
+            break;
+        }
+        bool active;
+        int32_t q = 0, enc = 0;
+        desc_pop(stk, top, active, q, enc);
+        const int32_t nd = enc >> 1;
+        const bool leaf = enc & 1;
+        bool hit = false;
+        Box qb{};
+        float4 hi = make_float4(0.f, 0.f, 0.f, 0.f);
+        int4 tp = make_int4(0, 0, 0, 0);
+        if (active) {
+            const float4 qlo = d.qleaf[q].lo, qhi = d.qleaf[q].hi;
+            const NodeRec* r = leaf ? &d.leaf[nd] : &d.inode[nd];
+            const float4 lo = r->lo;
+            hi = r->hi;
+            if (!leaf) tp = d.itopo[nd];
+            qb = rec_box(qlo, qhi);
+            hit = box_overlap(qb, lo, hi);
+            ++visits;
+        }
+        const bool grow = hit && !leaf;
+        const bool ok_l = desc_push<kSproutStack>(stk, top, grow, q, tp.x),
+                   ok_r = desc_push<kSproutStack>(stk, top, grow, q, tp.y);
+        bool pair = hit && leaf;
+        if (out.skip_adj && pair) pair = !faces_share_vertex(out.lfaces, q, nd);
+        out.pair_push(pair, make_int2(q, nd));
+        stage_push(out.fe, out.ovf, out.sb[1], out.sf[1], out.scap, active && leaf, make_int2(q, nd));
+        stage_push(out.fi, out.ovf, out.sb[0], out.sf[0], out.scap, active && !leaf && !hit, make_int2(q, nd));
+        if (grow && !(ok_l && ok_r)) {  // no room: this lane walks what did not fit (never a left child alone)
+            visits += stackless<true>(d, out, q, qb, ok_l ? tp.y : tp.x, f2i(hi.w));
+        }
+    }
+    return visits;
+}
 __global__ void __launch_bounds__(kBlock) k_update(DevState d, FrontIn in, FrontSink fi, FrontSink fe) {
-    __shared__ Stages st;
+    __shared__ StagesT<kSproutStage> st;
+    __shared__ DescStack<kWaves, kSproutStack> ds;
     stages_init(st);
+    const int w = threadIdx.x >> 6;
+    if (lane_id() == 0) ds.top[w] = 0;
+    lds_int2* stk = (lds_int2*)ds.item[w];
+    lds_u32* top = (lds_u32*)&ds.top[w];
     const Out out = make_out(st, fi, fe, d);
-    const int lane = lane_id();
     const uint32_t ni = min(*in.size[0], in.cap[0]), ne = min(*in.size[1], in.cap[1]), total = ni + ne;
     const uint32_t stride = gridDim.x * blockDim.x;
     uint32_t visits = 0;
-    const int64_t limit = 64 * (2 * d.maxT + 16);
-    // wave-uniform trip count: every lane of a wave takes part in the walk rounds
-    for (uint32_t k0 = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); k0 < total; k0 += stride) {
-        const uint32_t k = k0 + lane;
-        bool walk = false;
-        int32_t qi = 0, cur = -1, stop = -1, spine = -1;
-        Box qb{};
-        if (k < ni) {
-            const int32_t q = in.query[0][k];
-            int32_t node = (int32_t)in.node[0][k];
+    int32_t qn = 0, xn = 0;  // the next iteration's entry, loaded while this one's records are
+    auto load_entry = [&](uint32_t k) {
+        if (k >= total) return;
+        qn = k < ni ? in.query[0][k] : in.query[1][k - ni];
+        xn = (int32_t)(k < ni ? in.node[0][k] : in.node[1][k - ni]);
+    };
+    const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x;
+    load_entry(first);
+    // wave-uniform trip count: every lane of a wave takes part in the sprout rounds
+    for (uint32_t k = first; k - lane_id() < total; k += stride) {
+        const bool valid = k < total, internal = k < ni;
+        const int32_t q = qn, x = xn;
+        Box b{};
+        bool hit = false, climb = false;
+        int32_t node = x;  // climbing: a node that does not overlap, and its topology
+        int4 tp = make_int4(0, 0, 0, 0);
+        if (valid) {
             const float4 qlo = d.qleaf[q].lo, qhi = d.qleaf[q].hi;
-            const Box b = rec_box(qlo, qhi);
-            const float4 lo = d.inode[node].lo, hi = d.inode[node].hi;
+            const NodeRec* r = internal ? &d.inode[x] : &d.leaf[x];
+            const float4 lo = r->lo, hi = r->hi;
+            if (internal) tp = d.itopo[x];
+            b = rec_box(qlo, qhi);
+            hit = box_overlap(b, lo, hi);
+            climb = internal && !hit;
+            if (!internal) node = f2i(lo.w);  // the leaf's parent
             ++visits;
-            if (!box_overlap(b, lo, hi)) {  // prune: climb the left spine while not overlapping
-                const int32_t t = max(d.leaf_lca[f2i(lo.w)] >> 1, 0);
-                for (node--; node >= t; node--) {
-                    ++visits;
-                    if (node_overlap(d, node, b)) break;
-                }
-                bool keep = true;
-                if (node < t && node + 1 > 0) {
-                    ++visits;
-                    keep = node_overlap(d, d.int_par[node + 1], b);  // else a left sibling's entry covers it
-                }
-                if (keep) out.int_entry(q, node + 1);
-            } else {  // sprout: walk the subtree from its left child to its escape
-                qi = q;
-                qb = b;
-                cur = (d.int_lc[node] << 1) | (int32_t)(d.int_mark[node] & 1u);
-                stop = f2i(hi.w);
-                walk = cur != stop;
-            }
-        } else if (k < total) {
-            const int32_t q = in.query[1][k - ni];
-            const int32_t j = (int32_t)in.node[1][k - ni];
-            const float4 qlo = d.qleaf[q].lo, qhi = d.qleaf[q].hi;
-            const Box b = rec_box(qlo, qhi);
-            const float4 llo = d.leaf[j].lo, lhi = d.leaf[j].hi;
-            ++visits;
-            if (box_overlap(b, llo, lhi)) {
-                out.ext_entry(q, j);
-                out.pair(q, j);
-            } else {
-                const int32_t gfa = f2i(llo.w);
-                ++visits;
-                if (node_overlap(d, gfa, b)) {
-                    out.ext_entry(q, j);
-                } else if (!(d.leaf_mark[j] & 4u)) {  // right child: the left sibling's entry climbs
-                    const int32_t top = max(d.leaf_lca[j] >> 1, 0);
-                    int32_t node;
-                    for (node = gfa - 1; node >= top; node--) {
-                        ++visits;
-                        if (node_overlap(d, node, b)) break;
-                    }
-                    bool keep = true;
-                    if (node < top && node + 1 > 0) {
-                        ++visits;
-                        keep = node_overlap(d, d.int_par[node + 1], b);
-                    }
-                    if (keep) out.int_entry(q, node + 1);
-                }
-            }
         }
-        // the sprout walks of this iteration's entries, shared by the wave
-        for (int64_t round = 0; __ballot(walk) != 0ull; ++round) {
-            if (round > limit) {  // only a corrupted tree gets here (flag 16, a device error)
-                if (walk) atomicOr(&d.ctr[C_OVF], 16u);
+        load_entry(k + stride);
+        bool ext = valid && !internal && hit;
+        bool pair = ext;
+        if (out.skip_adj && pair) pair = !faces_share_vertex(out.lfaces, q, x);
+        if (valid && !internal && !hit) {
+            const bool right = (d.leaf_mark[x] & 4u) != 0u;
+            const int4 pt = d.itopo[node];
+            ++visits;
+            ext = node_overlap(d, node, b);
+            climb = !ext && !right;  // a right child's left sibling's entry climbs
+            tp = pt;
+        }
+        // prune: climb while the parent does not overlap either
+        bool keep = false;
+        while (climb) {
+            const int32_t par = tp.z >> 1;
+            if (par < 0) {
+                keep = true;
                 break;
             }
-            bool can_give = false;
-            int32_t give = -1;
-            if (walk) {
-                ++visits;
-                if (!(cur & 1)) {
-                    const int32_t nd = cur >> 1;
-                    const float4 lo = d.inode[nd].lo, hi = d.inode[nd].hi;
-                    if (spine < 0) spine = d.leaf_par[f2i(lo.w)];
-                    if (!box_overlap(qb, lo, hi)) {
-                        out.int_entry(qi, nd);
-                        cur = f2i(hi.w);
-                        spine = -1;
-                    } else {
-                        give = f2i(hi.w);
-                        can_give = give != stop;
-                        cur = nd == spine ? ((f2i(lo.w) << 1) | 1) : cur + 2;
-                        if (nd == spine) spine = -1;
-                    }
-                } else {
-                    const int32_t j = cur >> 1;
-                    const float4 llo = d.leaf[j].lo, lhi = d.leaf[j].hi;
-                    if (box_overlap(qb, llo, lhi)) out.pair(qi, j);
-                    out.ext_entry(qi, j);
-                    cur = f2i(lhi.w);
-                    spine = -1;
-                }
-                walk = cur != stop;
-            }
-            const uint64_t idle_m = __ballot(!walk), donors = __ballot(can_give);
-            const uint32_t pairs = (uint32_t)min(__popcll(idle_m), __popcll(donors));
-            if (pairs >= 8u || (pairs > 0u && __popcll(idle_m) >= 32)) {
-                const uint32_t ri = (uint32_t)__popcll(idle_m & lanes_below());
-                const uint32_t rd = (uint32_t)__popcll(donors & lanes_below());
-                const int src = (!walk && ri < pairs) ? kth_set_lane(donors, ri) : lane;
-                const int32_t g_q = __shfl(qi, src), g_cur = __shfl(give, src), g_stop = __shfl(stop, src);
-                const float g0 = __shfl(qb.mnx, src), g1 = __shfl(qb.mny, src), g2 = __shfl(qb.mnz, src);
-                const float g3 = __shfl(qb.mxx, src), g4 = __shfl(qb.mxy, src), g5 = __shfl(qb.mxz, src);
-                if (can_give && rd < pairs) stop = give;
-                if (!walk && ri < pairs) {
-                    walk = true;
-                    qi = g_q;
-                    cur = g_cur;
-                    stop = g_stop;
-                    spine = -1;
-                    qb = Box{g0, g1, g2, g3, g4, g5};
-                }
-            }
+            const int4 pt = d.itopo[par];
+            ++visits;
+            keep = node_overlap(d, par, b);
+            if (keep || (tp.z & 1)) break;  // from a right child: a left sibling's entry covers the parent
+            node = par;
+            tp = pt;
         }
+        out.pair_push(pair, make_int2(q, x));
+        stage_push(out.fe, out.ovf, out.sb[1], out.sf[1], out.scap, ext, make_int2(q, x));
+        stage_push(out.fi, out.ovf, out.sb[0], out.sf[0], out.scap, keep, make_int2(q, node));
+        // sprout: less than 64 items are left from before, so 128 more fit
+        desc_push<kSproutStack>(stk, top, internal && hit, q, tp.x);
+        desc_push<kSproutStack>(stk, top, internal && hit, q, tp.y);
+        visits += sprout_drain(d, out, stk, top, 64u);
     }
+    visits += sprout_drain(d, out, stk, top, 1u);
     out.final_flush();
     add_visits(d, visits);
 }
@@ -1589,30 +1633,6 @@ void launch_update(DevState& d, int32_t n, int quality, hipStream_t s, bool orde
 // dependent load: the node's record, and for an overlapping internal node its children). The
 // nodes tested and the pairs found are those of the lane's own walk; a stack that is full
 // leaves the lane to walk that subtree itself.
-constexpr uint32_t kDescStack = 512;
-template <int W>
-struct DescStack {
-    int2 item[W][kDescStack];  // (query, node << 1 | leaf)
-    uint32_t top[W];
-};
-
-// Pushes (q, node enc) for the lanes with pred set; returns false for a lane whose item did not
-// fit (it must then test that node itself). Called by all active lanes of the wave.
-__device__ inline bool desc_push(lds_int2* stk, lds_u32* top, bool pred, int32_t q, int32_t enc) {
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return true;
-    const uint32_t t = *top;
-    const uint32_t rank = (uint32_t)__popcll(m & lanes_below());
-    const bool fits = t + rank < kDescStack;
-    if (pred && fits) {
-        stk[t + rank].x = q;
-        stk[t + rank].y = enc;
-    }
-    const uint32_t pushed = (uint32_t)__popcll(__ballot(pred && fits));
-    if (lane_id() == __ffsll((long long)__ballot(1)) - 1) *top = t + pushed;
-    return fits || !pred;
-}
-
 // Tests node `enc` against q's box: an overlapping leaf is a pair, an overlapping internal node
 // pushes its two children (or, without room, is walked by this lane). Returns the node tests.
 __device__ inline uint32_t desc_test(const DevState& d, const Out& out, lds_int2* stk, lds_u32* top,
@@ -1657,8 +1677,6 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
                                       uint32_t least) {
     uint32_t visits = 0;
     const int lane = lane_id();
-    const uint32_t nact = (uint32_t)__popcll(__ballot(1));
-    const uint32_t rank = (uint32_t)__popcll(__ballot(1) & lanes_below());
     // every node is tested at most once per query walk; the bound only guards against a
     // corrupted tree (flag 16, reported as a device error, instead of a hang)
     const int64_t limit = 2 * d.maxT + 16;
@@ -1672,16 +1690,9 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
             }
             break;
         }
-        const uint32_t take = min(t, nact);
-        const bool active = rank < take;
+        bool active;
         int32_t q = 0, enc = 0;
-        if (active) {
-            q = stk[t - 1 - rank].x;
-            enc = stk[t - 1 - rank].y;
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane == __ffsll((long long)__ballot(1)) - 1) *top = t - take;
-        __builtin_amdgcn_wave_barrier();
+        desc_pop(stk, top, active, q, enc);
         visits += desc_test(d, out, stk, top, active, q, enc);
     }
     return visits;

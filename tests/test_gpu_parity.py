@@ -766,3 +766,31 @@ def test_sort_and_scan_tile_edges(pkg, oracle, T):
         for k in ("int_lc", "int_rc", "int_rx", "int_ry", "leaf_par", "leaf_lca"):
             np.testing.assert_array_equal(b[k], topo[k], err_msg=k)
     ctx.close()
+
+
+@pytest.mark.parametrize("kind,T,skip_adjacent", [("soup", 2, False), ("soup", 65, False), ("mesh", 130, True),
+                                                  ("bad", 400, False), ("soup", 900, False)])
+def test_update_sprouts_and_prunes_everything(pkg, oracle, kind, T, skip_adjacent):
+    """UPDATE from a spread scene to one where every box overlaps every other (each front entry sprouts
+    down to its leaves, past the room of the waves' stacks) and back (every entry climbs), twice:
+    fronts and pairs equal the oracle's."""
+    print(f"[gpu] update {kind} {T} skip {skip_adjacent}", flush=True)
+    faces, v = _soup(kind, T, np.random.default_rng(T))
+    spot = (np.random.default_rng(2).random(v.shape) + 0.1).astype(np.float32)
+    ctx = pkg.CollisionContext(T, len(v), int_front_cap=T * T + 64, ext_front_cap=T * T + 64, pair_cap=T * T + 64,
+                               skip_adjacent=skip_adjacent)
+    ctx.set_topology(faces, len(v))
+    orc = oracle.OracleContext(faces, len(v))
+    for fr, (xyz, op) in enumerate([(v, (0, 1)), (spot, (1, 2)), (v, (1, 2)), (v[::-1].copy(), (1, 2)), (spot, (1, 2))]):
+        for c in (ctx, orc):
+            c.update_vertices(xyz)
+            c.step(*op)
+        for w in (0, 1):
+            np.testing.assert_array_equal(_rows(ctx.export_front(w)), _rows(orc.front(w)), err_msg=f"{fr} {w}")
+        for f in (False, True):
+            want = oracle.pair_set(orc.pairs(f))
+            if skip_adjacent:  # the oracle lists them
+                p = (want.astype(np.uint64)[:, None] >> np.array([32, 0], np.uint64) & np.uint64(0xFFFFFFFF)).astype(int)
+                want = want[~(faces[p[:, 0]][:, :, None] == faces[p[:, 1]][:, None, :]).any((1, 2))]
+            np.testing.assert_array_equal(oracle.pair_set(ctx.pairs(f)), want, err_msg=f"{fr} filtered {f}")
+    ctx.close()
