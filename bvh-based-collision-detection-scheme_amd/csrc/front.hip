@@ -788,9 +788,10 @@ __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, uint32_t per, De
 //    covers everything between: the run is cut at its three widest jumps and a node is tested
 //    against the four pieces' boxes (2M-triangle folded cloth: 481 nodes per wave instead of 793,
 //    the worst wave 2281 instead of 59425);
-//  * leaves: each leaf reached (170 per wave there) is tested by every lane against its own query, its
-//    box kept in LDS (STAGED) or loaded once more for the wave through the scalar cache; hits go to
-//    the wave's LDS list.
+//  * leaves: those reached (170 per wave there) are tested against runs of 8 neighbouring queries (RUNS):
+//    a leaf per lane against each run's box first, then the 8 queries of the runs it overlaps, 8 such
+//    items per step, boxes in LDS; or every lane tests every leaf against its own query, the leaf's box
+//    loaded once for the wave through the scalar cache. Hits go to the wave's LDS list.
 // Every node test serves 64 queries and every leaf record is fetched once per wave, where a walk
 // or a front entry per query fetches two 32-byte records per test. A pair is found exactly when the
 // leaves' boxes overlap, as in a query's own walk: a node's box holds its leaves' boxes and a piece's
@@ -798,20 +799,24 @@ __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, uint32_t per, De
 // hold NaN, for which that is not so: they take the walks and fronts.)
 // skip_adj: pairs of triangles that share a vertex are removed when the LDS list is flushed (64 pairs
 // per step; the query's vertex ids come from its lane).
-// Bound by instruction issue (61 % of the VALU and 63 % of the scalar slots busy; half the node
-// rounds run with few nodes). Folded cloths: 180k triangles 185 -> 111 us (against the queries' own
-// walks sharing a wave's lanes), 64 scenes of 2.6M triangles 1.04 -> 0.56 ms (against a walk per
-// lane). KEEP's test of a front stays where there is one: 0.56 ms against 0.60 ms here on the 2M
-// cloth, and 12 us against 43 us on 2,560 triangles, where the tree's depth in rounds is what counts.
+// Bound by the latency of one round after another on small scenes, by instruction issue on large ones
+// (48 % of the VALU and 47 % of the scalar slots busy on 64 scenes of 2.6M triangles). Folded cloths: 180k
+// triangles 185 -> 93 us (against the queries' own walks sharing a wave's lanes), 64 scenes of 2.6M
+// triangles 1.04 -> 0.56 ms (against a walk per lane). KEEP's test of a front stays where there is one:
+// 0.44 ms against 0.66 ms here on the 2M cloth, 13 us against 17 us on 2,560 triangles.
 constexpr uint32_t kGroupStack = 512;  // encoded nodes per wave (2 KB)
 constexpr int kGroupPieces = 4;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef BVHCD_LDS f32x4 lds_f32x4;
-template <bool STAGED>
+typedef volatile BVHCD_LDS uint16_t lds_u16;
+constexpr int kRun = 8;             // neighbouring queries tested together (RUNS)
+template <bool RUNS>
 struct GroupLds {
-    static constexpr uint32_t kStage = STAGED ? 256 : 512;  // staged pairs per wave
-    f32x4 box[kWaves][STAGED ? 128 : 1][2];  // of the leaves reached: (lo, leaf id), (hi, -)
-    uint32_t cand[kWaves][STAGED ? 1 : 128]; // or their ids alone
+    static constexpr uint32_t kStage = RUNS ? 256 : 512;  // staged pairs per wave
+    f32x4 leaf[kWaves][RUNS ? 64 : 1][2];   // RUNS: a round's leaves by lane: (lo, id), (hi, -)
+    f32x4 query[kWaves][RUNS ? 64 : 1][2];  // and the queries: (lo, -), (hi, last leaf)
+    uint16_t item[kWaves][RUNS ? 64 * 64 / kRun : 2];  // run << 6 | lane of the leaf
+    uint32_t cand[kWaves][RUNS ? 1 : 128];  // else the leaves' ids
     uint32_t stack[kWaves][kGroupStack];
     int2 pairs[kWaves][kStage];
     uint32_t fill[kWaves][2];          // [1]: segment rotor (stage_flush)
@@ -819,6 +824,20 @@ struct GroupLds {
 typedef const __attribute__((address_space(4))) float4 const_float4;  // loaded through the scalar cache
 __device__ inline float lane_f(float v, int lane) {
     return i2f(__builtin_amdgcn_readlane(f2i(v), lane));
+}
+// Box of each aligned run of 8 lanes, in all its lanes.
+template <int CTRL>
+__device__ inline float dpp_f(float v) {
+    return i2f(__builtin_amdgcn_mov_dpp(f2i(v), CTRL, 0xF, 0xF, false));
+}
+template <int CTRL>
+__device__ inline Box dpp_merge(const Box& b) {
+    return box_merge(b, Box{dpp_f<CTRL>(b.mnx), dpp_f<CTRL>(b.mny), dpp_f<CTRL>(b.mnz), dpp_f<CTRL>(b.mxx),
+                            dpp_f<CTRL>(b.mxy), dpp_f<CTRL>(b.mxz)});
+}
+__device__ inline Box run_box(const Box& b) {  // lane ^ 1, lane ^ 2, then the other four
+    static_assert(kRun == 8, "two quad permutations and a half-row mirror");
+    return dpp_merge<0x141>(dpp_merge<0x4E>(dpp_merge<0xB1>(b)));
 }
 __device__ inline uint32_t wave_max(uint32_t v) {
     for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
@@ -830,16 +849,17 @@ __device__ inline void wave_lds_order() {  // LDS operations of one wave complet
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool BATCH, bool STAGED>
+template <bool BATCH, bool RUNS>
 __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, DevState d,
                                                      const uint64_t* __restrict__ keys,
                                                      const int32_t* __restrict__ scene_last) {
-    constexpr uint32_t kGroupStage = GroupLds<STAGED>::kStage;
-    constexpr int kAtOnce = STAGED ? 2 : 4;  // leaves loaded together
-    __shared__ GroupLds<STAGED> lds;
+    constexpr uint32_t kGroupStage = GroupLds<RUNS>::kStage;
+    __shared__ GroupLds<RUNS> lds;
     const int w = threadIdx.x >> 6, lane = lane_id();
     lds_u32* const stk = (lds_u32*)lds.stack[w];
-    lds_f32x4* const box = (lds_f32x4*)lds.box[w];
+    lds_f32x4* const lbox = (lds_f32x4*)lds.leaf[w];
+    lds_f32x4* const qbox = (lds_f32x4*)lds.query[w];
+    lds_u16* const item = (lds_u16*)lds.item[w];
     lds_u32* const cand = (lds_u32*)lds.cand[w];
     lds_int2* const sb = (lds_int2*)lds.pairs[w];
     lds_u32* const sf = (lds_u32*)lds.fill[w];
@@ -900,6 +920,12 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                            lane_f(pb.mxx, end), lane_f(pb.mxy, end), lane_f(pb.mxz, end)};
             if (rest) heads = rest;  // fewer pieces: the last one again
         }
+        Box run{};
+        if (RUNS) {
+            run = run_box(qb);
+            qbox[2 * lane] = f32x4{qb.mnx, qb.mny, qb.mnz, 0.f};
+            qbox[2 * lane + 1] = f32x4{qb.mxx, qb.mxy, qb.mxz, i2f(valid ? last : -1)};
+        }
 
         uint32_t fill = 0;
         auto flush = [&]() {
@@ -939,41 +965,74 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
             if (f) stage_flush(sink, ovf, sb, sf, f, ~0ull);
             fill = 0;
         };
-        auto emit = [&](bool hit, int32_t j) {  // room for 64 pairs is the caller's business
+        auto emit = [&](bool hit, int32_t qi, int32_t j) {  // room for 64 pairs is the caller's business
             const uint64_t m = __ballot(hit);
             if (m == 0ull) return;
             if (hit) {
                 const uint32_t slot = fill + (uint32_t)__popcll(m & lanes_below());
-                sb[slot].x = q;
+                sb[slot].x = qi;
                 sb[slot].y = j;
             }
             fill += (uint32_t)__popcll(m);
         };
-        // tests the first k (<= 64) of the leaves reached, kAtOnce loaded together (what lies past the
-        // k-th is some leaf and is not counted)
+        // RUNS: tests the leaves of the lanes with `reached` (box lo, hi, id nd): every run's box against
+        // every leaf, a lane each, then the 8 queries of the runs that it overlaps, 8 such items at once
+        auto test_runs = [&](bool reached, int32_t nd, const float4& lo, const float4& hi) {
+            constexpr int kAtOnce = 2;
+            constexpr uint32_t kItems = 64 / kRun;
+            if (reached) {
+                lbox[2 * lane] = f32x4{lo.x, lo.y, lo.z, i2f(nd)};
+                lbox[2 * lane + 1] = f32x4{hi.x, hi.y, hi.z, 0.f};
+            }
+            uint32_t items = 0;
+            for (uint32_t r = 0; r < size; r += kRun) {
+                const Box b{lane_f(run.mnx, (int)r), lane_f(run.mny, (int)r), lane_f(run.mnz, (int)r),
+                            lane_f(run.mxx, (int)r), lane_f(run.mxy, (int)r), lane_f(run.mxz, (int)r)};
+                const bool near = reached && nd > g0 + (int32_t)r && box_overlap(b, lo, hi);
+                const uint64_t m = __ballot(near);
+                if (near) item[items + (uint32_t)__popcll(m & lanes_below())] = (uint16_t)(r / kRun << 6 | (uint32_t)lane);
+                items += (uint32_t)__popcll(m);
+            }
+            wave_lds_order();
+            for (uint32_t k0 = 0; k0 < items; k0 += kAtOnce * kItems) {
+                if (fill > kGroupStage - 64u * kAtOnce) flush();
+                int32_t qi[kAtOnce], j[kAtOnce];
+                bool h[kAtOnce];
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) {
+                    const uint32_t k = k0 + u * kItems + (uint32_t)(lane / kRun);
+                    const uint32_t it = item[min(k, items - 1u)], lf = it & 63u, qs = (it >> 6) * kRun + (lane % kRun);
+                    const f32x4 a = lbox[2 * lf], b = lbox[2 * lf + 1], c = qbox[2 * qs], e = qbox[2 * qs + 1];
+                    j[u] = f2i(a.w);
+                    qi[u] = g0 + (int32_t)qs;
+                    h[u] = k < items && j[u] > qi[u] && j[u] <= f2i(e.w) &&
+                           box_overlap(Box{c.x, c.y, c.z, e.x, e.y, e.z}, make_float4(a.x, a.y, a.z, 0.f),
+                                       make_float4(b.x, b.y, b.z, 0.f));
+                }
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) emit(h[u], qi[u], j[u]);
+            }
+            wave_lds_order();
+        };
+        // else: tests the first k (<= 64) of the leaves reached, kAtOnce loaded together (what lies past
+        // the k-th is some leaf and is not counted)
         auto test_leaves = [&](uint32_t k) {
-            const int32_t cv = STAGED ? 0 : (int32_t)cand[min((uint32_t)lane, k - 1u)];
+            constexpr int kAtOnce = 4;
+            const int32_t cv = (int32_t)cand[min((uint32_t)lane, k - 1u)];
             for (uint32_t c = 0; c < k; c += kAtOnce) {
                 if (fill > kGroupStage - 64u * kAtOnce) flush();
                 float4 lo[kAtOnce], hi[kAtOnce];
                 int32_t j[kAtOnce];
 #pragma unroll
                 for (int u = 0; u < kAtOnce; ++u) {
-                    if (STAGED) {  // broadcast reads
-                        const f32x4 a = box[2 * (c + u)], b = box[2 * (c + u) + 1];
-                        lo[u] = make_float4(a.x, a.y, a.z, 0.f);
-                        hi[u] = make_float4(b.x, b.y, b.z, 0.f);
-                        j[u] = f2i(a.w);
-                    } else {
-                        j[u] = __builtin_amdgcn_readlane(cv, (int)(c + u));
-                        const_float4* r = (const_float4*)(uintptr_t)&d.leaf[j[u]];
-                        lo[u] = make_float4(r[0].x, r[0].y, r[0].z, 0.f);
-                        hi[u] = make_float4(r[1].x, r[1].y, r[1].z, 0.f);
-                    }
+                    j[u] = __builtin_amdgcn_readlane(cv, (int)(c + u));
+                    const_float4* r = (const_float4*)(uintptr_t)&d.leaf[j[u]];
+                    lo[u] = make_float4(r[0].x, r[0].y, r[0].z, 0.f);
+                    hi[u] = make_float4(r[1].x, r[1].y, r[1].z, 0.f);
                 }
 #pragma unroll
                 for (int u = 0; u < kAtOnce; ++u)
-                    emit(c + u < k && j[u] > after && (!BATCH || j[u] <= last) && box_overlap(qb, lo[u], hi[u]), j[u]);
+                    emit(c + u < k && j[u] > after && (!BATCH || j[u] <= last) && box_overlap(qb, lo[u], hi[u]), q, j[u]);
             }
         };
         uint32_t top = d.top_cut[64], ncand = 0;  // wave-uniform
@@ -1044,35 +1103,23 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                                 cur = d.itopo[x].x;
                             }
                         }
-                        emit(h, j);
+                        emit(h, q, j);
                     }
                 }
             }
+            if (RUNS) {
+                if (ml) test_runs(hit && leaf, nd, lo, hi);
+                continue;
+            }
             if (ml) {
-                if (hit && leaf) {
-                    const uint32_t slot = ncand + (uint32_t)__popcll(ml & lanes_below());
-                    if (STAGED) {
-                        box[2 * slot] = f32x4{lo.x, lo.y, lo.z, i2f(nd)};
-                        box[2 * slot + 1] = f32x4{hi.x, hi.y, hi.z, 0.f};
-                    } else {
-                        cand[slot] = (uint32_t)nd;
-                    }
-                }
+                if (hit && leaf) cand[ncand + (uint32_t)__popcll(ml & lanes_below())] = (uint32_t)nd;
                 ncand += (uint32_t)__popcll(ml);
                 wave_lds_order();
             }
             if (ncand >= 64u || (top == 0u && ncand > 0u)) {
                 test_leaves(min(ncand, 64u));
                 const uint32_t rest = ncand > 64u ? ncand - 64u : 0u;
-                if ((uint32_t)lane < rest) {
-                    if (STAGED) {
-                        const f32x4 a = box[2 * (64 + lane)], b = box[2 * (64 + lane) + 1];
-                        box[2 * lane] = a;
-                        box[2 * lane + 1] = b;
-                    } else {
-                        cand[lane] = cand[64 + lane];
-                    }
-                }
+                if ((uint32_t)lane < rest) cand[lane] = cand[64 + lane];
                 wave_lds_order();
                 ncand = rest;
                 if (top == 0u && ncand > 0u) {  // the last round's overhang
@@ -1087,10 +1134,11 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
 }
 
 // Queries per wave. Small scenes are bound by their heaviest wave, large ones by the node tests, which
-// 64 queries share: pure traversal, us, with 64 / 32 / 16 / 8: 2.6k 41 / 34 / 28 / 25, 41k 50 / 41 / 38 / 52,
-// 65k 114 / 95 / 78 / 80, 180k 134 / 111 / 125 / 178, 522k 345 / 350 / 457 / 641, 2.1M 693 / 877 / 1310.
+// 64 queries share: pure traversal, us, with 64 / 32 / 16 / 8: 2.6k 35 / 26 / 21 / 17, 28k 110 / 62 / 40 /
+// 34, 41k 49 / 36 / 30 / 42, 65k 124 / 73 / 47 / 59, 180k 128 / 93 / 100 / 148, 522k 328 / 286 / 320 / 475,
+// 718k 363 / 368 / 419 / 642, 2.1M 716 / 866 / 1223 / 1968.
 static uint32_t group_size(int32_t n) {
-    return n <= 4096 ? 8u : n <= 3 << 15 ? 16u : n <= 1 << 18 ? 32u : 64u;
+    return n <= 1 << 15 ? 8u : n <= 3 << 15 ? 16u : n <= 5 << 17 ? 32u : 64u;
 }
 // Workgroups of k_group_cd, one group per wave: the same number for each XCD's share.
 static unsigned group_grid(int32_t n) {
@@ -1098,14 +1146,14 @@ static unsigned group_grid(int32_t n) {
     return kXcds * ((share + kWaves - 1) / kWaves);
 }
 
-// The leaves' boxes staged in LDS up to kGroupStaged leaves: there few waves run and each waits for its
-// loads; on larger scenes the LDS would cost resident waves (staged / reloaded, us: 180k 131 / 146, 522k
-// 337 / 348, 1.2M 506 / 467, 8.4M 1997 / 1846).
-constexpr int32_t kGroupStaged = 1 << 19;
+// Leaf tests by runs of 8 queries (RUNS) up to this many leaves: an eighth of the box tests, but twice
+// the LDS and a third fewer resident waves, which larger scenes need (us, runs / every lane its query: 7k
+// 48 / 69, 65k 47 / 66, 130k 70 / 88, 318k 136 / 165, 718k 363 / 370, 1.2M 611 / 574, 2.1M 775 / 716).
+constexpr int32_t kGroupRuns = 3 << 18;
 template <bool BATCH>
 static void launch_group_cd(DevState& d, int32_t n, unsigned grid, const uint64_t* keys, const int32_t* scene_last,
                             hipStream_t s) {
-    if (n <= kGroupStaged)
+    if (n <= kGroupRuns)
         hipLaunchKernelGGL((k_group_cd<BATCH, true>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
     else
         hipLaunchKernelGGL((k_group_cd<BATCH, false>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
