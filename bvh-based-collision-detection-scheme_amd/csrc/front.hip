@@ -666,117 +666,136 @@ std::string tuning_report() {
     return r;
 }
 
-// ---------------------------------------------------------------- pure traversal / generate
-// Lane of the wave holding the k-th (0-based) set bit of m (k < popcount(m)).
-__device__ inline int kth_set_lane(uint64_t m, uint32_t k) {
-    int lo = 0, hi = 63;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if ((uint32_t)__popcll(m & ((2ull << mid) - 1ull)) > k) hi = mid;
-        else lo = mid + 1;
+// ---------------------------------------------------------------- per-wave stacks of node tests
+constexpr uint32_t kDescStack = 512;
+template <int W, uint32_t CAP = kDescStack>
+struct DescStack {
+    int2 item[W][CAP];  // (query, node << 1 | leaf)
+    uint32_t top[W];
+};
+
+// Pushes (q, node enc) for the lanes with pred set; returns false for a lane whose item did not
+// fit (it must then test that node itself). Called by all active lanes of the wave.
+template <uint32_t CAP = kDescStack>
+__device__ inline bool desc_push(lds_int2* stk, lds_u32* top, bool pred, int32_t q, int32_t enc) {
+    const uint64_t m = __ballot(pred);
+    if (m == 0) return true;
+    const uint32_t t = *top;
+    const uint32_t rank = (uint32_t)__popcll(m & lanes_below());
+    const bool fits = t + rank < CAP;
+    if (pred && fits) {
+        stk[t + rank].x = q;
+        stk[t + rank].y = enc;
     }
-    return lo;
+    const uint32_t pushed = (uint32_t)__popcll(__ballot(pred && fits));
+    if (lane_id() == __ffsll((long long)__ballot(1)) - 1) *top = t + pushed;
+    return fits || !pred;
 }
 
-// The stackless walk of stackless<FRONT>, one node test per lane and step, with the wave's
-// lanes sharing the work: a query's walk from `cur` to `stop` is, at an overlapping internal
-// node nd, nd's subtree followed by the walk from nd's escape to `stop`. So a lane at such a node
-// can hand the second part to an idle lane (its own walk then stops at nd's escape) — the walks
-// of a wave's `per` queries end at very different times (the longest is ~1.8x the mean on the folded 2M
-// cloth), and without this the wave waits for its longest one. The nodes tested, the entries
-// and the pairs are those of the queries' own walks; only their order changes.
+__device__ inline float lane_perm(int at, float v) { return i2f(__builtin_amdgcn_ds_bpermute(at, f2i(v))); }
+// Takes up to one item per active lane off the wave's stack; returns the number taken.
+__device__ inline uint32_t desc_pop(lds_int2* stk, lds_u32* top, bool& active, int32_t& q, int32_t& enc) {
+    const uint64_t m = __ballot(1);
+    const uint32_t t = *top, rank = (uint32_t)__popcll(m & lanes_below());
+    const uint32_t take = min(t, (uint32_t)__popcll(m));
+    active = rank < take;
+    if (active) {
+        q = stk[t - 1 - rank].x;
+        enc = stk[t - 1 - rank].y;
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (lane_id() == __ffsll((long long)m) - 1) *top = t - take;
+    __builtin_amdgcn_wave_barrier();
+    return take;
+}
+
+// ---------------------------------------------------------------- pure traversal / generate
+// Self-CD query leaf i walks the leaves after it, from lca[i + 1] (its record's escape) on: that node's
+// subtree, then the subtree at its escape, and so on to the end; inter-object: every query walks the
+// whole tree from its root lca[0]. A wave takes `per` queries; the nodes still to be tested lie on its
+// LDS stack as (query's lane | kChain for a walk's own nodes, encoded node), and every lane tests one
+// per round: a node that does not overlap and every leaf is an entry of the query's front, an
+// overlapping node pushes its children, a chain node the next one. The nodes tested, the entries and the
+// pairs are those of the queries' own walks. Bound by the latency of the rounds on small scenes, by the
+// vector L1 (three divergent 16-byte loads per test) and the staged output on large ones. Against a walk
+// per lane, parts of it handed to idle lanes, us: 2.6k triangles 48 -> 36, 41k 62 -> 45, 65k boxes 134 ->
+// 101, 130k 152 -> 115, 8.4M 3850 -> 3350.
+constexpr uint32_t kWalkStack = 256, kWalkStage = 192;  // 24 resident waves per CU
+constexpr int32_t kChain = 64;
 template <bool FRONT>
 __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, uint32_t per, DevState d, FrontSink fi, FrontSink fe) {
-    __shared__ Stages st;
+    __shared__ StagesT<kWalkStage> st;
+    __shared__ DescStack<kWaves, kWalkStack> ds;
     stages_init(st);
+    const int w = threadIdx.x >> 6, lane = lane_id();
+    if (lane == 0) ds.top[w] = 0;
+    lds_int2* stk = (lds_int2*)ds.item[w];
+    lds_u32* top = (lds_u32*)&ds.top[w];
     const Out out = make_out(st, fi, fe, d);
-    const int lane = lane_id();
     const int32_t nq = d.inter ? d.nq : n - 1;
-    const int32_t i = (int32_t)((blockIdx.x * kWaves + (threadIdx.x >> 6)) * per) + lane;
-    // self-CD: query leaf i walks the leaves after it (from lca[i + 1], its record's escape);
-    // inter-object: every query walks the whole tree from its root lca[0]
-    bool act = lane < (int)per && i < nq;
-    int32_t qi = i, cur = -1, stop = -1, spine = -1;  // spine: bottom of the spine being descended
-    Box qb{};
-    if (act) {
+    const int32_t q0 = (int32_t)((blockIdx.x * kWaves + w) * per), i = q0 + lane;
+    const bool query = lane < (int)per && i < nq;
+    Box own{};
+    int32_t start = -1;
+    if (query) {
         const float4 lo = d.qleaf[i].lo, hi = d.qleaf[i].hi;
-        qb = rec_box(lo, hi);
-        cur = d.inter ? d.leaf_lca[0] : f2i(hi.w);
-        act = cur != stop;
+        own = rec_box(lo, hi);
+        start = d.inter ? d.leaf_lca[0] : f2i(hi.w);
     }
-    uint32_t v = 0;
-    // every node is tested at most once per query walk; the bound only guards against a
-    // corrupted tree (flag 16, reported as a device error, instead of a hang)
+    uint32_t visits = 0;
+    desc_push<kWalkStack>(stk, top, query && start != -1, lane | kChain, start);
     const int64_t limit = 64 * (2 * d.maxT + 16);
-    for (int64_t round = 0; __ballot(act) != 0ull; ++round) {
-        if (round > limit) {
-            if (act) atomicOr(&d.ctr[C_OVF], 16u);
+    for (int64_t rounds = 0;; ++rounds) {
+        const uint32_t t = *top;
+        if (t == 0) break;
+        if (rounds > limit) {  // only a corrupted tree gets here (flag 16, a device error)
+            if (lane == 0) atomicOr(&d.ctr[C_OVF], 16u);
             break;
         }
-        bool emit_int = false, emit_ext = false, emit_pair = false, can_give = false;
-        int32_t node = 0, give = -1;
-        if (act) {
-            ++v;
-            if (!(cur & 1)) {
-                const int32_t nd = cur >> 1;
-                const float4 lo = d.inode[nd].lo, hi = d.inode[nd].hi;
-                if (spine < 0) spine = d.leaf_par[f2i(lo.w)];  // a new subtree: its left spine's bottom
-                node = nd;
-                if (!box_overlap(qb, lo, hi)) {
-                    emit_int = FRONT;
-                    cur = f2i(hi.w);
-                    spine = -1;
-                } else {
-                    give = f2i(hi.w);  // what follows nd's subtree
-                    can_give = give != stop;
-                    cur = nd == spine ? ((f2i(lo.w) << 1) | 1) : cur + 2;  // leftmost leaf, or nd + 1
-                    if (nd == spine) spine = -1;
-                }
-            } else {
-                const int32_t j = cur >> 1;
-                const float4 llo = d.leaf[j].lo, lhi = d.leaf[j].hi;
-                node = j;
-                emit_pair = box_overlap(qb, llo, lhi);
-                emit_ext = FRONT;
-                cur = f2i(lhi.w);
-                spine = -1;
-            }
-            act = cur != stop;
+        // an item pushes three at most: fewer are taken when the stack is nearly full
+        const uint32_t take = max(1u, min(min(t, 64u), (kWalkStack - t) / 2u));
+        const bool active = (uint32_t)lane < take;
+        int32_t x = 0, enc = 0;
+        if (active) {
+            x = stk[t - 1 - lane].x;
+            enc = stk[t - 1 - lane].y;
         }
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) *top = t - take;
+        __builtin_amdgcn_wave_barrier();
+        const int32_t nd = enc >> 1, q = q0 + (x & 63);
+        const bool leaf = enc & 1;
+        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+        int4 tp = make_int4(0, 0, 0, 0);
+        if (active) {
+            const NodeRec* r = leaf ? &d.leaf[nd] : &d.inode[nd];
+            lo = r->lo;
+            hi = r->hi;
+            if (!leaf) tp = d.itopo[nd];
+        }
+        const int from = (x & 63) << 2;
+        const Box qb{lane_perm(from, own.mnx), lane_perm(from, own.mny), lane_perm(from, own.mnz),
+                     lane_perm(from, own.mxx), lane_perm(from, own.mxy), lane_perm(from, own.mxz)};
+        const bool hit = active && box_overlap(qb, lo, hi);
+        visits += active ? 1u : 0u;
+        const bool next = active && (x & kChain) && f2i(hi.w) != -1, grow = hit && !leaf;
+        const bool ok_n = desc_push<kWalkStack>(stk, top, next, x, f2i(hi.w));
+        const bool ok_l = desc_push<kWalkStack>(stk, top, grow, x & 63, tp.x),
+                   ok_r = desc_push<kWalkStack>(stk, top, grow, x & 63, tp.y);
+        bool pair = hit && leaf;
+        if (out.skip_adj && pair) pair = !faces_share_vertex(out.lfaces, q, nd);
+        out.pair_push(pair, make_int2(q, nd));
         if (FRONT) {
-            stage_push(out.fi, out.ovf, out.sb[0], out.sf[0], out.scap, emit_int, make_int2(qi, node));
-            stage_push(out.fe, out.ovf, out.sb[1], out.sf[1], out.scap, emit_ext, make_int2(qi, node));
+            stage_push(out.fe, out.ovf, out.sb[1], out.sf[1], out.scap, active && leaf, make_int2(q, nd));
+            stage_push(out.fi, out.ovf, out.sb[0], out.sf[0], out.scap, active && !leaf && !hit, make_int2(q, nd));
         }
-        bool pair = emit_pair;
-        if (out.skip_adj && pair) pair = !faces_share_vertex(out.lfaces, qi, node);
-        out.pair_push(pair, make_int2(qi, node));
-        // idle lanes take the rest of other lanes' walks
-        const uint64_t idle = __ballot(!act), donors = __ballot(can_give);
-        const uint32_t pairs = (uint32_t)min(__popcll(idle), __popcll(donors));
-        if (pairs >= 8u || (pairs > 0u && __popcll(idle) >= 32)) {
-            const uint32_t ri = (uint32_t)__popcll(idle & lanes_below());
-            const uint32_t rd = (uint32_t)__popcll(donors & lanes_below());
-            const int src = (!act && ri < pairs) ? kth_set_lane(donors, ri) : lane;
-            const int32_t g_q = __shfl(qi, src), g_cur = __shfl(give, src), g_stop = __shfl(stop, src);
-            const float g0 = __shfl(qb.mnx, src), g1 = __shfl(qb.mny, src), g2 = __shfl(qb.mnz, src);
-            const float g3 = __shfl(qb.mxx, src), g4 = __shfl(qb.mxy, src), g5 = __shfl(qb.mxz, src);
-            if (can_give && rd < pairs) stop = give;  // the donor ends at nd's escape
-            if (!act && ri < pairs) {
-                act = true;
-                qi = g_q;
-                cur = g_cur;
-                stop = g_stop;
-                spine = -1;
-                qb = Box{g0, g1, g2, g3, g4, g5};
-            }
-        }
+        // no room (a full stack's last item only): this lane walks what did not fit
+        if (grow && !(ok_l && ok_r)) visits += stackless<FRONT>(d, out, q, qb, ok_l ? tp.y : tp.x, f2i(hi.w));
+        if (!ok_n) visits += stackless<FRONT>(d, out, q, qb, f2i(hi.w), -1);
     }
-    if (FRONT) {
-        out.final_flush();
-    } else {
-        out.pair_final();
-    }
-    add_visits(d, v);
+    if (FRONT) out.final_flush();
+    else out.pair_final();
+    add_visits(d, visits);
 }
 
 // ---------------------------------------------------------------- pairs of 64 queries at a time
@@ -1161,15 +1180,15 @@ static void launch_group_cd(DevState& d, int32_t n, unsigned grid, const uint64_
 
 // Queries of a traversal: the leaves before the last one (self-CD) or the other object's leaves.
 static int64_t query_count(const DevState& d, int32_t n) { return d.inter ? d.nq : n - 1; }
-// Queries a wave of k_traverse starts with; its other lanes take parts of their walks over. With few
-// waves the longest wave is the kernel's time, with enough of them full waves do the least: GENERATE in
-// query order, us, with 64 / 32 / 16: 2.6k 128 / 103 / 87, 41k 154 / 135 / 123, 65k 349 / 250 / 197,
-// 180k 342 / 275 / 297, 522k 1276 / 960 / 898, 1.2M 1600 / 1493 / 1677, 2.1M 2189 / 2253 / 2742.
-uint32_t walk_queries(int64_t nq) { return nq <= 3 << 18 ? 16u : nq <= 3 << 19 ? 32u : 64u; }
+// Queries a wave of k_traverse takes. With few waves the longest wave is the kernel's time, with enough of
+// them full waves do the least: GENERATE in node order, us, with 64 / 32 / 16 / 8: 2.6k 133 / 113 / 94 / 89,
+// 28k 359 / 267 / 214 / 187, 41k 196 / 167 / 148 / 150, 180k 547 / 463 / 438 / 464, 522k 2170 / 1712 / 1518 /
+// 1456, 1.2M 3615 / 2943 / 2692 / 2874, 2.1M 4158 / 3730 / 3737 / 4240, 8.4M 10622 / 10953 / 11817 / 14525.
+uint32_t walk_queries(int64_t nq) { return nq <= 1 << 15 ? 8u : nq <= 3 << 19 ? 16u : nq <= 1 << 22 ? 32u : 64u; }
 static unsigned walk_grid(int64_t nq) { return grid_for(nq, (int)(kWaves * walk_queries(nq))); }
 int64_t max_walk_waves(int64_t T) {
     int64_t w = 1;
-    for (const int64_t nq : {T, std::min<int64_t>(T, 3 << 19), std::min<int64_t>(T, 3 << 18)})
+    for (const int64_t nq : {T, std::min<int64_t>(T, 1 << 22), std::min<int64_t>(T, 3 << 19), std::min<int64_t>(T, 1 << 15)})
         w = std::max<int64_t>(w, (int64_t)walk_grid(nq) * kWaves);
     return w;
 }
@@ -1446,48 +1465,6 @@ void launch_generate(DevState& d, int32_t n, hipStream_t s, bool order) {
         if (!order) launch_query_order(d, n, s);
     }
     d.front_by_query = order ? 0 : 1;
-}
-
-// ---------------------------------------------------------------- per-wave stacks of node tests
-constexpr uint32_t kDescStack = 512;
-template <int W, uint32_t CAP = kDescStack>
-struct DescStack {
-    int2 item[W][CAP];  // (query, node << 1 | leaf)
-    uint32_t top[W];
-};
-
-// Pushes (q, node enc) for the lanes with pred set; returns false for a lane whose item did not
-// fit (it must then test that node itself). Called by all active lanes of the wave.
-template <uint32_t CAP = kDescStack>
-__device__ inline bool desc_push(lds_int2* stk, lds_u32* top, bool pred, int32_t q, int32_t enc) {
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return true;
-    const uint32_t t = *top;
-    const uint32_t rank = (uint32_t)__popcll(m & lanes_below());
-    const bool fits = t + rank < CAP;
-    if (pred && fits) {
-        stk[t + rank].x = q;
-        stk[t + rank].y = enc;
-    }
-    const uint32_t pushed = (uint32_t)__popcll(__ballot(pred && fits));
-    if (lane_id() == __ffsll((long long)__ballot(1)) - 1) *top = t + pushed;
-    return fits || !pred;
-}
-
-// Takes up to one item per active lane off the wave's stack; returns the number taken.
-__device__ inline uint32_t desc_pop(lds_int2* stk, lds_u32* top, bool& active, int32_t& q, int32_t& enc) {
-    const uint64_t m = __ballot(1);
-    const uint32_t t = *top, rank = (uint32_t)__popcll(m & lanes_below());
-    const uint32_t take = min(t, (uint32_t)__popcll(m));
-    active = rank < take;
-    if (active) {
-        q = stk[t - 1 - rank].x;
-        enc = stk[t - 1 - rank].y;
-    }
-    __builtin_amdgcn_wave_barrier();
-    if (lane_id() == __ffsll((long long)m) - 1) *top = t - take;
-    __builtin_amdgcn_wave_barrier();
-    return take;
 }
 
 // ---------------------------------------------------------------- UPDATE (prune / sprout)

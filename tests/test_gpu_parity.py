@@ -794,3 +794,38 @@ def test_update_sprouts_and_prunes_everything(pkg, oracle, kind, T, skip_adjacen
                 want = want[~(faces[p[:, 0]][:, :, None] == faces[p[:, 1]][:, None, :]).any((1, 2))]
             np.testing.assert_array_equal(oracle.pair_set(ctx.pairs(f)), want, err_msg=f"{fr} filtered {f}")
     ctx.close()
+
+
+@pytest.mark.parametrize("kind,T", [("soup", 2), ("mesh", 9), ("soup", 64), ("bad", 300), ("stack", 700), ("mesh", 32767),
+                                    ("mesh", 32770)])
+def test_generate_front_is_the_walks(pkg, oracle, kind, T):
+    """GENERATE off the waves' stacks: sizes around a wave's queries (8, 16 from 32769 triangles on) and a
+    scene whose boxes all overlap (the stacks at their limit): fronts and pairs equal the oracle's walks."""
+    print(f"[gpu] generate {kind} {T}", flush=True)
+    faces, v = _soup(kind, T, np.random.default_rng(T))
+    cap = T * T + 64 if T < 1000 else 128 * T
+    ctx = pkg.CollisionContext(T, len(v), int_front_cap=cap, ext_front_cap=cap, pair_cap=cap)
+    ctx.set_topology(faces, len(v))
+    orc = oracle.OracleContext(faces, len(v))
+    for c in (ctx, orc):
+        c.update_vertices(v)
+        c.step(0, 1)
+    for w in (0, 1):
+        np.testing.assert_array_equal(_rows(ctx.export_front(w)), _rows(orc.front(w)), err_msg=str(w))
+    np.testing.assert_array_equal(oracle.pair_set(ctx.pairs(False)), oracle.pair_set(orc.pairs(False)))
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [222, 223, 574, 629])
+def test_pure_traversal_equals_generate_at_its_switches(pkg, n):
+    """Cloths either side of the pair traversal's changes of queries per wave and of leaf test (98,304,
+    655,360 and 786,432 triangles): as many pairs, with the same digest, as GENERATE finds."""
+    sc = pkg.Scene.preset("cloth1024", n=n)
+    print(f"[gpu] pure traversal against GENERATE at {sc.num_tris}", flush=True)
+    ctx = _ctx(pkg, sc, narrow_phase=False)
+    ctx.update_vertices(sc.frame(sc.frames - 1))
+    ctx.step(pkg.BVH_BUILD, pkg.FRONT_PURE_BVH_CD)
+    got = ctx.digest(False)
+    ctx.step(pkg.BVH_NONE, pkg.FRONT_GENERATE)
+    assert got == ctx.digest(False) and got[1] > sc.num_tris
+    ctx.close()
