@@ -209,10 +209,12 @@ __device__ inline void wave_add(uint32_t* counter, int32_t key, bool pred, uint3
 // tbl[scene * blocks + b]. The exclusive scan of that table is every workgroup's first slot of every
 // scene, from which the scatter counts on in LDS. Global counters per scene instead, with one
 // atomic per distinct scene and wave, took 2.8 ms per pass on 64 scenes (15.5 M hits): all waves
-// add to a few neighbouring words. Bound by the list's traffic and the scene lookups.
+// add to a few neighbouring words. Bound by the loads in flight: count and scatter 94 + 140 us with 1024
+// workgroups, a segment search and a scene lookup per hit; 70 + 119 with the cursor and four rounds of
+// loads (wave_hits), 53 + 89 with 2048 workgroups (4096: the same).
 constexpr int kGroupScenes = 4096;      // most scenes a workgroup counts in LDS (16 KB)
 constexpr int64_t kGroupTable = 1 << 20;  // entries of the count table at most
-unsigned group_blocks(int32_t S) { return (unsigned)std::min<int64_t>(1024, kGroupTable / S); }
+unsigned group_blocks(int32_t S) { return (unsigned)std::min<int64_t>(2048, kGroupTable / S); }
 
 struct HitRange {
     uint32_t begin, end;  // whole waves of hits: begin is a multiple of 64
@@ -223,17 +225,70 @@ __device__ inline HitRange hit_range(uint32_t total) {
     return {b, (uint32_t)min((uint64_t)b + per, (uint64_t)total)};
 }
 
+// The hits of kHitRounds rounds of a wave, round u's first one at k0 + u * kBlock: a lane's pair and its
+// scene. The rounds' loads go out together; the segment is followed from round to round, and the scene
+// as long as all pairs of a round are of it (then looked up for the round's first pair, and by every
+// lane only where a round holds several).
+constexpr int kHitRounds = 4;
+struct HitCursor {
+    int seg = 0;                      // wave-uniform, as is all of this
+    int32_t scene = 0, lo = 0, hi = 0;  // the last scene and its triangles
+};
+struct WaveHits {
+    int2 p[kHitRounds];
+    int32_t s[kHitRounds];
+    bool ok[kHitRounds], one[kHitRounds];  // one: the whole round is of scene s
+};
+__device__ inline WaveHits wave_hits(const DevState& d, const uint32_t* pre, uint32_t k0, uint32_t end, HitCursor& c,
+                                     const int32_t* __restrict__ tri_scene, const int64_t* __restrict__ toff) {
+    WaveHits h;
+#pragma unroll
+    for (int u = 0; u < kHitRounds; ++u) {
+        const uint32_t b = k0 + u * kBlock, k = b + lane_id();
+        h.ok[u] = k < end;
+        h.p[u] = make_int2(0, 0);
+        if (b >= end) continue;
+        while ((uint32_t)__builtin_amdgcn_readfirstlane((int)pre[c.seg + 1]) <= b) ++c.seg;
+        int g = c.seg;
+        if (h.ok[u]) {
+            while (pre[g + 1] <= k) ++g;
+            h.p[u] = d.np[(int64_t)g * d.pair_seg_cap + (int64_t)(k - pre[g])];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kHitRounds; ++u) {
+        h.s[u] = 0;
+        h.one[u] = true;
+        if (k0 + u * kBlock >= end) continue;
+        auto others = [&]() { return __ballot(h.ok[u] && (h.p[u].x < c.lo || h.p[u].x >= c.hi)) != 0ull; };
+        if (others()) {
+            c.scene = tri_scene[__builtin_amdgcn_readfirstlane(h.p[u].x)];
+            c.lo = (int32_t)toff[c.scene];
+            c.hi = (int32_t)toff[c.scene + 1];
+            h.one[u] = !others();
+        }
+        h.s[u] = c.scene;
+        if (!h.one[u] && h.ok[u]) h.s[u] = tri_scene[h.p[u].x];
+    }
+    return h;
+}
+
 __global__ void __launch_bounds__(kBlock) k_group_count(DevState d, int32_t S, const int32_t* __restrict__ tri_scene,
-                                                        uint32_t* __restrict__ tbl) {
+                                                        const int64_t* __restrict__ toff, uint32_t* __restrict__ tbl) {
     __shared__ uint32_t pre[kPairSegs + 1];
     __shared__ uint32_t cnt[kGroupScenes];
     for (int32_t i = threadIdx.x; i < S; i += kBlock) cnt[i] = 0u;
     const uint32_t m = seg_prefix(d.pcnt + kPairSegs * kCntStride, (uint32_t)d.pair_seg_cap, pre);  // holds a barrier
     const HitRange r = hit_range(m);
-    for (uint32_t k0 = r.begin + (threadIdx.x & ~63u); k0 < r.end; k0 += kBlock) {  // wave-uniform
-        const uint32_t k = k0 + lane_id();
-        const bool ok = k < r.end;
-        wave_add(cnt, ok ? tri_scene[d.np[seg_slot(pre, k, d.pair_seg_cap)].x] : 0, ok, nullptr);
+    const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
+    HitCursor c;
+    for (uint32_t k0 = r.begin + w0; k0 < r.end; k0 += kHitRounds * kBlock) {  // wave-uniform
+        const WaveHits h = wave_hits(d, pre, k0, r.end, c, tri_scene, toff);
+#pragma unroll
+        for (int u = 0; u < kHitRounds; ++u) {
+            if (!h.one[u]) wave_add(cnt, h.s[u], h.ok[u], nullptr);
+            else if (h.ok[u] && lane_id() == 0) atomicAdd(&cnt[h.s[u]], min(64u, r.end - (k0 + u * kBlock)));
+        }
     }
     __syncthreads();
     for (int32_t i = threadIdx.x; i < S; i += kBlock) tbl[(int64_t)i * gridDim.x + blockIdx.x] = cnt[i];
@@ -256,16 +311,23 @@ __global__ void __launch_bounds__(kBlock) k_group_scatter(DevState d, int32_t S,
         }
     }
     const HitRange r = hit_range(m);
-    for (uint32_t k0 = r.begin + (threadIdx.x & ~63u); k0 < r.end; k0 += kBlock) {  // wave-uniform
-        const uint32_t k = k0 + lane_id();
-        const bool ok = k < r.end;
-        const int2 p = ok ? d.np[seg_slot(pre, k, d.pair_seg_cap)] : make_int2(0, 0);
-        const int32_t s = ok ? tri_scene[p.x] : 0;
-        uint32_t slot = 0;
-        wave_add(next, s, ok, &slot);
-        if (ok) {
-            const int32_t o = (int32_t)toff[s];
-            out[slot] = make_int2(p.x - o, p.y - o);
+    const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
+    HitCursor c;
+    for (uint32_t k0 = r.begin + w0; k0 < r.end; k0 += kHitRounds * kBlock) {  // wave-uniform
+        const WaveHits h = wave_hits(d, pre, k0, r.end, c, tri_scene, toff);
+#pragma unroll
+        for (int u = 0; u < kHitRounds; ++u) {
+            uint32_t slot = 0;
+            if (!h.one[u]) {
+                wave_add(next, h.s[u], h.ok[u], &slot);
+            } else if (__ballot(h.ok[u]) != 0ull) {
+                if (lane_id() == 0) slot = atomicAdd(&next[h.s[u]], min(64u, r.end - (k0 + u * kBlock)));
+                slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot) + lane_id();
+            }
+            if (h.ok[u]) {
+                const int32_t o = (int32_t)toff[h.s[u]];
+                out[slot] = make_int2(h.p[u].x - o, h.p[u].y - o);
+            }
         }
     }
 }
@@ -333,7 +395,8 @@ void record_frame(bvhcd_batch* b, int bvh_op, unsigned grid) {
     launch_pair_totals(d, s, true);
     if (b->S <= kGroupScenes) {
         const unsigned g = group_blocks(b->S);
-        hipLaunchKernelGGL(k_group_count, dim3(g), dim3(kBlock), 0, s, d, b->S, b->tri_scene, b->gtbl);
+        hipLaunchKernelGGL(k_group_count, dim3(g), dim3(kBlock), 0, s, d, b->S, b->tri_scene, toff_dev_of(b),
+                           b->gtbl);
         launch_exscan(d, b->gtbl, b->gtbl, (int64_t)b->S * g, nullptr, s);
         hipLaunchKernelGGL(k_group_scatter, dim3(g), dim3(kBlock), 0, s, d, b->S, b->tri_scene, toff_dev_of(b),
                            b->gtbl, b->scnt, b->grouped);
