@@ -390,7 +390,7 @@ void record_frame(bvhcd_batch* b, int bvh_op, unsigned grid) {
         launch_refit_prep(d, n, s);
     }
     launch_refit(d, n, s);
-    launch_batch_cd(d, n, b->keys, b->scene_last, grid, s);
+    launch_batch_cd(d, n, b->keys, b->scene_last, grid, bvh_op == BVHCD_BVH_BUILD, s);
     launch_narrow(d, s, true);  // launch_batch_cd reset the counters
     launch_pair_totals(d, s, true);
     if (b->S <= kGroupScenes) {
@@ -491,6 +491,8 @@ int bvhcd_batch_create(const bvhcd_config* cfg, int32_t S, const int64_t* tps, c
     ok &= balloc(b, d.int_ry, T);
     ok &= balloc(b, d.itopo, T);
     ok &= balloc(b, d.top_cut, 65);
+    ok &= balloc(b, d.cut, (size_t)cut_groups(T) * kCutCap);
+    ok &= balloc(b, d.cut_cnt, (size_t)cut_groups(T));
     ok &= balloc(b, d.tri_finite, T);
     ok &= balloc(b, d.lfaces, 3 * T);
     ok &= balloc(b, d.rp_cstart, (size_t)refit_chunks((int32_t)T) + 1);
@@ -716,9 +718,9 @@ int bvhcd_batch_autotune(bvhcd_batch* b) {
     float best_ms = 1e30f;
     unsigned best = batch_grid(b);
     for (unsigned g : {1024u, 2048u, 4096u, 8192u, 0xFFFFFFu}) {
-        launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, g, b->stream);  // warm-up
+        launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, g, false, b->stream);  // warm-up
         (void)hipEventRecord(e0, b->stream);
-        for (int r = 0; r < 3; ++r) launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, g, b->stream);
+        for (int r = 0; r < 3; ++r) launch_batch_cd(b->d, (int32_t)b->T, b->keys, b->scene_last, g, false, b->stream);
         (void)hipEventRecord(e1, b->stream);
         if (hipEventSynchronize(e1) != hipSuccess) {
             (void)hipEventDestroy(e0);

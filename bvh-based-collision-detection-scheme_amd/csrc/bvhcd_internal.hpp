@@ -288,6 +288,10 @@ struct DevState {
     const float* qverts = nullptr;
     int32_t nq = 0;
     int inter = 0;
+    // batched scenes: the cut of the tree at which each group of queries' search ended (kCutCap encoded
+    // nodes per group and how many there are; above kCutCap: not held), recorded by a build's traversal
+    uint32_t* cut = nullptr;
+    uint32_t* cut_cnt = nullptr;
     int64_t topo_version = 0;       // host-side: bumped by every topology change (refit preparation)
     int front_by_query = 0;         // host-side: the last produced fronts are ordered by query leaf
 };
@@ -371,6 +375,7 @@ __device__ inline bool leaves_share_vertex(const DevState& d, int32_t a, int32_t
     return faces_share_vertex(d.lfaces, a, b);
 }
 
+constexpr uint32_t kCutCap = 512;
 constexpr int kSceneParts = 1024;
 // Launch helpers
 constexpr int kBlock = 256;

@@ -823,6 +823,13 @@ __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, uint32_t per, De
 // triangles 185 -> 93 us (against the queries' own walks sharing a wave's lanes), 64 scenes of 2.6M
 // triangles 1.04 -> 0.56 ms (against a walk per lane). KEEP's test of a front stays where there is one:
 // 0.44 ms against 0.66 ms here on the 2M cloth, 13 us against 17 us on 2,560 triangles.
+// A group's cut (CUT): the nodes at which its search ended, which cover every leaf the group can meet.
+// The tree of the batched scenes stays for the refits between two builds: the build's traversal records
+// the groups' cuts, the others start from them instead of from the root (on 64 scenes 24 rounds of nodes
+// become 6; 0.61 -> 0.49 ms a refit
+// frame) and go on below a node that overlaps by now. A cut of more than kCutCap nodes isn't held,
+// its group starts from the root.
+enum GroupCut : int { kCutNone = 0, kCutRecord = 1, kCutRead = 2 };
 constexpr uint32_t kGroupStack = 512;  // encoded nodes per wave (2 KB)
 constexpr int kGroupPieces = 4;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -868,7 +875,7 @@ __device__ inline void wave_lds_order() {  // LDS operations of one wave complet
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool BATCH, bool RUNS>
+template <bool BATCH, bool RUNS, int CUT>
 __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, DevState d,
                                                      const uint64_t* __restrict__ keys,
                                                      const int32_t* __restrict__ scene_last) {
@@ -1054,22 +1061,42 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                     emit(c + u < k && j[u] > after && (!BATCH || j[u] <= last) && box_overlap(qb, lo[u], hi[u]), q, j[u]);
             }
         };
-        uint32_t top = d.top_cut[64], ncand = 0;  // wave-uniform
-        stk[lane] = d.top_cut[lane];
+        uint32_t top = 0, ncand = 0;         // wave-uniform
+        uint32_t cn = 0, next = 0, rec = 0;  // the cut's nodes, those taken of them, nodes recorded
+        uint32_t ids = 0;                    // the cut's next 64 nodes
+        uint32_t* const cut = CUT ? d.cut + (int64_t)gi * kCutCap : nullptr;
+        if (CUT == kCutRead) cn = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.cut_cnt[gi]);
+        if (CUT == kCutRead && cn <= kCutCap) {
+            if ((uint32_t)lane < cn) ids = cut[lane];
+        } else {  // from the cut near the root
+            cn = 0;
+            top = d.top_cut[64];
+            stk[lane] = d.top_cut[lane];
+        }
         // every node enters the stack at most once; the bound only guards against a corrupted tree
         // (flag 16, reported as a device error, instead of a hang)
         const int64_t limit = 2 * d.maxT + 16;
-        for (int64_t round = 0; top > 0; ++round) {
+        for (int64_t round = 0; top > 0 || next < cn; ++round) {
             if (round > limit) {
                 if (lane == 0) atomicOr(ovf, 16u);
                 break;
             }
-            const uint32_t take = max(1u, min(min(top, 64u), kGroupStack - top));
-            top -= take;
+            uint32_t take;
+            int32_t e = 0;
+            if (CUT == kCutRead && next < cn && top < 64u) {
+                take = min(cn - next, 64u);
+                e = (int32_t)ids;
+                next += take;
+                ids = next + lane < cn ? cut[next + lane] : 0u;
+            } else {
+                take = max(1u, min(min(top, 64u), kGroupStack - top));
+                top -= take;
+                if ((uint32_t)lane < take) e = (int32_t)stk[top + lane];
+            }
             const bool act = (uint32_t)lane < take;
-            const int32_t e = act ? (int32_t)stk[top + lane] : 0, nd = e >> 1;
+            const int32_t nd = e >> 1;
             const bool leaf = e & 1;
-            bool hit = false;
+            bool hit = false, ends = false;  // ends: the search stops at this node, or walks on below it
             float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
             int4 tp = make_int4(0, 0, 0, 0);
             if (act) {
@@ -1082,7 +1109,9 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                 bool any = false;
 #pragma unroll
                 for (int c = 0; c < kGroupPieces; ++c) any |= box_overlap(piece[c], lo, hi);
-                hit = any && end > g0 && (!BATCH || begin <= glast);
+                const bool ours = end > g0 && (!BATCH || begin <= glast);
+                hit = any && ours;
+                ends = ours && (leaf || !any);
             }
             const uint64_t mi = __ballot(hit && !leaf), ml = __ballot(hit && leaf);
             if (mi) {
@@ -1094,6 +1123,7 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                 }
                 const uint64_t mf = __ballot(hit && !leaf && fits);
                 top += 2u * (uint32_t)__popcll(mf);
+                ends = ends || (hit && !leaf && !fits);
                 // no room (only a full stack's last item, see `take`): the lanes walk that subtree
                 for (uint64_t over = mi & ~mf; over; over &= over - 1ull) {
                     const int src = __ffsll((long long)over) - 1;
@@ -1126,6 +1156,12 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                     }
                 }
             }
+            if (CUT == kCutRecord) {
+                const uint64_t me = __ballot(ends);
+                const uint32_t slot = rec + (uint32_t)__popcll(me & lanes_below());
+                if (ends && slot < kCutCap) cut[slot] = (uint32_t)e;
+                rec += (uint32_t)__popcll(me);
+            }
             if (RUNS) {
                 if (ml) test_runs(hit && leaf, nd, lo, hi);
                 continue;
@@ -1135,19 +1171,21 @@ __global__ void __launch_bounds__(kBlock) k_group_cd(int32_t n, uint32_t size, D
                 ncand += (uint32_t)__popcll(ml);
                 wave_lds_order();
             }
-            if (ncand >= 64u || (top == 0u && ncand > 0u)) {
+            const bool done = top == 0u && next >= cn;
+            if (ncand >= 64u || (done && ncand > 0u)) {
                 test_leaves(min(ncand, 64u));
                 const uint32_t rest = ncand > 64u ? ncand - 64u : 0u;
                 if ((uint32_t)lane < rest) cand[lane] = cand[64 + lane];
                 wave_lds_order();
                 ncand = rest;
-                if (top == 0u && ncand > 0u) {  // the last round's overhang
+                if (done && ncand > 0u) {  // the last round's overhang
                     test_leaves(ncand);
                     ncand = 0;
                 }
             }
         }
         flush();
+        if (CUT == kCutRecord && lane == 0) d.cut_cnt[gi] = rec;  // above kCutCap: not held
     }
     add_visits(d, visits);
 }
@@ -1169,13 +1207,14 @@ static unsigned group_grid(int32_t n) {
 // the LDS and a third fewer resident waves, which larger scenes need (us, runs / every lane its query: 7k
 // 48 / 69, 65k 47 / 66, 130k 70 / 88, 318k 136 / 165, 718k 363 / 370, 1.2M 611 / 574, 2.1M 775 / 716).
 constexpr int32_t kGroupRuns = 3 << 18;
-template <bool BATCH>
+int64_t cut_groups(int64_t n) { return (n + group_size((int32_t)n) - 1) / group_size((int32_t)n); }
+template <bool BATCH, int CUT>
 static void launch_group_cd(DevState& d, int32_t n, unsigned grid, const uint64_t* keys, const int32_t* scene_last,
                             hipStream_t s) {
     if (n <= kGroupRuns)
-        hipLaunchKernelGGL((k_group_cd<BATCH, true>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
+        hipLaunchKernelGGL((k_group_cd<BATCH, true, CUT>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
     else
-        hipLaunchKernelGGL((k_group_cd<BATCH, false>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
+        hipLaunchKernelGGL((k_group_cd<BATCH, false, CUT>), dim3(grid), dim3(kBlock), 0, s, n, group_size(n), d, keys, scene_last);
 }
 
 // Queries of a traversal: the leaves before the last one (self-CD) or the other object's leaves.
@@ -1200,7 +1239,7 @@ void launch_pure_cd(DevState& d, int32_t n, hipStream_t s) {
     reset_step_counters(d, s);
     const int64_t nq = query_count(d, n);
     if (group_ok(d) && nq > 0)
-        launch_group_cd<false>(d, n, group_grid(n), nullptr, nullptr, s);
+        launch_group_cd<false, kCutNone>(d, n, group_grid(n), nullptr, nullptr, s);
     else if (nq > 0) {
         hipLaunchKernelGGL(k_traverse<false>, dim3(walk_grid(nq)), dim3(kBlock), 0, s, n, walk_queries(nq), d,
                            null_sink(), null_sink());
@@ -1214,10 +1253,12 @@ void launch_pure_cd(DevState& d, int32_t n, hipStream_t s) {
 // groups of its XCD's share in turn. Counters are cleared with a kernel (no memset nodes) so that
 // the sequence can be captured in a graph.
 void launch_batch_cd(DevState& d, int32_t n, const uint64_t* keys, const int32_t* scene_last, unsigned grid,
-                     hipStream_t s) {
+                     bool built, hipStream_t s) {
     reset_step_counters(d, s);
     const unsigned g = std::min(group_grid(n), kXcds * std::max(grid / kXcds, 1u));
-    if (n >= 2) launch_group_cd<true>(d, n, g, keys, scene_last, s);
+    if (n < 2) return;
+    if (built) launch_group_cd<true, kCutRecord>(d, n, g, keys, scene_last, s);
+    else launch_group_cd<true, kCutRead>(d, n, g, keys, scene_last, s);
 }
 
 // ---------------------------------------------------------------- ordering

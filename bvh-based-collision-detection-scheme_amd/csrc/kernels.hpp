@@ -48,9 +48,11 @@ void launch_emit_full64(DevState& d, const uint64_t* keys, int32_t n, hipStream_
 // (tkeys, tvals).
 bool radix_sort_u64_dev(DevState& d, uint64_t* keys, int32_t* vals, uint64_t* tkeys, int32_t* tvals, int64_t n,
                         int nbits, hipStream_t s);
-// Batched self-CD over per-scene subtrees, at most `grid` workgroups; pairs into d.bp.
+// Batched self-CD over per-scene subtrees, at most `grid` workgroups; pairs into d.bp. built: the first
+// one on a new tree, which records the groups' cuts for the others.
 void launch_batch_cd(DevState& d, int32_t n, const uint64_t* keys, const int32_t* scene_last, unsigned grid,
-                     hipStream_t s);
+                     bool built, hipStream_t s);
+int64_t cut_groups(int64_t n);  // groups of queries over n triangles
 void launch_emit_runs(DevState& d, int32_t n, const int32_t* rt_of_leaf, int32_t* leaf_lo, int32_t* leaf_hi,
                       int32_t* split_lo, int32_t* split_hi, int32_t* base, int32_t* keep_par, uint32_t* keep_mark,
                       hipStream_t s);

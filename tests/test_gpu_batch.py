@@ -201,3 +201,38 @@ def test_batch_grouping_by_scene_count(pkg, num):
             want = [(i, j) for i in range(tris[k]) for j in range(i + 1, tris[k])]
             np.testing.assert_array_equal(_set(b.pairs(k)), np.array(want, np.int32).reshape(-1, 2))
     b.close()
+
+
+@pytest.mark.parametrize("t_max", [700, 9000])
+def test_batch_refits_far_from_the_build(pkg, oracle, t_max):
+    """Refits whose vertices have moved far since the build (the groups' recorded cuts lie deep above the
+    new overlaps) and a build on crumpled scenes (cuts too long to be held), eagerly and by graph: every
+    scene's pairs are those of a context of its own."""
+    print(f"[gpu] batch refits far from the build, {t_max}", flush=True)
+    scenes = _scenes(pkg, 5, seed=3, frames=12, t_min=300, t_max=t_max)
+    rng = np.random.default_rng(t_max)
+    flat = [s.frame(2) for s in scenes]
+    crumpled = [(f * 0.3 + rng.normal(0, 0.03, f.shape)).astype(np.float32) for f in flat]
+    plan = [(flat, pkg.BVH_BUILD), (crumpled, pkg.BVH_REFIT), (flat, pkg.BVH_REFIT), (crumpled, pkg.BVH_BUILD),
+            (crumpled, pkg.BVH_REFIT), (flat, pkg.BVH_REFIT)]
+    want = []
+    for k, sc in enumerate(scenes):
+        ctx = pkg.CollisionContext(sc.num_tris, sc.num_verts, pair_cap=1 << 22)
+        ctx.set_topology(sc.faces(), sc.num_verts)
+        want.append([])
+        for v, op in plan:
+            ctx.update_vertices(v[k])
+            ctx.step(op, pkg.FRONT_PURE_BVH_CD)
+            want[k].append(oracle.pair_set(ctx.pairs(True)))
+        ctx.close()
+    for use_graph in (False, True):
+        b = pkg.Batch([s.num_tris for s in scenes], [s.num_verts for s in scenes], pair_cap=1 << 23)
+        b.set_topology(np.concatenate([s.faces() for s in scenes]))
+        for f, (v, op) in enumerate(plan):
+            b.update_vertices(np.concatenate(v))
+            b.step(op, use_graph=use_graph)
+            b.pair_counts()
+            for k in range(len(scenes)):
+                np.testing.assert_array_equal(oracle.pair_set(b.pairs(k)), want[k][f],
+                                              err_msg=f"scene {k} frame {f} graph {use_graph}")
+        b.close()
