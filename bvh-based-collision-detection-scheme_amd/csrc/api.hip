@@ -184,6 +184,11 @@ int allocate(bvhcd_ctx* c) {
     ok &= dalloc(c, d.prim_map, T);
     ok &= dalloc(c, d.inode, T);
     ok &= dalloc(c, d.leaf, T);
+    if (T >= kQFrom) {
+        ok &= dalloc(c, d.qnode, T);
+        ok &= dalloc(c, d.qleafrec, T);
+        ok &= dalloc(c, d.qgrid, 16);
+    }
     ok &= dalloc(c, d.int_lc, T);
     ok &= dalloc(c, d.int_rc, T);
     ok &= dalloc(c, d.int_par, T);

@@ -61,6 +61,48 @@ __device__ inline Box tri_box(const int32_t* __restrict__ faces, const float* __
     return bx;
 }
 
+// ------------------------------------------------------------------ 16-byte node records
+// A box on a 20-bit grid per axis, in fields of 21 bits: x = the minima, y = 1048575 - the maxima. All
+// coordinates go through one non-decreasing map, so the grid decides the boxes' order wherever two
+// grid coordinates differ; only equal ones leave it open. For records a, b the fields of a.x + b.y are
+// a.min - b.max + 1048575, those of b.x + a.y are b.min - a.max + 1048575: above 1048575 the boxes are
+// apart, below they overlap on that axis, at 1048575 the grid can't tell.
+constexpr uint64_t kQOne = 1ull | 1ull << 21 | 1ull << 42, kQTop = kQOne << 20;
+constexpr float kQMax = 1048575.f;
+__device__ inline uint64_t q_min(float x, float lo, float scale) {  // NaN: 0 (a NaN bound is never past another)
+    return (uint64_t)(uint32_t)fminf(fmaxf((x - lo) * scale, 0.f), kQMax);
+}
+__device__ inline uint64_t q_max(float x, float lo, float scale) {  // NaN: the largest
+    return (uint64_t)(1048575u - (uint32_t)fmaxf(fminf((x - lo) * scale, kQMax), 0.f));
+}
+__device__ inline ulonglong2 q_record(const float* __restrict__ g, const Box& b) {
+    return make_ulonglong2(q_min(b.mnx, g[0], g[3]) | q_min(b.mny, g[1], g[4]) << 21 | q_min(b.mnz, g[2], g[5]) << 42,
+                           q_max(b.mxx, g[0], g[3]) | q_max(b.mxy, g[1], g[4]) << 21 | q_max(b.mxz, g[2], g[5]) << 42);
+}
+// The grid of a scene: its box and an eighth on each side. Boxes that leave it by the next refit end up at
+// its edges, where the grid can't tell.
+__device__ inline void q_axis(float* g, float mn, float mx, int axis) {
+    const float ext = mx - mn;
+    const bool ok = ext > 0.f && ext < 1e30f && fabsf(mn) < 1e30f;
+    g[axis] = ok ? mn - 0.125f * ext : 0.f;
+    g[3 + axis] = ok ? fmaxf(fminf(838860.f / ext, 1e30f), 1e-30f) : 1e-30f;
+}
+__device__ inline void q_grid(float* g, const Box& b) {
+    q_axis(g, b.mnx, b.mxx, 0);
+    q_axis(g, b.mny, b.mxy, 1);
+    q_axis(g, b.mnz, b.mxz, 2);
+}
+// Are the boxes apart; unless they are, `open` where the grid can't tell.
+__device__ inline bool q_apart(const ulonglong2& a, const ulonglong2& b, bool& open) {
+    const uint64_t s = a.x + b.y, t = b.x + a.y;
+    open = (((s + kQOne) | (t + kQOne)) & kQTop) != 0ull;
+    return ((s | t) & kQTop) != 0ull;
+}
+// Contexts of this many triangles have the records, and KEEP tests them first from that many on. (With 15
+// bits per coordinate, in three words, 5 % of the entries stayed open on sheets that lie on one another,
+// and their second tests took KEEP from 1.17 to 1.53 ms on 8.4M triangles.)
+constexpr int32_t kQFrom = 1 << 20;
+
 // ------------------------------------------------------------------ Morton (30-bit)
 __host__ __device__ inline uint32_t expand_bits(uint32_t v) {
     v = (v * 0x00010001u) & 0xFF0000FFu;
@@ -151,6 +193,12 @@ struct DevState {
     int32_t* prim_map = nullptr;    // T triangle -> slot
     NodeRec* inode = nullptr;       // T-1 (preorder)
     NodeRec* leaf = nullptr;        // T
+    // KEEP's 16-byte node records (q_record; null: none) and the grids they are on: 2 x 8 words, the
+    // current one at 8 * qpar, the other one left by a refit for the next
+    ulonglong2* qnode = nullptr;    // T-1
+    ulonglong2* qleafrec = nullptr; // T
+    float* qgrid = nullptr;
+    int qpar = 0;                   // host-side
     int32_t* int_lc = nullptr;      // T-1
     int32_t* int_rc = nullptr;
     int32_t* int_par = nullptr;

@@ -1764,14 +1764,19 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
     return visits;
 }
 
-// KEEP over the current front, U entries per thread per loop iteration with all their loads
-// issued together: the kernel is bound by the latency of dependent loads (entry, then the two
-// node records), so more loads in flight per wave is what speeds it up.
+// KEEP over the current front, U entries per thread per loop iteration with all their loads issued
+// together. Bound by the vector L1: a wave's load of 64 different records takes 65 cycles of its CU
+// whatever the load's width, so a box in two 16-byte loads costs 130 of the 215 cycles that 64 entries
+// take (74 % of the L1's cycles busy, 40 % of the VALU's). On large scenes (Q) the entries are therefore
+// tested on 16-byte records, one load each, and the few that those leave open (0.2 %), like the descents,
+// on the boxes. KEEP, us, boxes -> Q: 1.2M triangles 267..428 -> 242..355 over ten frames of a front, 2.1M
+// 414..638 -> 363..583, 8.4M 1170 -> 1033; the refit that writes the records takes 9 us (2.1M) and 67 us
+// (8.4M) longer. Below a million triangles the gain is within that cost.
 // implicit: the current front's shared-vertex head (C_ADJ entries after the last partition) is
 // not tested when the last refit found every coordinate finite: its pairs are broad-phase hits
 // whatever the positions (both boxes hold the shared vertex) and are counted, not listed.
 // W = waves per workgroup (the tuner picks it with the grid and U).
-template <int U, int W>
+template <int U, int W, bool Q>
 __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int implicit) {
     __shared__ StagesBPT<W> st;
     __shared__ DescStack<W> ds;
@@ -1823,12 +1828,22 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
             q[u] = qn[u];
             nd[u] = ndn[u];
         }
-        float4 qlo[U], qhi[U], lo[U], hi[U];
+        float4 qlo[Q ? 1 : U], qhi[Q ? 1 : U], lo[Q ? 1 : U], hi[Q ? 1 : U];
+        ulonglong2 qa[Q ? U : 1], na[Q ? U : 1];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+            const bool internal = k0 + u * stride < ni;
+            if (Q) {
+                qa[u] = na[u] = make_ulonglong2(0ull, 0ull);
+                if (q[u] >= 0) {
+                    qa[u] = d.qleafrec[q[u]];
+                    na[u] = internal ? d.qnode[nd[u]] : d.qleafrec[nd[u]];
+                }
+                continue;
+            }
             qlo[u] = qhi[u] = lo[u] = hi[u] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (q[u] >= 0) {
-                const NodeRec* r = k0 + u * stride < ni ? &d.inode[nd[u]] : &d.leaf[nd[u]];
+                const NodeRec* r = internal ? &d.inode[nd[u]] : &d.leaf[nd[u]];
                 qlo[u] = d.qleaf[q[u]].lo;
                 qhi[u] = d.qleaf[q[u]].hi;
                 lo[u] = r->lo;
@@ -1839,8 +1854,20 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const bool internal = k0 + u * stride < ni;
-            const Box qb = rec_box(qlo[u], qhi[u]);
-            const bool hit = q[u] >= 0 && box_overlap(qb, lo[u], hi[u]);
+            bool hit;
+            if (Q) {  // where the grid can't tell, the entry itself goes on the stack for a test of the boxes
+                bool open;
+                hit = q[u] >= 0 && !q_apart(qa[u], na[u], open);
+                const bool later = hit && open;
+                if (!desc_push(stk, stop, later, q[u], nd[u] << 1 | (internal ? 0 : 1))) {  // no room: here
+                    const NodeRec *a = &d.qleaf[q[u]], *b = internal ? &d.inode[nd[u]] : &d.leaf[nd[u]];
+                    hit = box_overlap(rec_box(a->lo, a->hi), b->lo, b->hi);
+                } else {
+                    hit = hit && !open;
+                }
+            } else {
+                hit = q[u] >= 0 && box_overlap(rec_box(qlo[u], qhi[u]), lo[u], hi[u]);
+            }
             visits += q[u] >= 0 ? 1u : 0u;
             // the node now overlaps: its children go on the wave's stack
             const bool desc = internal && hit;
@@ -1851,7 +1878,8 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
             const bool ok_r = desc_push(stk, stop, desc, q[u], rc);
             if (desc && !(ok_l && ok_r)) {  // no room on the stack: this lane walks the subtree
                 const int32_t start = ok_l ? rc : lc;
-                visits += stackless<false>(d, out, q[u], qb, start, f2i(hi[u].w));
+                const float4 a = d.qleaf[q[u]].lo, b = d.qleaf[q[u]].hi;
+                visits += stackless<false>(d, out, q[u], rec_box(a, b), start, f2i(d.inode[nd[u]].hi.w));
             }
             bool emit = hit && !internal;
             if (out.skip_adj && emit) emit = !faces_share_vertex(out.lfaces, q[u], nd[u]);
@@ -1958,7 +1986,10 @@ void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
     if (!counters_zeroed) reset_step_counters(d, s);
     const unsigned sh = tuned_shape(TK_KEEP, n, d.inter ? d.nq : 0), g = shape_grid(sh), w = shape_waves(sh);
     const FrontIn in = cur_front(d);
-#define BVHCD_KEEP(U, W) hipLaunchKernelGGL((k_keep<U, W>), dim3(g), dim3(64 * W), 0, s, d, in, implicit)
+    const bool q = !d.inter && d.qnode && n >= kQFrom;
+#define BVHCD_KEEP(U, W)                                                                             \
+    if (q) hipLaunchKernelGGL((k_keep<U, W, true>), dim3(g), dim3(64 * W), 0, s, d, in, implicit);   \
+    else hipLaunchKernelGGL((k_keep<U, W, false>), dim3(g), dim3(64 * W), 0, s, d, in, implicit)
     switch (shape_unroll(sh) * 16 + w) {
         case 4 * 16 + 8: BVHCD_KEEP(4, 8); break;
         case 4 * 16 + 2: BVHCD_KEEP(4, 2); break;
@@ -2071,7 +2102,7 @@ void launch_front_restr_apply(DevState& d, int32_t n, uint32_t ntasks, hipStream
     FrontIn kept = cur_front(d);
     kept.size[0] = d.ctr + C_KEPT_I;
     kept.size[1] = d.ctr + C_KEPT_E;
-    hipLaunchKernelGGL((k_keep<1, kWaves>), dim3(stream_grid()), dim3(kBlock), 0, s, d, kept, 0);
+    hipLaunchKernelGGL((k_keep<1, kWaves, false>), dim3(stream_grid()), dim3(kBlock), 0, s, d, kept, 0);
     // the walks write segments into the spare buffers, then append after the kept entries
     front_begin(d, s);
     FrontSink fi = next_sink(d, 0), fe = next_sink(d, 1);

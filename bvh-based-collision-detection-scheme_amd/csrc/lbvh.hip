@@ -1316,6 +1316,13 @@ __device__ inline void store_box(NodeRec* rec, const Box& b) {
     p[0].x = b.mnx; p[0].y = b.mny; p[0].z = b.mnz;
     p[1].x = b.mxx; p[1].y = b.mxy; p[1].z = b.mxz;
 }
+// An internal node's records. The root (preorder: id 0) also gives the next refit its grid.
+__device__ inline void store_node(const DevState& d, int32_t id, const Box& b) {
+    store_box(&d.inode[id], b);
+    if (!d.qnode) return;
+    d.qnode[id] = q_record(d.qgrid + 8 * d.qpar, b);
+    if (id == 0) q_grid(d.qgrid + 8 * (d.qpar ^ 1), b);
+}
 
 __global__ void __launch_bounds__(kRefitBlock) k_refit(int32_t n, DevState d) {
     __shared__ Box sb[kChunkCap];
@@ -1361,6 +1368,7 @@ __global__ void __launch_bounds__(kRefitBlock) k_refit(int32_t n, DevState d) {
             bad |= fin ? 0 : 1;
             sb[x - s] = b;
             store_box(&d.leaf[x], b);
+            if (d.qleafrec) d.qleafrec[x] = q_record(d.qgrid + 8 * d.qpar, b);
         }
     }
     int2 v[kRefitPerT];
@@ -1393,7 +1401,7 @@ __global__ void __launch_bounds__(kRefitBlock) k_refit(int32_t n, DevState d) {
 #pragma unroll
     for (int k = 0; k < kRefitPerT; ++k) {
         if (v[k].x < 0) continue;
-        store_box(&d.inode[v[k].x], out[k]);
+        store_node(d, v[k].x, out[k]);
         // a treelet root under an LDS-sized top tree also hands its box to the top kernel, which
         // then loads it without a dependent load
         if (dest[k] >= 0) {
@@ -1455,7 +1463,7 @@ __device__ inline void refit_top_records(const DevState& d, Box* lds, int32_t m,
 #pragma unroll
             for (int j = 0; j < K; ++j)
                 if (at + (int32_t)threadIdx.x + j * kTopBlock < b1 && (whole || top_depth(e[j]) == lev))
-                    store_box(&d.inode[e[j].x], box_merge(l[j], r[j]));
+                    store_node(d, e[j].x, box_merge(l[j], r[j]));
         };
         int32_t at = b0;
         for (; b1 - at > 2 * kTopBlock; at += 4 * kTopBlock) batch(at, std::integral_constant<int, 4>{});
@@ -1477,7 +1485,7 @@ __device__ inline void refit_top_climb(const DevState& d, int32_t m) {
         const int lk = top_kind(e, 0), rk = top_kind(e, 1);
         if ((lk == 0 && rp_is_top(d, e.y)) || (rk == 0 && rp_is_top(d, e.z))) continue;
         Box b = box_merge(below_top_record(d, lk, e.y), below_top_record(d, rk, e.z));
-        store_box(&d.inode[e.x], b);
+        store_node(d, e.x, b);
         for (int32_t q = e.x;;) {
             const int4 tq = d.itopo[q];
             const int32_t u = tq.z >> 1;
@@ -1491,7 +1499,7 @@ __device__ inline void refit_top_climb(const DevState& d, int32_t m) {
                 flag[u] = 0;
             }
             b = box_merge(b, below_top_record(d, sk, sib));
-            store_box(&d.inode[u], b);
+            store_node(d, u, b);
             q = u;
         }
     }
@@ -1590,7 +1598,7 @@ __global__ void __launch_bounds__(kTopBlock) k_refit_top(DevState d, int32_t chu
 #pragma unroll
     for (int k = 0; k < kTopPer; ++k) {
         const int32_t i = threadIdx.x + k * kTopBlock;
-        if (i < p1) store_box(&d.inode[e[k].x], tb[i]);
+        if (i < p1) store_node(d, e[k].x, tb[i]);
     }
     if (threadIdx.x < 64) {
         // wave 0: LDS operations of one wave complete in issue order, so a level's writes are
@@ -1607,7 +1615,7 @@ __global__ void __launch_bounds__(kTopBlock) k_refit_top(DevState d, int32_t chu
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        if (i < m) store_box(&d.inode[ew.x], tb[i]);
+        if (i < m) store_node(d, ew.x, tb[i]);
     }
     // the upper nodes above the segments: merged through the node records by the segment
     // workgroup that finishes last (release of this workgroup's records, then a counter; the
@@ -1628,6 +1636,7 @@ void launch_refit(DevState& d, int32_t n, hipStream_t s, bool zero_step_counters
     hipLaunchKernelGGL(k_refit, dim3(refit_chunks(n)), dim3(kRefitBlock), 0, s, n, d);
     hipLaunchKernelGGL(k_refit_top, dim3(kTopGrid), dim3(kTopBlock), 0, s, d, refit_chunks(n),
                        zero_step_counters ? 1 : 0);
+    d.qpar ^= 1;
 }
 
 // ======================================================================= prim map / misc
@@ -1649,6 +1658,10 @@ __global__ void __launch_bounds__(kBlock) k_leaf_setup(int32_t n, int32_t chunks
         *d.rp_tcount = 0u;
         *d.rp_tdone = 0u;
         *d.rp_tdeep = 0u;
+        if (d.qgrid) {  // the first refit's grid
+            const float* b = d.scene_box;
+            q_grid(d.qgrid + 8 * d.qpar, Box{b[0], b[1], b[2], b[3], b[4], b[5]});
+        }
     }
 }
 void launch_leaf_setup(DevState& d, int32_t n, hipStream_t s) {

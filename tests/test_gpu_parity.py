@@ -829,3 +829,53 @@ def test_pure_traversal_equals_generate_at_its_switches(pkg, n):
     ctx.step(pkg.BVH_NONE, pkg.FRONT_GENERATE)
     assert got == ctx.digest(False) and got[1] > sc.num_tris
     ctx.close()
+
+
+@pytest.mark.parametrize("state", ["flat", "folded", "far", "tiny", "bad", "boxes"])
+def test_keep_on_grid_records_equals_boxes(pkg, state):
+    """KEEP's 16-byte records (scenes of 2^20 triangles or more) against GENERATE's boxes on the same tree:
+    a flat sheet (every coordinate of one axis on one grid line), a folded one, scenes that left the
+    grid or shrank to a few grid lines since the build, infinities and NaN, and boxes given by the caller
+    with NaN among them."""
+    sc = pkg.Scene.preset("cloth1024", n=726)
+    print(f"[gpu] keep on grid records: {state}, {sc.num_tris}", flush=True)
+    assert sc.num_tris >= 1 << 20
+    faces, rng = sc.faces(), np.random.default_rng(4)
+    v0 = sc.frame(0 if state == "flat" else sc.frames - 2)
+    v1 = sc.frame(1 if state == "flat" else sc.frames - 1)
+    if state == "far":
+        v1 = v1 + np.float32(300.0)
+    if state == "tiny":
+        v1 = (v1 * np.float32(1e-4)).astype(np.float32)
+    if state == "bad":
+        v1 = v1.copy()
+        v1[rng.integers(0, len(v1), 40)] = np.nan
+        v1[rng.integers(0, len(v1), 3), 1] = np.inf
+        v1[7, 2] = -np.inf
+    ctx = _ctx(pkg, sc, narrow_phase=False)
+    frames = [v0, v1, v1, v0]
+    if state == "boxes":
+        frames = [np.concatenate([v[faces].min(1), v[faces].max(1)], 1).astype(np.float32) for v in frames]
+        for k in (1, 2):
+            frames[k][rng.integers(0, len(faces), 30), rng.integers(0, 6, 30)] = np.nan
+    for k, x in enumerate(frames):
+        if state == "boxes":
+            ctx.update_boxes(x)
+        else:
+            ctx.update_vertices(x)
+        if k == 0:
+            ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)
+            continue
+        if state == "boxes":  # a fresh front of the same boxes holds each entry as its box test has it
+            ctx.step(pkg.BVH_REFIT, pkg.FRONT_GENERATE)
+            want = ctx.digest(False)
+            ctx.step(pkg.BVH_NONE, pkg.FRONT_KEEP)
+            assert ctx.digest(False) == want, k
+            continue
+        ctx.step(pkg.BVH_REFIT, pkg.FRONT_KEEP)
+        keep = ctx.digest(False)
+        ctx.step(pkg.BVH_NONE, pkg.FRONT_PURE_BVH_CD)
+        assert keep == ctx.digest(False) and keep[1] > sc.num_tris, k
+        ctx.step(pkg.BVH_NONE, pkg.FRONT_GENERATE)
+        assert keep == ctx.digest(False), k
+    ctx.close()
