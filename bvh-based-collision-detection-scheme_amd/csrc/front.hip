@@ -1904,35 +1904,39 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
 // flags its tile (flags in registers), takes the tile's places with one atomic, the head's from the
 // front's start and the rest's from its end, and reads the entries again to place them. A tile keeps
 // its order; tiles follow one another about as they are dispatched. Bound by the faces gathered per
-// entry (both triangles'), once: 2M cloth, 35M entries 0.30 -> 0.28 ms against counting, a scan and a
-// scatter that tested every entry twice; 41k triangles 40 -> 19 us.
-template <int ITEMS>
-__global__ void __launch_bounds__(kBlock) k_adj_partition(DevState d, FrontIn in, uint32_t* __restrict__ dst_node,
+// entry (both triangles'), once. The tiles' atomics follow one another, about 30 per us, so that large
+// scenes take tiles of 16384 entries, by 1024 threads: the 2M cloth's 35M entries 0.29 -> 0.22 ms against
+// 256 threads with four times the rounds, 0.25 ms with tiles of 4096; 8.4M sheets' 74M 0.52 -> 0.43 ms.
+// (Counting, a scan and a scatter, each entry tested twice: 0.30 ms; 41k triangles 40 us, here 17.)
+constexpr int kAdjItems = 16;  // entries per thread
+template <int W>
+__global__ void __launch_bounds__(64 * W) k_adj_partition(DevState d, FrontIn in, uint32_t* __restrict__ dst_node,
                                                           int32_t* __restrict__ dst_query, uint32_t* dst_size) {
-    static_assert(ITEMS * kWaves <= kBlock, "one thread per round and wave in the scan");
-    __shared__ uint32_t cnt[ITEMS * kWaves];  // flagged entries before each round's wave
+    constexpr int ITEMS = kAdjItems, B = 64 * W;
+    static_assert(ITEMS * W % 64 == 0, "whole waves of counts");
+    __shared__ uint32_t cnt[ITEMS * W];  // flagged entries before each round's wave
     __shared__ uint32_t base_head, base_rest;
     const uint32_t ne = min(*in.size[1], in.cap[1]);
     if (blockIdx.x == 0 && threadIdx.x == 0) *dst_size = ne;
-    const uint64_t b0 = (uint64_t)blockIdx.x * (kBlock * ITEMS);
+    const uint64_t b0 = (uint64_t)blockIdx.x * (B * ITEMS);
     if (b0 >= ne) return;  // block-uniform
-    const uint32_t left = (uint32_t)min<uint64_t>(ne - b0, kBlock * ITEMS);  // the tile's entries
+    const uint32_t left = (uint32_t)min<uint64_t>(ne - b0, B * ITEMS);  // the tile's entries
     const uint32_t* node = in.node[1] + b0;
     const int32_t* query = in.query[1] + b0;
     const int w = threadIdx.x >> 6;
     uint64_t flags = 0;
 #pragma unroll 4
     for (int r = 0; r < ITEMS; ++r) {
-        const uint32_t i = r * kBlock + threadIdx.x;
+        const uint32_t i = r * B + threadIdx.x;
         const bool adj = i < left && leaves_share_vertex(d, query[i], (int32_t)node[i]);
         flags |= adj ? 1ull << r : 0ull;
         const uint64_t m = __ballot(adj);
-        if (lane_id() == 0) cnt[r * kWaves + w] = (uint32_t)__popcll(m);
+        if (lane_id() == 0) cnt[r * W + w] = (uint32_t)__popcll(m);
     }
     __syncthreads();
     if (threadIdx.x < 64) {  // exclusive scan of the counts
         uint32_t carry = 0;
-        for (int g = 0; g < ITEMS * kWaves; g += 64) {
+        for (int g = 0; g < ITEMS * W; g += 64) {
             const uint32_t v = cnt[g + threadIdx.x];
             uint32_t x = v;
             for (int off = 1; off < 64; off <<= 1) {
@@ -1953,11 +1957,11 @@ __global__ void __launch_bounds__(kBlock) k_adj_partition(DevState d, FrontIn in
     __syncthreads();
 #pragma unroll 4
     for (int r = 0; r < ITEMS; ++r) {
-        const uint32_t i = r * kBlock + threadIdx.x;
+        const uint32_t i = r * B + threadIdx.x;
         const bool adj = (flags >> r) & 1ull;
         const uint64_t m = __ballot(adj);
         if (i >= left) continue;
-        const uint32_t before = cnt[r * kWaves + w] + (uint32_t)__popcll(m & lanes_below());  // flagged ones
+        const uint32_t before = cnt[r * W + w] + (uint32_t)__popcll(m & lanes_below());  // flagged ones
         const uint32_t o = adj ? base_head + before : base_rest + (i - before);
         dst_node[o] = node[i];
         dst_query[o] = query[i];
@@ -1969,12 +1973,13 @@ void launch_adj_partition(DevState& d, int32_t n, hipStream_t s) {
     const int nb = d.fcur[1] ^ 1;
     fill_u32(d.ctr + C_ADJ, 2, 0u, s);
     // tiles of 16384 entries on large scenes: the tiles' atomics follow one another
+    const int64_t waves = (d.front_cap[1] + 64 * kAdjItems - 1) / (64 * kAdjItems);
     if (n > (1 << 19))
-        hipLaunchKernelGGL(k_adj_partition<64>, dim3(grid_for(d.front_cap[1], 64 * kBlock)), dim3(kBlock), 0, s, d, in,
-                           d.fnode[1][nb], d.fquery[1][nb], d.fsize + 2 + nb);
+        hipLaunchKernelGGL(k_adj_partition<16>, dim3(grid_for(waves, 16)), dim3(1024), 0, s, d, in, d.fnode[1][nb],
+                           d.fquery[1][nb], d.fsize + 2 + nb);
     else
-        hipLaunchKernelGGL(k_adj_partition<16>, dim3(grid_for(d.front_cap[1], 16 * kBlock)), dim3(kBlock), 0, s, d, in,
-                           d.fnode[1][nb], d.fquery[1][nb], d.fsize + 2 + nb);
+        hipLaunchKernelGGL(k_adj_partition<4>, dim3(grid_for(waves, 4)), dim3(256), 0, s, d, in, d.fnode[1][nb],
+                           d.fquery[1][nb], d.fsize + 2 + nb);
     d.fcur[1] = nb;
     d.adj_version = d.front_version;
 }
