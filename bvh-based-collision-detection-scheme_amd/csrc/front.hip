@@ -632,16 +632,18 @@ int size_class(int64_t n) {
 }  // namespace
 
 // The shapes used until a kernel is tuned. n = triangles of the scene (of the querying object for an
-// inter-object front). KEEP on small scenes is bound by the length of its dependent rounds, and one
-// resident set of workgroups with two entries in flight per thread has the fewest; on large ones by
-// throughput, where small workgroups leave the tail early. One launch, ms, 2048 x 256 threads with one
-// entry each -> these: 41k triangles 0.037 -> 0.025, 65k 0.040 -> 0.029, 130k 0.046 -> 0.036,
-// 1.2M 0.357 -> 0.307, 2.1M 0.654 -> 0.531 (node order), 0.698 -> 0.601 (query order), 8.4M 1.18 -> 0.98.
+// inter-object front). KEEP up to half a million triangles is bound by the length of its dependent rounds,
+// and one resident set of workgroups (1536 of 256 threads; 1024 start sooner on the smallest) has the
+// fewest; above by throughput, where small workgroups leave the tail early. KEEP and narrow phase, us,
+// 1024 x 256 / 1536 x 256 / 16384 x 128 threads: 216k triangles 59 / 59 / -, 272k 70 / 70 / 83, 498k 97 / 96 /
+// 102 (8192 x 128), 625k 296 / 288 / 281, 2.1M 845 / 865 / 829 (two entries in flight per thread).
 // The narrow phase: 4096 x 256 -> 16384 x 256 from a million triangles on, 2.1M 0.253 -> 0.235,
 // 8.4M 0.341 -> 0.311; below it is the same within 0.5 us from 1024 workgroups on.
 static unsigned default_shape(int kernel, int64_t n) {
     switch (kernel) {
-        case TK_KEEP: return n <= (1 << 18) ? make_shape(1024u, 2u) : make_shape(16384u, 2u, n <= (1 << 22) ? 2u : 8u);
+        case TK_KEEP:
+            return n <= (1 << 19) ? make_shape(n <= (1 << 17) ? 1024u : 1536u, 2u)
+                                  : make_shape(16384u, 2u, n <= (1 << 22) ? 2u : 8u);
         case TK_NARROW: return make_shape(n <= (1 << 19) ? 1024u : n <= (1 << 20) ? 4096u : 16384u, 1u);
         default: return 0xFFFFFFu;  // batched traversal: one group of queries per wave
     }
