@@ -15,6 +15,7 @@ namespace bvhcd {
 constexpr int kPairSegs = 64;   // pair-list segments (one append counter each)
 constexpr int kCntStride = 32;  // words between two segment counters (128 bytes)
 constexpr int kVisitWord = 4;   // words 4, 5 of a broad-phase segment's counter block: node tests
+constexpr int kOpenWord = 6;    // word 6 there: KEEP entries that the grid records left open
 constexpr int kDroppedWord = 2; // word of a list's counter block: entries no segment had room for
 
 // ------------------------------------------------------------------ node records (HBM layout)
@@ -362,6 +363,7 @@ enum Counter : int {
     C_FREQ_I = 13,     // capacity the last produced internal / external front needed
     C_FREQ_E = 14,
     // words 16..23 hold 64-bit counters (see Counter64)
+    C_KEEP_OPEN = 24,  // entries that the last KEEP's grid records left open
     C_NO_IMPLICIT = 25,// the last refit cannot vouch for shared-vertex pairs: a vertex coordinate
                        // above 1e8 in magnitude (or NaN / inf), or boxes given by the caller
     C_BADFACE = 26,    // set_topology: a face vertex id outside its vertex range
@@ -392,6 +394,10 @@ __device__ inline unsigned long long* visit_word(const DevState& d, uint32_t g) 
 // implicit pairs, node tests); lane g of one wave of 64 threads.
 __device__ inline void zero_step_counters(const DevState& d, int g) {
     *visit_word(d, g) = 0ull;
+    uint32_t open = d.pcnt[g * kCntStride + kOpenWord];
+    d.pcnt[g * kCntStride + kOpenWord] = 0u;
+    for (int off = 32; off > 0; off >>= 1) open += __shfl_xor(open, off);
+    if (g == 0) d.ctr[C_KEEP_OPEN] = open;
     d.pcnt[g * kCntStride] = 0u;                // broad-phase segment counters
     d.pcnt[(kPairSegs + g) * kCntStride] = 0u;  // narrow-phase segment counters
     if (g == 0) {

@@ -327,6 +327,7 @@ __device__ inline Out make_out(StagesT<CAP>& st, const FrontSink& fi, const Fron
     return o;
 }
 
+constexpr uint32_t kOpenSample = 16;
 __device__ inline bool node_overlap(const DevState& d, int32_t nd, const Box& q) {
     const float4 lo = d.inode[nd].lo, hi = d.inode[nd].hi;
     return box_overlap(q, lo, hi);
@@ -1771,15 +1772,19 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
 // whatever the load's width, so a box in two 16-byte loads costs 130 of the 215 cycles that 64 entries
 // take (74 % of the L1's cycles busy, 40 % of the VALU's). On large scenes (Q) the entries are therefore
 // tested on 16-byte records, one load each, and the few that those leave open (0.2 %), like the descents,
-// on the boxes. KEEP, us, boxes -> Q: 1.2M triangles 267..428 -> 242..355 over ten frames of a front, 2.1M
-// 414..638 -> 363..583, 8.4M 1170 -> 1033; the refit that writes the records takes 9 us (2.1M) and 67 us
+// on the boxes. Scenes whose coordinates coincide exactly, such as sheets of one grid on one another,
+// leave many open: where the last KEEP's records left more than one entry in 64 open (counted by one
+// workgroup in kOpenSample), this kernel ends at once and the one without Q that is launched after it
+// (otherwise) does the work; the count is handed on until a step without KEEP clears it. (Both loops in
+// one kernel: 8 % slower.) KEEP, us, boxes -> Q: 2.1M triangles 432..646 -> 365..596 over ten frames of a front, sheets of
+// 2.9M 375 -> 265, of 8.4M 1150 -> 1033 (without shared-vertex pairs) and 937 -> 745; the refit that writes the records takes 9 us (2.1M) and 67 us
 // (8.4M) longer. Below a million triangles the gain is within that cost.
 // implicit: the current front's shared-vertex head (C_ADJ entries after the last partition) is
 // not tested when the last refit found every coordinate finite: its pairs are broad-phase hits
 // whatever the positions (both boxes hold the shared vertex) and are counted, not listed.
 // W = waves per workgroup (the tuner picks it with the grid and U).
 template <int U, int W, bool Q>
-__global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int implicit) {
+__global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int implicit, int otherwise) {
     __shared__ StagesBPT<W> st;
     __shared__ DescStack<W> ds;
     stages_init(st);
@@ -1792,11 +1797,18 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
     // with skip_adj the head's pairs are filtered out anyway: skipped and not counted
     const uint32_t head = implicit ? min(d.ctr[C_ADJ], ne) : 0u;
     const uint32_t skip = d.skip_adj || d.ctr[C_NO_IMPLICIT] == 0u ? head : 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) d.ctr[C_IMPLICIT] = d.skip_adj ? 0u : skip;
     ne -= skip;
     const uint32_t total = ni + ne;
+    if (Q || otherwise) {  // the boxes at once: see below
+        const uint32_t open = d.ctr[C_KEEP_OPEN];
+        const bool boxes = open > total / (64u * kOpenSample);
+        if (Q && boxes && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(d.pcnt + kOpenWord, open);
+        if (Q == boxes) return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) d.ctr[C_IMPLICIT] = d.skip_adj ? 0u : skip;
     const uint32_t* ext_node = in.node[1] + skip;
     const int32_t* ext_query = in.query[1] + skip;
+    uint32_t opened = 0;
     const XcdLoop it = xcd_loop(total);
     const uint32_t stride = it.stride;
     if (it.begin - threadIdx.x >= it.end) return;  // the whole workgroup lies past the end
@@ -1861,6 +1873,7 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
                 bool open;
                 hit = q[u] >= 0 && !q_apart(qa[u], na[u], open);
                 const bool later = hit && open;
+                opened += later ? 1u : 0u;
                 if (!desc_push(stk, stop, later, q[u], nd[u] << 1 | (internal ? 0 : 1))) {  // no room: here
                     const NodeRec *a = &d.qleaf[q[u]], *b = internal ? &d.inode[nd[u]] : &d.leaf[nd[u]];
                     hit = box_overlap(rec_box(a->lo, a->hi), b->lo, b->hi);
@@ -1897,6 +1910,11 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
         if (last) break;
     }
     out.pair_final();
+    if (Q && blockIdx.x / kXcds % kOpenSample == 0) {
+        for (int off = 32; off > 0; off >>= 1) opened += __shfl_xor(opened, off);
+        if (lane_id() == 0 && opened)
+            atomicAdd(d.pcnt + (blockIdx.x * W + w) % kPairSegs * kCntStride + kOpenWord, opened);
+    }
     add_visits(d, visits);
 }
 
@@ -1995,8 +2013,8 @@ void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
     const FrontIn in = cur_front(d);
     const bool q = !d.inter && d.qnode && n >= kQFrom;
 #define BVHCD_KEEP(U, W)                                                                             \
-    if (q) hipLaunchKernelGGL((k_keep<U, W, true>), dim3(g), dim3(64 * W), 0, s, d, in, implicit);   \
-    else hipLaunchKernelGGL((k_keep<U, W, false>), dim3(g), dim3(64 * W), 0, s, d, in, implicit)
+    if (q) hipLaunchKernelGGL((k_keep<U, W, true>), dim3(g), dim3(64 * W), 0, s, d, in, implicit, 0); \
+    else hipLaunchKernelGGL((k_keep<U, W, false>), dim3(g), dim3(64 * W), 0, s, d, in, implicit, 0)
     switch (shape_unroll(sh) * 16 + w) {
         case 4 * 16 + 8: BVHCD_KEEP(4, 8); break;
         case 4 * 16 + 2: BVHCD_KEEP(4, 2); break;
@@ -2009,6 +2027,8 @@ void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
         default: BVHCD_KEEP(1, 4); break;
     }
 #undef BVHCD_KEEP
+    // one resident set of workgroups: it mostly ends at once
+    if (q) hipLaunchKernelGGL((k_keep<2, 4, false>), dim3(1536), dim3(256), 0, s, d, in, implicit, 1);
 }
 
 // ---------------------------------------------------------------- incremental front restructure
@@ -2109,7 +2129,7 @@ void launch_front_restr_apply(DevState& d, int32_t n, uint32_t ntasks, hipStream
     FrontIn kept = cur_front(d);
     kept.size[0] = d.ctr + C_KEPT_I;
     kept.size[1] = d.ctr + C_KEPT_E;
-    hipLaunchKernelGGL((k_keep<1, kWaves, false>), dim3(stream_grid()), dim3(kBlock), 0, s, d, kept, 0);
+    hipLaunchKernelGGL((k_keep<1, kWaves, false>), dim3(stream_grid()), dim3(kBlock), 0, s, d, kept, 0, 0);
     // the walks write segments into the spare buffers, then append after the kept entries
     front_begin(d, s);
     FrontSink fi = next_sink(d, 0), fe = next_sink(d, 1);

@@ -879,3 +879,23 @@ def test_keep_on_grid_records_equals_boxes(pkg, state):
         ctx.step(pkg.BVH_NONE, pkg.FRONT_GENERATE)
         assert keep == ctx.digest(False), k
     ctx.close()
+
+
+def test_keep_of_coinciding_coordinates(pkg):
+    """Sheets of one grid on one another (2^20 triangles and more): the grid records leave so many entries
+    open that the following KEEPs test the boxes at once. Every frame's pairs, with a REORDER and an
+    UPDATE between, are those of a pure traversal in another context."""
+    sc = pkg.Scene.preset("layers4", n=370)
+    print(f"[gpu] keep of coinciding coordinates, {sc.num_tris}", flush=True)
+    assert sc.num_tris >= 1 << 20
+    ctx, ref = _ctx(pkg, sc, narrow_phase=False), _ctx(pkg, sc, narrow_phase=False)
+    ops = [pkg.FRONT_GENERATE, pkg.FRONT_KEEP, pkg.FRONT_KEEP, pkg.FRONT_KEEP, pkg.FRONT_REORDER, pkg.FRONT_KEEP,
+           pkg.FRONT_UPDATE, pkg.FRONT_KEEP, pkg.FRONT_KEEP]
+    for k, op in enumerate(ops):
+        v = sc.frame(sc.frames - len(ops) + k)
+        for c, o in ((ctx, op), (ref, pkg.FRONT_PURE_BVH_CD)):
+            c.update_vertices(v)
+            c.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, o)
+        assert ctx.digest(False) == ref.digest(False), (k, op)
+    ctx.close()
+    ref.close()
