@@ -327,7 +327,7 @@ __device__ inline Out make_out(StagesT<CAP>& st, const FrontSink& fi, const Fron
     return o;
 }
 
-constexpr uint32_t kOpenSample = 16;
+constexpr uint32_t kOpenSample = 16, kOpenMost = 20;
 __device__ inline bool node_overlap(const DevState& d, int32_t nd, const Box& q) {
     const float4 lo = d.inode[nd].lo, hi = d.inode[nd].hi;
     return box_overlap(q, lo, hi);
@@ -1771,10 +1771,12 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
 // together. Bound by the vector L1: a wave's load of 64 different records takes 65 cycles of its CU
 // whatever the load's width, so a box in two 16-byte loads costs 130 of the 215 cycles that 64 entries
 // take (74 % of the L1's cycles busy, 40 % of the VALU's). On large scenes (Q) the entries are therefore
-// tested on 16-byte records, one load each, and the few that those leave open (0.2 %), like the descents,
+// tested on 16-byte records, one load each, and the few that those leave open (0.2 %
+// on scenes in motion), like the descents,
 // on the boxes. Scenes whose coordinates coincide exactly, such as sheets of one grid on one another,
-// leave many open: where the last KEEP's records left more than one entry in 64 open (counted by one
-// workgroup in kOpenSample), this kernel ends at once and the one without Q that is launched after it
+// leave many open: where the last KEEP's records left more than one entry in kOpenMost open (counted by one
+// workgroup in kOpenSample; 2.8 % open: 545 us against 650 on the boxes, 4.4 %: 253 / 240, 11 %: 1400 /
+// 1107), this kernel ends at once and the one without Q that is launched after it
 // (otherwise) does the work; the count is handed on until a step without KEEP clears it. (Both loops in
 // one kernel: 8 % slower.) KEEP, us, boxes -> Q: 2.1M triangles 432..646 -> 365..596 over ten frames of a front, sheets of
 // 2.9M 375 -> 265, of 8.4M 1150 -> 1033 (without shared-vertex pairs) and 937 -> 745; the refit that writes the records takes 9 us (2.1M) and 67 us
@@ -1801,7 +1803,7 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
     const uint32_t total = ni + ne;
     if (Q || otherwise) {  // the boxes at once: see below
         const uint32_t open = d.ctr[C_KEEP_OPEN];
-        const bool boxes = open > total / (64u * kOpenSample);
+        const bool boxes = open > total / (kOpenMost * kOpenSample);
         if (Q && boxes && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(d.pcnt + kOpenWord, open);
         if (Q == boxes) return;
     }
