@@ -885,7 +885,7 @@ int bvhcd_set_topology(bvhcd_ctx* c, const int32_t* faces, int64_t T, int64_t V,
     c->T = T;
     c->V = V;
     c->built = c->front_valid = c->restr_pending = c->learned_frame = c->repair_pending = false;
-    c->hres_valid = false;
+    c->hres_valid = c->totals_pending = false;
     c->keep_base = -1.0;
     c->keep_excess = 0.0;
     c->rebuild_ms = -1.0;
@@ -894,7 +894,9 @@ int bvhcd_set_topology(bvhcd_ctx* c, const int32_t* faces, int64_t T, int64_t V,
     c->frame = 0;
     c->d.fcur[0] = c->d.fcur[1] = 0;
     HIPCHK(c, hipMemsetAsync(c->d.fsize, 0, 4 * sizeof(uint32_t), c->stream));
+    // no pairs until the next step: the totals, and the segment counters that they are summed from
     HIPCHK(c, hipMemsetAsync(c->d.ctr, 0, 32 * sizeof(uint32_t), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->d.pcnt, 0, 2 * kPairSegs * kCntStride * sizeof(uint32_t), c->stream));
     // the learned schedule's decision buffers are sized here, not on its first decision frame
     if (c->learned && c->cfg.scheduler == BVHCD_SCHED_LEARNED && learned_reserve(c->learned, (int32_t)T))
         return fail(c, BVHCD_E_OOM, "learned decision buffers");
