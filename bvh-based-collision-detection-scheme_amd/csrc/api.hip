@@ -333,11 +333,15 @@ void ensure_totals(bvhcd_ctx* c) {
     c->totals_pending = false;
 }
 
-// The last step's totals and overflow flags in d.hres: one launch and one synchronisation, nothing
-// when they are there already.
-int read_totals(bvhcd_ctx* c) {
+// The last step's totals and overflow flags in d.hres: one launch (which `launch` makes) and one
+// synchronisation, nothing when they are there already. A launch that fails leaves an error, if the
+// caller's thread had none before.
+template <class Launch>
+int read_totals(bvhcd_ctx* c, Launch launch) {
     if (c->hres_valid) return BVHCD_OK;
-    launch_pair_totals(c->d, c->stream, c->cfg.narrow_phase != 0);
+    const bool clean = hipPeekAtLastError() == hipSuccess;
+    launch();
+    if (clean) HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->totals_pending = false;
     c->hres_valid = true;
@@ -1049,14 +1053,11 @@ int bvhcd_get_pairs(bvhcd_ctx* c, int32_t* out, int64_t cap, int64_t* num, int w
     const int kind = filtered ? 1 : 0;
     // into a device buffer: totals and pairs in one launch, one synchronisation for both
     const bool fused = where == BVHCD_MEM_DEVICE && out && cap > 0 && !c->hres_valid;
-    if (fused)
-        launch_totals_and_gather(c->d, kind, reinterpret_cast<int2*>(out), cap, c->cfg.narrow_phase != 0, c->stream);
-    if (fused) {
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        c->totals_pending = false;
-        c->hres_valid = true;
-    }
-    int st = read_totals(c);
+    const bool narrow = c->cfg.narrow_phase != 0;
+    int st = read_totals(c, [&]() {
+        if (fused) launch_totals_and_gather(c->d, kind, reinterpret_cast<int2*>(out), cap, narrow, c->stream);
+        else launch_pair_totals(c->d, c->stream, narrow);
+    });
     if (st) return st;
     const volatile uint32_t* res = c->d.hres;
     const uint32_t cnt = res[kind ? H_NP : H_BP];

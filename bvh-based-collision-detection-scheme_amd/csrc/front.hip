@@ -2368,6 +2368,7 @@ void launch_pair_gather(DevState& d, int kind, int2* dst, int64_t first, int64_t
                        (uint64_t)first, (uint64_t)count, 0);
 }
 void launch_totals_and_gather(DevState& d, int kind, int2* dst, int64_t cap, bool narrow, hipStream_t s) {
+    cap = std::min(cap, d.pair_cap + d.front_cap[1]);  // as many pairs as there can be: the grid follows it
     hipLaunchKernelGGL(k_pair_gather<true>, dim3(std::min(grid_for(cap), 2048u)), dim3(kBlock), 0, s, d, kind, dst,
                        (uint64_t)0, (uint64_t)cap, narrow ? 1 : 0);
 }

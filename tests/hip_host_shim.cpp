@@ -43,6 +43,7 @@ int hipGetDeviceCount(int* n) { return *n = 1, 0; }
 int hipGetDevice(int* d) { return *d = 0, 0; }
 int hipSetDevice(int) { return 0; }
 int hipGetLastError() { return 0; }
+int hipPeekAtLastError() { return 0; }
 const char* hipGetErrorString(int) { return "shim"; }
 int hipMemGetInfo(size_t* f, size_t* t) { return *f = *t = (size_t)64 << 30, 0; }
 int hipMalloc(void** p, size_t n) { return (*p = calloc(n, 1)) ? 0 : 2; }

@@ -58,3 +58,25 @@ def test_new_topology_starts_without_pairs(pkg, oracle, front, read, first):
         np.testing.assert_array_equal(oracle.pair_set(ctx.pairs(filtered)), oracle.pair_set(
             oracle.bruteforce_pairs(small.faces(), small.frame(0), filtered)))
     ctx.close()
+
+
+@pytest.mark.parametrize("cap", [1, (1 << 32) - 1, 1 << 32, 1 << 40, (1 << 40) + 256, (1 << 63) - 1])
+def test_device_read_out_takes_any_capacity(pkg, oracle, cap):
+    """The caller's capacity says how many pairs its buffer takes, not how many there are: every frame's
+    count and pairs are the frame's own whatever it is (the buffer here holds them all)."""
+    print(f"[gpu] device read-out with capacity {cap}", flush=True)
+    sc = pkg.Scene.preset("cloth256", n=40)
+    ctx = pkg.CollisionContext(sc.num_tris, sc.num_verts)
+    ctx.set_topology(sc.faces(), sc.num_verts)
+    for k, fr in enumerate((0, 290)):
+        v = sc.frame(fr)
+        ctx.update_vertices(v)
+        ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)
+        want = oracle.pair_set(oracle.bruteforce_pairs(sc.faces(), v, False))
+        buf = _device_buffer(len(want) + 64)
+        assert ctx.pairs_to_device(buf.data_ptr(), cap, filtered=False) == len(want)
+        got = buf.cpu().numpy()
+        if cap >= len(want):
+            np.testing.assert_array_equal(oracle.pair_set(got[: len(want)]), want)
+        assert (got[min(cap, len(want)):] == -1).all() and (got[: min(cap, len(want))] >= 0).all()
+    ctx.close()
