@@ -409,12 +409,14 @@ void frame_bytes(double T, double V, int bvh_op, int front_op, double visits, do
 // Host vertices of this size go through the pinned stages (bvhcd_update_vertices).
 bool staged_upload(const bvhcd_ctx* c) { return sizeof(float) * 3 * (size_t)c->V <= kStageBytes; }
 // Once kernels that read an own vertex buffer are enqueued, the next upload into that buffer on the
-// copy stream must wait for them, also when a later part of the step fails. (Staged uploads are
-// ordered by the context stream, and the size class only changes with the topology, whose call waits
-// for the stream.)
+// copy stream must wait for them, also when a later part of the step fails. (Uploads through a buffer's
+// stage are ordered by the context stream. A stage stays once it is there, and the size class only
+// changes with the topology, whose call waits for the stream; without a stage, small uploads go on the
+// copy stream too.)
 void mark_consumed(bvhcd_ctx* c) {
-    if (!staged_upload(c) && (c->d.verts == c->own_verts || c->d.verts == c->own_verts2))
-        (void)hipEventRecord(c->consumed[c->d.verts == c->own_verts2 ? 1 : 0], c->stream);
+    if (c->d.verts != c->own_verts && c->d.verts != c->own_verts2) return;
+    const int b = c->d.verts == c->own_verts2 ? 1 : 0;
+    if (!(staged_upload(c) && c->stage[b])) (void)hipEventRecord(c->consumed[b], c->stream);
 }
 
 // ---------------------------------------------------------------- BVH maintenance
@@ -832,6 +834,7 @@ int bvhcd_create(const bvhcd_config* cfg, bvhcd_ctx** out) {
     bool ok = st == 0 && hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking) == hipSuccess;
     for (int b = 0; b < 2 && ok; ++b) {
         ok &= hipEventCreateWithFlags(&c->copied[b], hipEventDisableTiming) == hipSuccess;
+        ok &= hipEventCreateWithFlags(&c->staged[b], hipEventDisableTiming) == hipSuccess;
         ok &= hipEventCreateWithFlags(&c->consumed[b], hipEventDisableTiming) == hipSuccess;
         ok &= ok && hipEventRecord(c->consumed[b], c->stream) == hipSuccess;
     }
@@ -927,8 +930,7 @@ int bvhcd_update_vertices(bvhcd_ctx* c, const float* xyz, int64_t V, int where) 
     const int b = c->vbuf ^ 1;
     float* dst = b ? c->own_verts2 : c->own_verts;
     if (staged_upload(c) && pinned(c->stage[b], std::min<size_t>(3 * (size_t)c->d.maxV, kStageBytes / sizeof(float)))) {
-        if (!c->staged[b]) HIPCHK(c, hipEventCreateWithFlags(&c->staged[b], hipEventDisableTiming));
-        else HIPCHK(c, hipEventSynchronize(c->staged[b]));
+        HIPCHK(c, hipEventSynchronize(c->staged[b]));
         std::memcpy(c->stage[b], xyz, sizeof(float) * 3 * V);
         HIPCHK(c, hipMemcpyAsync(dst, c->stage[b], sizeof(float) * 3 * V, hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipEventRecord(c->staged[b], c->stream));

@@ -1,0 +1,87 @@
+"""The order in which the host side queues its work, on the CPU: the library on a HIP runtime that notes
+the calls instead of running kernels (hip_host_shim.cpp), each case in a process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, re, sys
+shim = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+shim.shim_log.restype = ctypes.c_char_p
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from conftest import load_package
+pkg = load_package()
+def log():
+    return [l.split() for l in shim.shim_log().decode().splitlines()]
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("shim") / "hip_host_shim.so")
+    subprocess.run(["g++", "-std=c++20", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(HERE, "hip_host_shim.cpp")],
+                   check=True)
+    return so
+
+
+def run(shim, code, *args):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, shim, HERE, *map(str, args)], capture_output=True,
+                       text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+UPLOADS = """
+refused, V = sys.argv[3] == "refused", int(sys.argv[4])
+faces = np.arange(30, dtype=np.int32).reshape(-1, 3)
+if refused:  # the stages' size
+    shim.shim_refuse_pinned(ctypes.c_size_t(12 * V))
+ctx = pkg.CollisionContext(10, V)
+ctx.set_topology(faces, V)
+dev = np.zeros((V, 3), np.float32)
+for k in range(8):
+    if k == 5:  # a device copy in between, into the buffer of the last upload
+        ctx.update_vertices(dev.ctypes.data, pkg.MEM_DEVICE)
+    else:
+        ctx.update_vertices(np.full((V, 3), k, np.float32))
+    ctx.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, pkg.FRONT_KEEP if k else pkg.FRONT_GENERATE)
+text = log()
+main = next(l[-1] for l in text if l[0] == "launch")
+# walk the log: what of the context's stream each copy onto another stream is known to follow
+launched, recorded, waited, read_at, uploads = 0, {}, {}, {}, 0
+current = None
+for l in text:
+    if l[0] == "launch" and l[-1] == main:
+        launched += 1
+        if current:
+            read_at[current] = launched  # the step's kernels read the current buffer
+    elif l[0] == "record":
+        recorded[l[1]] = (l[-1], launched)
+    elif l[0] == "wait":
+        st, at = recorded[l[1]]
+        if st == main:
+            waited[l[-1]] = max(waited.get(l[-1], 0), at)
+    elif l[0] == "copy" and launched >= 0 and l[1] in BUFFERS(text):
+        if l[-1] != main:
+            assert waited.get(l[-1], 0) >= read_at.get(l[1], 0), (l, waited, read_at)
+            uploads += 1
+        current = l[1]
+assert uploads == (0 if not refused and V < 87382 else 7), uploads
+"""
+
+
+@pytest.mark.parametrize("V", [30, 87381, 87382])
+@pytest.mark.parametrize("pinned", ["there", "refused"])
+def test_uploads_follow_the_steps_that_read_their_buffer(shim, pinned, V):
+    """Host vertices up to 1 MB go through a pinned stage on the context's stream, larger ones and those
+    whose stage cannot be had on the copy stream: there every upload has waited for the kernels of the
+    last step that read its buffer."""
+    run(shim, """
+def BUFFERS(text):  # the two vertex buffers: the targets of the eight updates
+    seen = [l[1] for l in text if l[0] == "copy"]
+    return {x for x in seen if seen.count(x) >= 3}
+""" + UPLOADS, pinned, V)
