@@ -427,16 +427,7 @@ int do_build(bvhcd_ctx* c) {
     launch_box_and_codes(d, n, d.codes, d.prim_idx, s);
     radix_sort_u32(d, d.codes, d.prim_idx, d.keys_tmp, d.vals_tmp, n, 30, s);
     launch_leaf_setup(d, n, s);
-    if (n >= 2) {
-        launch_emit_full(d, n, s);
-    } else {
-        // single leaf: no internal nodes; lca = {leaf 0, end}
-        const int32_t lca[2] = {1, -1};
-        HIPCHK(c, hipMemcpyAsync(d.leaf_lca, lca, sizeof(lca), hipMemcpyHostToDevice, s));
-        HIPCHK(c, hipStreamSynchronize(s));
-        HIPCHK(c, hipMemsetAsync(d.leaf_par, 0xff, sizeof(int32_t), s));
-        fill_u32(d.leaf_mark, 1, 3u, s);
-    }
+    if (n >= 2) launch_emit_full(d, n, s);  // else the single leaf is the tree (launch_leaf_setup)
     launch_refit_prep(d, n, s);
     return BVHCD_OK;
 }

@@ -1611,7 +1611,8 @@ __global__ void __launch_bounds__(kBlock) k_update(DevState d, FrontIn in, Front
         bool ext = valid && !internal && hit;
         bool pair = ext;
         if (out.skip_adj && pair) pair = !faces_share_vertex(out.lfaces, q, x);
-        if (valid && !internal && !hit) {
+        if (valid && !internal && !hit && node < 0) ext = true;  // the only leaf: the root's entry stays
+        else if (valid && !internal && !hit) {
             const bool right = (d.leaf_mark[x] & 4u) != 0u;
             const int4 pt = d.itopo[node];
             ++visits;

@@ -1694,8 +1694,9 @@ void launch_refit(DevState& d, int32_t n, hipStream_t s, bool zero_step_counters
 
 // ======================================================================= prim map / misc
 // After a sort: the inverse permutation; the faces gathered into leaf order, so that refit and the
-// narrow phase read them sequentially instead of gathering by triangle id every frame; and the start
-// values of the emission and the refit preparation that follow.
+// narrow phase read them sequentially instead of gathering by triangle id every frame; the start
+// values of the emission and the refit preparation that follow; and the tree of a single leaf, which has
+// no emission: no parent, nothing after it (an inter-object front walks and prunes such a tree too).
 __global__ void __launch_bounds__(kBlock) k_leaf_setup(int32_t n, int32_t chunks, DevState d) {
     const int32_t x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= n) return;
@@ -1711,6 +1712,13 @@ __global__ void __launch_bounds__(kBlock) k_leaf_setup(int32_t n, int32_t chunks
         *d.rp_tcount = 0u;
         *d.rp_tdone = 0u;
         *d.rp_tdeep = 0u;
+        if (n == 1) {
+            d.leaf[0].lo.w = d.leaf[0].hi.w = i2f(-1);
+            d.leaf_par[0] = -1;
+            d.leaf_mark[0] = 3u;
+            d.leaf_lca[0] = 1;
+            d.leaf_lca[1] = -1;
+        }
         if (d.qgrid) {  // the first refit's grid
             const float* b = d.scene_box;
             q_grid(d.qgrid + 8 * d.qpar, Box{b[0], b[1], b[2], b[3], b[4], b[5]});

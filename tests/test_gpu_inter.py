@@ -108,3 +108,47 @@ def test_inter_front_full_cloth(pkg, oracle):
     assert len(inter.pairs(False)) > 0
     inter.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("before", [0, 40])
+def test_inter_front_on_one_triangle(pkg, oracle, before):
+    """A queried context of a single triangle (fresh, or after a larger mesh): the tree is one leaf with no
+    parent and nothing after it. Every query's front is that leaf, whatever the step, and the pairs are
+    those of the boxes and of the oracle's pair test on both meshes together."""
+    print(f"[gpu] inter front on one triangle, {before} before", flush=True)
+    rng = np.random.default_rng(5)
+    one = np.array([[0, 0, 0], [1, 0, 0.1], [0, 1, 0]], np.float32)
+    Tb = 300
+    fb = np.arange(3 * Tb, dtype=np.int32).reshape(-1, 3)
+    ctx = pkg.CollisionContext(max(before, 1), 3 * max(before, 1))
+    if before:
+        f = np.arange(3 * before, dtype=np.int32).reshape(-1, 3)
+        ctx.set_topology(f, 3 * before)
+        ctx.update_vertices(rng.random((3 * before, 3)).astype(np.float32))
+        ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)
+    ctx.set_topology(np.array([[0, 1, 2]], np.int32), 3)
+    inter = pkg.InterFront(ctx, Tb, 3 * Tb, int_front_cap=4096, ext_front_cap=4096, pair_cap=4096)
+    inter.set_topology(fb, 3 * Tb)
+    both = np.concatenate([[[0, 1, 2]], fb + 3]).astype(np.int32)
+    for k, op in enumerate([pkg.FRONT_GENERATE, pkg.FRONT_KEEP, pkg.FRONT_UPDATE, pkg.FRONT_REORDER,
+                            pkg.FRONT_UPDATE, pkg.FRONT_PURE_BVH_CD, pkg.FRONT_KEEP]):
+        c = rng.random((Tb, 1, 3)) * 2.0 - 0.5 + 0.3 * k
+        vb = (c + 0.4 * rng.random((Tb, 3, 3))).reshape(-1, 3).astype(np.float32)
+        ctx.update_vertices(one)
+        ctx.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, pkg.FRONT_KEEP if k else pkg.FRONT_GENERATE)
+        inter.update_vertices(vb)
+        inter.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, op)
+        for filtered in (False, True):
+            want = oracle.bruteforce_pairs(both, np.concatenate([one, vb]), filtered).reshape(-1, 2)
+            want = np.sort(want, 1)
+            want = want[want[:, 0] == 0][:, 1] - 1
+            got = inter.pairs(filtered)
+            assert (got[:, 0] == 0).all()
+            np.testing.assert_array_equal(np.sort(got[:, 1]), np.sort(want), err_msg=f"{k} {filtered}")
+        if k == 0:
+            assert len(want) > 0
+        if op != pkg.FRONT_PURE_BVH_CD:
+            assert len(inter.export_front(0)) == 0
+            np.testing.assert_array_equal(_rows(inter.export_front(1)), [[q, 0] for q in range(Tb)])
+    inter.close()
+    ctx.close()
