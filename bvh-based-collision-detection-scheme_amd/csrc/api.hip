@@ -605,7 +605,7 @@ int run_front(bvhcd_ctx* c, int& front_op) {
             break;
         case BVHCD_FRONT_REORDER:
             begin(c, S_FRONT);
-            launch_reorder(d, n, s);
+            launch_reorder(d, n, s, c->step_zeroed);
             end(c, S_FRONT);
             break;
         case BVHCD_FRONT_KEEP:

@@ -2146,8 +2146,8 @@ void launch_front_restr_apply(DevState& d, int32_t n, uint32_t ntasks, hipStream
 // with each bucket's non-overlapping entries first. Its bucket starts go to scratch (`cursor`):
 // intbeg keeps the last ordering's offsets, which the quality check reads (the front need not
 // have been node-ordered since: an incremental restructure appends entries).
-void launch_reorder(DevState& d, int32_t n, hipStream_t s) {
-    launch_keep(d, n, s);
+void launch_reorder(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
+    launch_keep(d, n, s, counters_zeroed);
     if (n < 2) return;
     order_front(d, 0, n - 1, d.intcnt, d.cursor, true, s);
 }

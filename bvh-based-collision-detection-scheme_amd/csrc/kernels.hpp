@@ -79,7 +79,7 @@ int64_t max_walk_waves(int64_t T);  // producing waves of a GENERATE over up to 
 void launch_generate(DevState& d, int32_t n, hipStream_t s, bool order = true);  // traversal + ordering
 void launch_update(DevState& d, int32_t n, int quality, hipStream_t s, bool order = true);
 void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed = false);
-void launch_reorder(DevState& d, int32_t n, hipStream_t s);
+void launch_reorder(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed = false);
 // Incremental front restructure: classify the current fronts against the runs in rt_of_leaf
 // (old topology; kept entries to the other buffers, walks to d.rtasks with their count in
 // ctr[C_TASKS]), then, after the rebuild, pairs of the kept entries plus the walks.

@@ -85,3 +85,20 @@ def BUFFERS(text):  # the two vertex buffers: the targets of the eight updates
     seen = [l[1] for l in text if l[0] == "copy"]
     return {x for x in seen if seen.count(x) >= 3}
 """ + UPLOADS, pinned, V)
+
+
+def test_counters_are_cleared_once_a_step(shim):
+    """A refit clears the step's counters for the KEEP or REORDER that follows it: cleared twice, what the
+    last KEEP's records left open would be lost on the way."""
+    run(shim, """
+ctx = pkg.CollisionContext(100, 300)
+ctx.set_topology(np.arange(300, dtype=np.int32).reshape(-1, 3), 300)
+v = np.zeros((300, 3), np.float32)
+for k, (bvh, front, resets) in enumerate([(pkg.BVH_BUILD, pkg.FRONT_GENERATE, 1), (pkg.BVH_REFIT, pkg.FRONT_KEEP, 0),
+                                          (pkg.BVH_REFIT, pkg.FRONT_REORDER, 0), (pkg.BVH_NONE, pkg.FRONT_REORDER, 1),
+                                          (pkg.BVH_NONE, pkg.FRONT_KEEP, 1)]):
+    shim.shim_clear()
+    ctx.update_vertices(v)
+    ctx.step(bvh, front)
+    assert sum("k_reset_step" in l[1] for l in log()) == resets, (k, log())
+""")
