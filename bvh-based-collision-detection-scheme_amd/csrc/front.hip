@@ -653,6 +653,7 @@ unsigned tuned_shape(int kernel, int64_t n, int64_t queries) {
     const unsigned g = g_grid[kernel][size_class(n)];
     return g ? g : default_shape(kernel, queries ? queries : n);
 }
+bool shape_set(int kernel, int64_t n) { return g_grid[kernel][size_class(n)] != 0; }
 void set_tuned_shape(int kernel, int64_t n, unsigned sh) { g_grid[kernel][size_class(n)] = sh; }
 void record_tuning(int kernel, int64_t n, unsigned sh, float ms) {
     g_trials.push_back({kernel, size_class(n), sh, ms});
@@ -2007,17 +2008,11 @@ void launch_adj_partition(DevState& d, int32_t n, hipStream_t s) {
     d.adj_version = d.front_version;
 }
 
-void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
-    // inter-object fronts pair triangles of two objects: no shared vertices, no partition
-    const int implicit = d.inter ? 0 : 1;
-    if (implicit && d.adj_version != d.front_version) launch_adj_partition(d, n, s);
-    if (!counters_zeroed) reset_step_counters(d, s);
-    const unsigned sh = tuned_shape(TK_KEEP, n, d.inter ? d.nq : 0), g = shape_grid(sh), w = shape_waves(sh);
-    const FrontIn in = cur_front(d);
-    const bool q = !d.inter && d.qnode && n >= kQFrom;
-#define BVHCD_KEEP(U, W)                                                                             \
-    if (q) hipLaunchKernelGGL((k_keep<U, W, true>), dim3(g), dim3(64 * W), 0, s, d, in, implicit, 0); \
-    else hipLaunchKernelGGL((k_keep<U, W, false>), dim3(g), dim3(64 * W), 0, s, d, in, implicit, 0)
+// sh: a launch shape (make_shape); the shapes' unrolls and workgroup sizes are all instantiated.
+template <bool Q>
+static void keep_in_shape(unsigned sh, const DevState& d, const FrontIn& in, int implicit, int otherwise, hipStream_t s) {
+    const unsigned g = shape_grid(sh), w = shape_waves(sh);
+#define BVHCD_KEEP(U, W) hipLaunchKernelGGL((k_keep<U, W, Q>), dim3(g), dim3(64 * W), 0, s, d, in, implicit, otherwise)
     switch (shape_unroll(sh) * 16 + w) {
         case 4 * 16 + 8: BVHCD_KEEP(4, 8); break;
         case 4 * 16 + 2: BVHCD_KEEP(4, 2); break;
@@ -2030,8 +2025,24 @@ void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
         default: BVHCD_KEEP(1, 4); break;
     }
 #undef BVHCD_KEEP
-    // one resident set of workgroups: it mostly ends at once
-    if (q) hipLaunchKernelGGL((k_keep<2, 4, false>), dim3(1536), dim3(256), 0, s, d, in, implicit, 1);
+}
+
+void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
+    // inter-object fronts pair triangles of two objects: no shared vertices, no partition
+    const int implicit = d.inter ? 0 : 1;
+    if (implicit && d.adj_version != d.front_version) launch_adj_partition(d, n, s);
+    if (!counters_zeroed) reset_step_counters(d, s);
+    const unsigned sh = tuned_shape(TK_KEEP, n, d.inter ? d.nq : 0);
+    const FrontIn in = cur_front(d);
+    if (!d.inter && d.qnode && n >= kQFrom) {
+        keep_in_shape<true>(sh, d, in, implicit, 0, s);
+        // The boxes, where the records left too much open: in the tuned shape too, so that tuning times the
+        // kernel that does the work and a shape that is set holds for both. Untuned, one resident set of
+        // workgroups: it mostly ends at once.
+        keep_in_shape<false>(shape_set(TK_KEEP, n) ? sh : make_shape(1536u, 2u), d, in, implicit, 1, s);
+    } else {
+        keep_in_shape<false>(sh, d, in, implicit, 0, s);
+    }
 }
 
 // ---------------------------------------------------------------- incremental front restructure

@@ -39,6 +39,7 @@ inline unsigned shape_unroll(unsigned sh) { return ((sh >> 24) & 15u) ? ((sh >> 
 inline unsigned shape_waves(unsigned sh) { return (sh >> 28) ? (sh >> 28) : 4u; }
 // The shape set for the size class of n, else the default for `queries` (0: n).
 unsigned tuned_shape(int kernel, int64_t n, int64_t queries = 0);
+bool shape_set(int kernel, int64_t n);
 void set_tuned_shape(int kernel, int64_t n, unsigned sh);
 void record_tuning(int kernel, int64_t n, unsigned sh, float ms);
 std::string tuning_report();

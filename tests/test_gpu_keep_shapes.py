@@ -1,0 +1,49 @@
+"""KEEP's launch shapes on scenes of 2^20 triangles and more, where it tests 16-byte grid records first."""
+import pytest
+
+from conftest import load_package
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(16384, 1, 128), (300, 1, 256), (4096, 1, 512), (16384, 2, 128), (1536, 2, 256), (777, 2, 512),
+          (64, 4, 128), (3001, 4, 256), (8192, 4, 512), (8, 4, 512)]
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    return load_package()
+
+
+@pytest.mark.parametrize("preset,n,skip_adjacent", [("cloth1024", 726, False), ("cloth1024", 726, True),
+                                                    ("layers4", 370, False)])
+def test_keep_launch_shapes_on_grid_records(pkg, preset, n, skip_adjacent):
+    """Every unroll and workgroup size, on a folded cloth (the records decide nearly every entry) and on
+    sheets of one grid on one another (they leave many open, the boxes are tested instead): the pairs of
+    a pure traversal in another context."""
+    sc = pkg.Scene.preset(preset, n=n)
+    print(f"[gpu] keep shapes on grid records: {preset} {sc.num_tris} skip {skip_adjacent}", flush=True)
+    assert sc.num_tris >= 1 << 20
+    ctx, ref = (pkg.CollisionContext(sc.num_tris, sc.num_verts, narrow_phase=False, skip_adjacent=skip_adjacent)
+                for _ in range(2))
+    frames = [sc.frame(sc.frames - 6 + k) for k in range(4)]
+    want = []
+    ref.set_topology(sc.faces(), sc.num_verts)
+    for v in frames:
+        ref.update_vertices(v)
+        ref.step(pkg.BVH_BUILD, pkg.FRONT_PURE_BVH_CD)
+        want.append(ref.digest(False))
+    assert len(set(want)) == len(want) and want[0][1] > 0
+    ref.close()
+    ctx.set_topology(sc.faces(), sc.num_verts)
+    ctx.update_vertices(frames[0])
+    ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)
+    try:
+        for k, shape in enumerate(SHAPES):
+            pkg.autotune_set(pkg.TUNE_KEEP, sc.num_tris, *shape)
+            for at in (1 + k % 3, 0):  # away from where the front was made, and back
+                ctx.update_vertices(frames[at])
+                ctx.step(pkg.BVH_REFIT, pkg.FRONT_KEEP)
+                assert ctx.digest(False) == want[at], (shape, at)
+    finally:
+        pkg.autotune_set(pkg.TUNE_KEEP, sc.num_tris, 16384, 2, 128)  # the size's default
+        ctx.close()

@@ -102,3 +102,25 @@ for k, (bvh, front, resets) in enumerate([(pkg.BVH_BUILD, pkg.FRONT_GENERATE, 1)
     ctx.step(bvh, front)
     assert sum("k_reset_step" in l[1] for l in log()) == resets, (k, log())
 """)
+
+
+@pytest.mark.parametrize("T", [200000, 1 << 20])
+def test_a_set_keep_shape_holds_for_every_keep_kernel(shim, T):
+    """autotune_set's grid, unroll and workgroup size reach the kernel that tests the grid records and the
+    one that tests the boxes instead (scenes of 2^20 triangles and more launch both)."""
+    run(shim, """
+T = int(sys.argv[3])
+ctx = pkg.CollisionContext(T, 3, int_front_cap=4096, ext_front_cap=4096, pair_cap=4096)
+ctx.set_topology(np.tile(np.array([[0, 1, 2]], np.int32), (T, 1)), 3)
+ctx.update_vertices(np.zeros((3, 3), np.float32))
+ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)
+ctx.step(pkg.BVH_REFIT, pkg.FRONT_KEEP)
+for grid, unroll, block in [(777, 4, 512), (64, 1, 128), (3000, 2, 256)]:
+    pkg.autotune_set(pkg.TUNE_KEEP, T, grid, unroll, block)
+    shim.shim_clear()
+    ctx.step(pkg.BVH_REFIT, pkg.FRONT_KEEP)
+    keeps = [l for l in log() if l[0] == "launch" and "6k_keepI" in l[1]]
+    assert len(keeps) == (2 if T >= 1 << 20 else 1)
+    for l in keeps:
+        assert "k_keepILi%dELi%dE" % (unroll, block // 64) in l[1] and l[3] == str(grid) and l[5] == str(block), keeps
+""", T)
