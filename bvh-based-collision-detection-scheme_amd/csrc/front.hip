@@ -637,7 +637,10 @@ int size_class(int64_t n) {
 // and one resident set of workgroups (1536 of 256 threads; 1024 start sooner on the smallest) has the
 // fewest; above by throughput, where small workgroups leave the tail early. KEEP and narrow phase, us,
 // 1024 x 256 / 1536 x 256 / 16384 x 128 threads: 216k triangles 59 / 59 / -, 272k 70 / 70 / 83, 498k 97 / 96 /
-// 102 (8192 x 128), 625k 296 / 288 / 281, 2.1M 845 / 865 / 829 (two entries in flight per thread).
+// 102 (8192 x 128), 625k 296 / 288 / 281, 2.1M 845 / 865 / 829 (two entries in flight per thread). From
+// 2^22 triangles on larger workgroups: 16384 of 128 / 256 / 512 threads, 8.4M sheets on the boxes 1273 /
+// 1204 / 1154, on the records (launch_keep) 803 / 735 / 793; 4.2M on the records 411 / 407 / 437, 2.1M
+// 446 / 508 / 636.
 // The narrow phase: 4096 x 256 -> 16384 x 256 from a million triangles on, 2.1M 0.253 -> 0.235,
 // 8.4M 0.341 -> 0.311; below it is the same within 0.5 us from 1024 workgroups on.
 static unsigned default_shape(int kernel, int64_t n) {
@@ -1777,10 +1780,11 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
 // on scenes in motion), like the descents,
 // on the boxes. Scenes whose coordinates coincide exactly, such as sheets of one grid on one another,
 // leave many open: where the last KEEP's records left more than one entry in kOpenMost open (counted by one
-// workgroup in kOpenSample; 2.8 % open: 545 us against 650 on the boxes, 4.4 %: 253 / 240, 11 %: 1400 /
-// 1107), this kernel ends at once and the one without Q that is launched after it
-// (otherwise) does the work; the count is handed on until a step without KEEP clears it. (Both loops in
-// one kernel: 8 % slower.) KEEP, us, boxes -> Q: 2.1M triangles 432..646 -> 365..596 over ten frames of a front, sheets of
+// workgroup in kOpenSample), this kernel ends at once and the one without Q that is launched after it
+// (otherwise) does the work; the count is handed on until a step without KEEP or REORDER clears it.
+// (Both loops in one kernel: 8 % slower.) Records / boxes, us: 3.9 % open 289 / 304 (sheets of 2.1M), 1073 / 1209 (of
+// 8.4M); 4.4 % 193 / 197 (cloth of 1.3M), 288 / 331 (of 2.1M); 4.6 % 297 / 305; 5.8 % 305 / 304; 6.3 %
+// 1179 / 1204; 7.6 % 322 / 301; 8.4 % 1244 / 1212; 13 % 388 / 318. KEEP, us, boxes -> Q: 2.1M triangles 432..646 -> 365..596 over ten frames of a front, sheets of
 // 2.9M 375 -> 265, of 8.4M 1150 -> 1033 (without shared-vertex pairs) and 937 -> 745; the refit that writes the records takes 9 us (2.1M) and 67 us
 // (8.4M) longer. Below a million triangles the gain is within that cost.
 // implicit: the current front's shared-vertex head (C_ADJ entries after the last partition) is
@@ -2035,11 +2039,13 @@ void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
     const unsigned sh = tuned_shape(TK_KEEP, n, d.inter ? d.nq : 0);
     const FrontIn in = cur_front(d);
     if (!d.inter && d.qnode && n >= kQFrom) {
-        keep_in_shape<true>(sh, d, in, implicit, 0, s);
+        const bool set = shape_set(TK_KEEP, n), large = n > 1 << 22;
+        keep_in_shape<true>(!set && large ? make_shape(16384u, 2u, 4u) : sh, d, in, implicit, 0, s);
         // The boxes, where the records left too much open: in the tuned shape too, so that tuning times the
-        // kernel that does the work and a shape that is set holds for both. Untuned, one resident set of
-        // workgroups: it mostly ends at once.
-        keep_in_shape<false>(shape_set(TK_KEEP, n) ? sh : make_shape(1536u, 2u), d, in, implicit, 1, s);
+        // kernel that does the work and a shape that is set holds for both. Untuned, up to 2^22 triangles
+        // one resident set of workgroups, as it mostly ends at once (8.4M sheets on the boxes 1281 us, and
+        // 1167 in the boxes' own shape, which costs 8 where the records do the work).
+        keep_in_shape<false>(set || large ? sh : make_shape(1536u, 2u), d, in, implicit, 1, s);
     } else {
         keep_in_shape<false>(sh, d, in, implicit, 0, s);
     }

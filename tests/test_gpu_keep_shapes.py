@@ -1,4 +1,5 @@
 """KEEP's launch shapes on scenes of 2^20 triangles and more, where it tests 16-byte grid records first."""
+import numpy as np
 import pytest
 
 from conftest import load_package
@@ -47,3 +48,26 @@ def test_keep_launch_shapes_on_grid_records(pkg, preset, n, skip_adjacent):
     finally:
         pkg.autotune_set(pkg.TUNE_KEEP, sc.num_tris, 16384, 2, 128)  # the size's default
         ctx.close()
+
+
+@pytest.mark.parametrize("jitter", [0.0, 0.02])
+def test_keep_default_shapes_of_large_scenes(pkg, jitter):
+    """More than 2^22 triangles, where the records and the boxes have shapes of their own: sheets of one grid
+    on one another (the boxes), and every vertex displaced by 2 % of an edge (the records)."""
+    sc = pkg.Scene.preset("layers4", n=726)
+    print(f"[gpu] keep default shapes: {sc.num_tris}, jitter {jitter}", flush=True)
+    assert sc.num_tris > 1 << 22
+    move = np.random.default_rng(1).standard_normal((sc.num_verts, 3)).astype(np.float32) * np.float32(jitter / 725)
+    ctx = pkg.CollisionContext(sc.num_tris, sc.num_verts, narrow_phase=False)
+    ctx.set_topology(sc.faces(), sc.num_verts)
+    got = []
+    frames = [sc.frame(sc.frames - 4 + k) + move for k in range(4)]
+    for k, v in enumerate(frames):
+        ctx.update_vertices(v)
+        ctx.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, pkg.FRONT_KEEP if k else pkg.FRONT_GENERATE)
+        got.append(ctx.digest(False))
+    for v, d in zip(frames, got):
+        ctx.update_vertices(v)
+        ctx.step(pkg.BVH_BUILD, pkg.FRONT_PURE_BVH_CD)
+        assert ctx.digest(False) == d and d[1] > sc.num_tris
+    ctx.close()
