@@ -1885,13 +1885,15 @@ __global__ void __launch_bounds__(64 * W) k_keep(DevState d, FrontIn in, int imp
                 if (!desc_push(stk, stop, later, q[u], nd[u] << 1 | (internal ? 0 : 1))) {  // no room: here
                     const NodeRec *a = &d.qleaf[q[u]], *b = internal ? &d.inode[nd[u]] : &d.leaf[nd[u]];
                     hit = box_overlap(rec_box(a->lo, a->hi), b->lo, b->hi);
+                    ++visits;
                 } else {
                     hit = hit && !open;
+                    visits += q[u] >= 0 && !later ? 1u : 0u;  // an open entry's is counted with its boxes
                 }
             } else {
                 hit = q[u] >= 0 && box_overlap(rec_box(qlo[u], qhi[u]), lo[u], hi[u]);
+                visits += q[u] >= 0 ? 1u : 0u;
             }
-            visits += q[u] >= 0 ? 1u : 0u;
             // the node now overlaps: its children go on the wave's stack
             const bool desc = internal && hit;
             int4 tp = make_int4(0, 0, 0, 0);

@@ -71,3 +71,24 @@ def test_keep_default_shapes_of_large_scenes(pkg, jitter):
         ctx.step(pkg.BVH_BUILD, pkg.FRONT_PURE_BVH_CD)
         assert ctx.digest(False) == d and d[1] > sc.num_tris
     ctx.close()
+
+
+def test_keep_counts_every_entry_once(pkg):
+    """Node tests of a KEEP: an entry that the grid records leave open counts once, like any other. On
+    coinciding sheets the first KEEP tests the records and the second the boxes at once, on the same
+    front and vertices: both report the same number."""
+    sc = pkg.Scene.preset("layers4", n=370)
+    print(f"[gpu] keep node tests, {sc.num_tris}", flush=True)
+    ctx = pkg.CollisionContext(sc.num_tris, sc.num_verts, narrow_phase=False)
+    ctx.set_topology(sc.faces(), sc.num_verts)
+    ctx.update_vertices(sc.frame(sc.frames - 2))
+    ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)
+    ctx.update_vertices(sc.frame(sc.frames - 1))
+    tests = []
+    for op in (pkg.BVH_REFIT, pkg.BVH_NONE, pkg.BVH_NONE):
+        ctx.step(op, pkg.FRONT_KEEP)
+        s = ctx.stats()
+        tests.append(s["node_visits"])
+    assert tests[0] == tests[1] == tests[2]
+    assert tests[0] >= s["int_front"] + s["ext_front"] - s["implicit_pairs"] > sc.num_tris
+    ctx.close()
