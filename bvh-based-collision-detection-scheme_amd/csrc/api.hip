@@ -1631,6 +1631,7 @@ int bvhcd_inter_create(bvhcd_ctx* def, const bvhcd_config* cfg, bvhcd_inter** ou
         delete x;
         return st;
     }
+    x->rigid->d.qnode = nullptr;  // its leaves are queries, tested on their boxes: no KEEP reads its records
     DevState& o = x->own;
     const int64_t Tq = cfg->max_tris, Td = def->d.maxT, lim = 0x7FFFFFFFll;
     int64_t ci = cfg->int_front_cap > 0 ? cfg->int_front_cap : 48 * Tq + (1 << 20);

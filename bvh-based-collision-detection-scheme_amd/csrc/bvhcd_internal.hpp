@@ -429,6 +429,11 @@ __device__ inline bool leaves_share_vertex(const DevState& d, int32_t a, int32_t
     return faces_share_vertex(d.lfaces, a, b);
 }
 
+// Does KEEP of a scene of n triangles test the 16-byte records first (so that refits write them).
+__host__ __device__ inline bool keeps_on_records(const DevState& d, int32_t n) {
+    return !d.inter && d.qnode && n >= kQFrom;
+}
+
 constexpr uint32_t kCutCap = 512;
 constexpr int kSceneParts = 1024;
 // Launch helpers

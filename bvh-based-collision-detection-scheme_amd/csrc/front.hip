@@ -2040,7 +2040,7 @@ void launch_keep(DevState& d, int32_t n, hipStream_t s, bool counters_zeroed) {
     if (!counters_zeroed) reset_step_counters(d, s);
     const unsigned sh = tuned_shape(TK_KEEP, n, d.inter ? d.nq : 0);
     const FrontIn in = cur_front(d);
-    if (!d.inter && d.qnode && n >= kQFrom) {
+    if (keeps_on_records(d, n)) {
         const bool set = shape_set(TK_KEEP, n), large = n > 1 << 22;
         keep_in_shape<true>(!set && large ? make_shape(16384u, 2u, 4u) : sh, d, in, implicit, 0, s);
         // The boxes, where the records left too much open: in the tuned shape too, so that tuning times the

@@ -1684,10 +1684,17 @@ __global__ void __launch_bounds__(kTopBlock) k_refit_top(DevState d, int32_t chu
     if (threadIdx.x == 0) *d.rp_tdone = 0;
 }
 
+// The 16-byte records are written for scenes whose KEEP reads them: in a context of 2^21 triangles they took
+// the refit of 41k 18.9 us instead of 16.8, of 718k 49.4 instead of 40.4.
 void launch_refit(DevState& d, int32_t n, hipStream_t s, bool zero_step_counters) {
     if (n < 1) return;
-    hipLaunchKernelGGL(k_refit, dim3(refit_chunks(n)), dim3(kRefitBlock), 0, s, n, d);
-    hipLaunchKernelGGL(k_refit_top, dim3(kTopGrid), dim3(kTopBlock), 0, s, d, refit_chunks(n),
+    DevState v = d;
+    if (!keeps_on_records(d, n)) {
+        v.qnode = nullptr;
+        v.qleafrec = nullptr;
+    }
+    hipLaunchKernelGGL(k_refit, dim3(refit_chunks(n)), dim3(kRefitBlock), 0, s, n, v);
+    hipLaunchKernelGGL(k_refit_top, dim3(kTopGrid), dim3(kTopBlock), 0, s, v, refit_chunks(n),
                        zero_step_counters ? 1 : 0);
     d.qpar ^= 1;
 }
@@ -1719,7 +1726,7 @@ __global__ void __launch_bounds__(kBlock) k_leaf_setup(int32_t n, int32_t chunks
             d.leaf_lca[0] = 1;
             d.leaf_lca[1] = -1;
         }
-        if (d.qgrid) {  // the first refit's grid
+        if (keeps_on_records(d, n)) {  // the first refit's grid
             const float* b = d.scene_box;
             q_grid(d.qgrid + 8 * d.qpar, Box{b[0], b[1], b[2], b[3], b[4], b[5]});
         }

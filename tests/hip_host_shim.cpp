@@ -89,8 +89,14 @@ int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* sh, void** s) {
     *s = g_stream;
     return 0;
 }
-int hipLaunchKernel(const void* f, Dim3 g, Dim3 b, void**, size_t, void* s) {
-    note("launch %s grid %u block %u stream %p", names()[f].c_str(), g.x, b.x, s);
+int hipLaunchKernel(const void* f, Dim3 g, Dim3 b, void** args, size_t, void* s) {
+    const std::string& name = names()[f];
+    // the refit kernels: how many of the first 14 words of the device state are set (up to the KEEP records)
+    int set = 0;
+    if (name.find("k_refit") != std::string::npos)
+        for (int i = 0; i < 14; ++i)
+            set += static_cast<void**>(args[name.find("k_refit_top") != std::string::npos ? 0 : 1])[i] != nullptr;
+    note("launch %s grid %u block %u set %d stream %p", name.c_str(), g.x, b.x, set, s);
     return 0;
 }
 void** __hipRegisterFatBinary(const void*) {

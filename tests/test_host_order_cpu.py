@@ -124,3 +124,35 @@ for grid, unroll, block in [(777, 4, 512), (64, 1, 128), (3000, 2, 256)]:
     for l in keeps:
         assert "k_keepILi%dELi%dE" % (unroll, block // 64) in l[1] and l[3] == str(grid) and l[5] == str(block), keeps
 """, T)
+
+
+def test_refits_write_the_records_that_keep_reads(shim):
+    """The 16-byte records are written by refits of scenes of 2^20 triangles and more, not by those of a
+    smaller scene in a large context nor of an inter-object front's second object."""
+    run(shim, """
+T = 1 << 20
+caps = dict(int_front_cap=4096, ext_front_cap=4096, pair_cap=4096)
+v = np.zeros((3, 3), np.float32)
+faces = np.tile(np.array([[0, 1, 2]], np.int32), (T, 1))
+ctx = pkg.CollisionContext(T, 3, **caps)
+def refits(step):  # the pointers that the two refit kernels have
+    shim.shim_clear()
+    step()
+    kernels = [int(l[7]) for l in log() if l[0] == "launch" and "k_refit" in l[1]]
+    assert len(kernels) == 2 and kernels[0] == kernels[1]
+    return kernels[0]
+ctx.set_topology(faces, 3)
+ctx.update_vertices(v)
+full = refits(lambda: ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE))
+for n, records in [(T, True), (T - 1, False), (5000, False), (T, True)]:
+    ctx.set_topology(faces[:n], 3)
+    ctx.update_vertices(v)
+    want = full if records else full - 2  # without the internal nodes' and the leaves' records
+    assert refits(lambda: ctx.step(pkg.BVH_BUILD, pkg.FRONT_GENERATE)) == want
+    assert refits(lambda: ctx.step(pkg.BVH_REFIT, pkg.FRONT_KEEP)) == want
+inter = pkg.InterFront(ctx, T, 3, **caps)
+inter.set_topology(faces, 3)
+inter.update_vertices(v)
+for op in (pkg.BVH_BUILD, pkg.BVH_REFIT):
+    assert refits(lambda: inter.step(op, pkg.FRONT_KEEP)) == full - 2
+""")
