@@ -34,9 +34,8 @@ namespace bvhcd {
 
 constexpr int kWaves = kBlock / 64;
 constexpr uint32_t kStage = 256;   // staged entries per wave, single-list kernels
-// Per list when a kernel stages three lists. 128 would fit 8 waves/SIMD in LDS, but every flush
-// is one atomic on the list's single counter and those serialise (measured: GENERATE 2.9 ms at
-// 256, 5.5 ms at 128 on the 2M-triangle cloth), so fewer, larger flushes win.
+// Per list where the incremental restructure stages three lists (GENERATE and UPDATE: kWalkStage,
+// kSproutStage, which leave them more resident waves). A flush is one atomic on a segment counter.
 constexpr uint32_t kStage3 = 256;
 
 __device__ inline uint64_t lanes_below() { return (1ull << lane_id()) - 1ull; }
@@ -728,6 +727,7 @@ __device__ inline uint32_t desc_pop(lds_int2* stk, lds_u32* top, bool& active, i
 // per lane, parts of it handed to idle lanes, us: 2.6k triangles 48 -> 36, 41k 62 -> 45, 65k boxes 134 ->
 // 101, 130k 152 -> 115, 8.4M 3850 -> 3350.
 constexpr uint32_t kWalkStack = 256, kWalkStage = 192;  // 24 resident waves per CU
+static_assert(kWalkStage <= kStage3, "k_wave_order's lanes hold a chunk (one flush) of up to kStage3 entries");
 constexpr int32_t kChain = 64;
 template <bool FRONT>
 __global__ void __launch_bounds__(kBlock) k_traverse(int32_t n, uint32_t per, DevState d, FrontSink fi, FrontSink fe) {

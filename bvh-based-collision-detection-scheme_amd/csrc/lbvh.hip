@@ -466,6 +466,8 @@ __global__ void __launch_bounds__(kBlock) k_sort_pass(const K* __restrict__ keys
 
 // Tiles of 1024 keys up to this many keys (256 workgroups), of 4096 above.
 constexpr int64_t kSortSmall = 1 << 18;
+constexpr int kSortSmallTile = 1024;
+static_assert(kSortSmall <= kSortChained, "small tiles are chained");
 size_t sort_state_words(int64_t n) {
     const int64_t tiles = n <= kSortSmall ? (n + 1023) / 1024 : std::max<int64_t>((n + 4095) / 4096, kSortSmall / 1024);
     return (size_t)(2 * kRadix * std::max<int64_t>(tiles, 1));
@@ -481,7 +483,7 @@ static bool sort_passes(DevState& d, K* keys, int32_t* vals, K* tkeys, int32_t* 
                         int passes, hipStream_t s) {
     constexpr int kTile = kBlock * ITEMS;
     const unsigned tiles = (unsigned)((n + kTile - 1) / kTile);
-    if (n > kSortChained) {
+    if constexpr (kTile > kSortSmallTile) if (n > kSortChained) {
         uint32_t* table = reinterpret_cast<uint32_t*>(d.sort_state);
         for (int p = 0; p < passes; ++p) {
             hipLaunchKernelGGL((k_sort_table<K, ITEMS>), dim3(tiles), dim3(kBlock), 0, s, keys, n, dn, 8 * p, table);
@@ -510,7 +512,7 @@ bool radix_sort_passes(DevState& d, K* keys, int32_t* vals, K* tkeys, int32_t* t
     if (n <= 1 && !dn) return false;
     if (n < 1) return false;
     const int passes = (nbits + 7) / 8;
-    return n <= kSortSmall ? sort_passes<K, 4>(d, keys, vals, tkeys, tvals, n, dn, passes, s)
+    return n <= kSortSmall ? sort_passes<K, kSortSmallTile / kBlock>(d, keys, vals, tkeys, tvals, n, dn, passes, s)
                            : sort_passes<K, 16>(d, keys, vals, tkeys, tvals, n, dn, passes, s);
 }
 
