@@ -92,3 +92,29 @@ def test_keep_counts_every_entry_once(pkg):
     assert tests[0] == tests[1] == tests[2]
     assert tests[0] >= s["int_front"] + s["ext_front"] - s["implicit_pairs"] > sc.num_tris
     ctx.close()
+
+
+def test_keep_of_moved_boxes_descends(pkg):
+    """Boxes given by the caller, moved since the front was made: KEEP's records and descents find what a
+    pure traversal of the same boxes finds, on a cloth that folds on and one that falls back open."""
+    sc = pkg.Scene.preset("cloth1024", n=726)
+    print(f"[gpu] keep of moved boxes, {sc.num_tris}", flush=True)
+    faces = sc.faces()
+    ctx, ref = (pkg.CollisionContext(sc.num_tris, sc.num_verts, narrow_phase=False) for _ in range(2))
+    for c in (ctx, ref):
+        c.set_topology(faces, sc.num_verts)
+    seen = set()
+    for k, fr in enumerate([-12, -8, -1, -12]):
+        v = sc.frame(sc.frames + fr)[faces]
+        boxes = np.concatenate([v.min(1), v.max(1)], 1)
+        for c, op in ((ctx, pkg.FRONT_KEEP if k else pkg.FRONT_GENERATE), (ref, pkg.FRONT_PURE_BVH_CD)):
+            c.update_boxes(boxes)
+            c.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, op)
+        s = ctx.stats()
+        assert ctx.digest(False) == ref.digest(False) and s["implicit_pairs"] == 0, fr
+        if k in (1, 2):
+            assert s["node_visits"] > s["int_front"] + s["ext_front"], fr  # it did descend
+        seen.add(ctx.digest(False))
+    assert len(seen) == 3
+    ctx.close()
+    ref.close()
