@@ -313,6 +313,13 @@ __global__ void k_check_faces(int64_t n, const int32_t* __restrict__ f, int32_t 
     if (any) atomicOr(bad, 1u);
 }
 
+// What a new topology clears, in one launch.
+__global__ void __launch_bounds__(1024) k_forget(DevState d) {
+    for (int i = threadIdx.x; i < 2 * kPairSegs * kCntStride; i += 1024) d.pcnt[i] = 0u;
+    if (threadIdx.x < 4) d.fsize[threadIdx.x] = 0u;
+    if (threadIdx.x < 32) d.ctr[threadIdx.x] = 0u;
+}
+
 __global__ void k_log_frame(DevState d, int cur_int, int cur_ext, uint64_t* out) {
     if (threadIdx.x != 0) return;
     out[0] = ctr64(d.ctr)[C64_VISITS];
@@ -409,14 +416,12 @@ void frame_bytes(double T, double V, int bvh_op, int front_op, double visits, do
 // Host vertices of this size go through the pinned stages (bvhcd_update_vertices).
 bool staged_upload(const bvhcd_ctx* c) { return sizeof(float) * 3 * (size_t)c->V <= kStageBytes; }
 // Once kernels that read an own vertex buffer are enqueued, the next upload into that buffer on the
-// copy stream must wait for them, also when a later part of the step fails. (Uploads through a buffer's
-// stage are ordered by the context stream. A stage stays once it is there, and the size class only
-// changes with the topology, whose call waits for the stream; without a stage, small uploads go on the
-// copy stream too.)
+// copy stream must wait for them, also when a later part of the step fails. (Staged uploads are
+// ordered by the context stream, and the size class only changes with the topology, whose call waits
+// for the stream. Small uploads whose stage can't be had record the event themselves.)
 void mark_consumed(bvhcd_ctx* c) {
-    if (c->d.verts != c->own_verts && c->d.verts != c->own_verts2) return;
-    const int b = c->d.verts == c->own_verts2 ? 1 : 0;
-    if (!(staged_upload(c) && c->stage[b])) (void)hipEventRecord(c->consumed[b], c->stream);
+    if (!staged_upload(c) && (c->d.verts == c->own_verts || c->d.verts == c->own_verts2))
+        (void)hipEventRecord(c->consumed[c->d.verts == c->own_verts2 ? 1 : 0], c->stream);
 }
 
 // ---------------------------------------------------------------- BVH maintenance
@@ -891,10 +896,9 @@ int bvhcd_set_topology(bvhcd_ctx* c, const int32_t* faces, int64_t T, int64_t V,
     c->d.front_version++;
     c->frame = 0;
     c->d.fcur[0] = c->d.fcur[1] = 0;
-    HIPCHK(c, hipMemsetAsync(c->d.fsize, 0, 4 * sizeof(uint32_t), c->stream));
-    // no pairs until the next step: the totals, and the segment counters that they are summed from
-    HIPCHK(c, hipMemsetAsync(c->d.ctr, 0, 32 * sizeof(uint32_t), c->stream));
-    HIPCHK(c, hipMemsetAsync(c->d.pcnt, 0, 2 * kPairSegs * kCntStride * sizeof(uint32_t), c->stream));
+    // no front and no pairs until the next step: sizes, totals, and the segment counters that those are
+    // summed from
+    hipLaunchKernelGGL(k_forget, dim3(1), dim3(1024), 0, c->stream, c->d);
     // the learned schedule's decision buffers are sized here, not on its first decision frame
     if (c->learned && c->cfg.scheduler == BVHCD_SCHED_LEARNED && learned_reserve(c->learned, (int32_t)T))
         return fail(c, BVHCD_E_OOM, "learned decision buffers");
@@ -932,6 +936,8 @@ int bvhcd_update_vertices(bvhcd_ctx* c, const float* xyz, int64_t V, int where) 
     // Larger ones: the upload goes on the copy stream into the buffer the latest step did not
     // read (once the step before it, which did, is done), so it overlaps the steps still
     // running; the call returns when the copy is complete (the caller may reuse xyz).
+    // (Small ones without a stage wait for all that is queued: their steps record no events.)
+    if (staged_upload(c)) HIPCHK(c, hipEventRecord(c->consumed[b], c->stream));
     HIPCHK(c, hipStreamWaitEvent(c->copy_stream, c->consumed[b], 0));
     HIPCHK(c, hipMemcpyAsync(dst, xyz, sizeof(float) * 3 * V, hipMemcpyHostToDevice, c->copy_stream));
     HIPCHK(c, hipEventRecord(c->copied[b], c->copy_stream));
