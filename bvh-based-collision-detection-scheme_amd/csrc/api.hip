@@ -1748,8 +1748,10 @@ int bvhcd_inter_step(bvhcd_inter* x, int rigid_op, int front_op) {
     launch_pair_totals(v, s, x->narrow);
     inter_keep_view(x, v);
     x->last_front = front_op;
-    // the next host upload into the querying object's vertex buffer waits for these kernels
+    // the next host uploads into either object's vertex buffer wait for these kernels (the narrow phase
+    // reads both)
     mark_consumed(rg);
+    mark_consumed(def);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ifail(x, BVHCD_E_DEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
     return BVHCD_OK;

@@ -156,3 +156,35 @@ inter.update_vertices(v)
 for op in (pkg.BVH_BUILD, pkg.BVH_REFIT):
     assert refits(lambda: inter.step(op, pkg.FRONT_KEEP)) == full - 2
 """)
+
+
+@pytest.mark.parametrize("Vd,Vr", [(87382, 30), (30, 87382), (90000, 90000)])
+def test_uploads_follow_the_inter_steps_that_read_their_buffer(shim, Vd, Vr):
+    """An inter-object step reads both objects' vertices (its narrow phase): the next upload into either
+    one's buffer on the copy stream waits for it, not only for the queried context's own step."""
+    run(shim, """
+Vd, Vr = int(sys.argv[3]), int(sys.argv[4])
+faces = np.arange(30, dtype=np.int32).reshape(-1, 3)
+ctx = pkg.CollisionContext(10, Vd)
+ctx.set_topology(faces, Vd)
+inter = pkg.InterFront(ctx, 10, Vr, int_front_cap=4096, ext_front_cap=4096, pair_cap=4096)
+inter.set_topology(faces, Vr)
+large = {"d": Vd > 87381, "r": Vr > 87381}
+read = {}
+checked = 0
+for k in range(6):
+    for who, obj, V in (("d", ctx, Vd), ("r", inter, Vr)):
+        shim.shim_clear()
+        obj.update_vertices(np.zeros((V, 3), np.float32))
+        if large[who] and k >= 2:  # waited for an event recorded after the inter step before last
+            waits = [l for l in log() if l[0] == "wait"]
+            assert len(waits) == 1 and waits[0][1] in read[k - 2], (k, who, waits, read)
+            checked += 1
+    shim.shim_clear()
+    ctx.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, pkg.FRONT_KEEP if k else pkg.FRONT_GENERATE)
+    inter.step(pkg.BVH_REFIT if k else pkg.BVH_BUILD, pkg.FRONT_KEEP if k else pkg.FRONT_GENERATE)
+    text = log()
+    last = max(i for i, l in enumerate(text) if l[0] == "launch")
+    read[k] = {l[1] for l in text[last:] if l[0] == "record"}  # events recorded after its last kernel
+assert checked == 4 * sum(large.values())
+""", Vd, Vr)
