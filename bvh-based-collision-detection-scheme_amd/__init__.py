@@ -511,7 +511,7 @@ def autotune_report() -> str:
 
 # ----------------------------------------------------------------------------- batched scenes
 class Batch:
-    """Many independent scenes per launch: one tree whose subtrees are the scenes, a persistent
+    """Many independent scenes per launch: one tree whose subtrees are the scenes, one
     self-CD traversal, per-scene narrow-phase hits, and (use_graph) one hipGraph per frame."""
 
     def __init__(self, tris_per_scene, verts_per_scene, *, pair_cap=0, device=0, stream=None):

@@ -10,8 +10,8 @@
 //    subtree (a scene boundary differs in a bit above the Morton bits, i.e. a larger delta than
 //    anything inside a scene); each scene's subtree is the LBVH the scene alone would get;
 //  * refit and the narrow phase run once over all triangles;
-//  * the self-CD traversal is one launch: a wave takes 64 queries at a time, each paired only with
-//    its own scene's leaves to its right;
+//  * the self-CD traversal is one launch: a wave takes 8 to 64 queries (by the triangles) at a
+//    time, each paired only with its own scene's leaves to its right;
 //  * the narrow-phase hits are grouped per scene on the device (counts, exclusive scan,
 //    scatter) into scene-local triangle ids;
 //  * every launch of a frame reads its sizes from device memory and clears its counters with

@@ -610,8 +610,8 @@ static unsigned stream_grid() { return 2048; }
 
 // ---------------------------------------------------------------- launch-shape tuning
 // The reference picks one block size per kernel from the occupancy API
-// (system/CudaDevice/CudaDevice.cu:60-94). Here the grid of the grid-stride and persistent
-// kernels, KEEP's entries per thread and the workgroup size of KEEP and the narrow phase (2, 4
+// (system/CudaDevice/CudaDevice.cu:60-94). Here the grid of the grid-stride kernels,
+// KEEP's entries per thread and the workgroup size of KEEP and the narrow phase (2, 4
 // or 8 wave64s, their LDS sized to match) are tuned per kernel and size class ceil(log2 n), by
 // timing candidates on live data (bvhcd_autotune / bvhcd_batch_autotune). The table is
 // process-wide and not locked.

@@ -26,7 +26,7 @@ bool radix_sort_u32_dev(DevState& d, uint32_t* keys, int32_t* vals, uint32_t* tk
 void radix_sort_u64(DevState& d, uint64_t* keys, int32_t* vals, uint64_t* tkeys, int32_t* tvals, int64_t n, int nbits,
                     hipStream_t s);
 void launch_emit_full(DevState& d, int32_t n, hipStream_t s);
-// Launch-shape tuning: grid sizes (workgroups) of the grid-stride / persistent kernels per size
+// Launch-shape tuning: grid sizes (workgroups) of the grid-stride kernels per size
 // class ceil(log2 n), process-wide; 0 entries fall back to the defaults.
 enum TunedKernel { TK_KEEP = 0, TK_NARROW = 1, TK_BATCH_CD = 2, TK_COUNT = 3 };
 // A launch shape: grid size (low 24 bits) and items per thread per loop iteration (1, 2, 4).

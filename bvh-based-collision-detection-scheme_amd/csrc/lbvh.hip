@@ -108,7 +108,8 @@ void launch_box_and_codes(DevState& d, int32_t T, uint32_t* codes, int32_t* vals
 }
 
 // ======================================================================= chained tiles
-// The scan and the sort's digit passes run as one launch each: tiles hand their running sums on to
+// The scan and the sort's digit passes run as one launch each, by the published single-pass scan with
+// decoupled look-back (Merrill and Garland 2016): tiles hand their running sums on to
 // the following ones through a word per tile (and digit), a 64-bit (flag, value) pair written and
 // read in one access: kTileSum = the tile's own sum, kTileRun = the sum of all tiles up to it. A
 // workgroup takes its tile from a counter, so every tile it waits for belongs to a workgroup that is
@@ -1386,9 +1387,9 @@ __global__ void __launch_bounds__(kRefitBlock) k_refit(int32_t n, DevState d) {
     const int2 info = d.rp_cinfo[c];  // (internal nodes, deepest level | treelet roots << 16)
     // leaf boxes: LDS + records; per-triangle finiteness for the narrow phase. A leaf's face
     // indices arrive in one load and its three vertices together, the leaves of a thread one
-    // after another: measured fastest on the 2M-triangle cloth (k_refit 46.8 us, against 50.4
-    // with every index and vertex loaded on its own and 63-69 with all of a thread's loads in
-    // flight at once, which congests the gathers).
+    // after another: measured fastest on the 2M-triangle cloth (k_refit without KEEP's records
+    // 46.8 us, with them 67.8; against 50.4 with every index and vertex loaded on its own and 63-69 with all of a thread's
+    // loads in flight at once, which congests the gathers).
     int bad = 0;
 #pragma unroll
     for (int k = 0; k < kRefitPerT; ++k) {

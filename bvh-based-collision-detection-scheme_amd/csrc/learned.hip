@@ -320,8 +320,9 @@ int learned_forward_noalloc(LearnedState* L, int device, const float* feats, int
 //    the gradient of layer 1's output) go through an LDS transpose (16 x 64 tile of the wave, row
 //    stride 68: writes and reads free of bank conflicts).
 // Each workgroup leaves its sums in `part` (kGradStride words), which k_train_finish adds up in a
-// fixed order: repeated runs give the same bits. Bound by MFMA issue and the launch itself:
-// 49,061 rows take 0.042 ms. (One thread per row, adding each of its 5313 gradients to the
+// fixed order: repeated runs give the same bits. 49,061 rows take 41 us: 24 whatever the rows (weights
+// into LDS, the workgroup's sums), then 6.8 for each further tile of a wave, of which its 224 MFMA
+// take 3 and the LDS transposes the rest (one wave per SIMD). (One thread per row, adding each of its 5313 gradients to the
 // workgroup's LDS sums, took 19.5 ms: all 64 lanes added to one LDS word at a time.)
 constexpr int kTrainBlock = 256;
 constexpr int kTrainWaves = kTrainBlock / 64;

@@ -155,11 +155,14 @@ int  bvhcd_create(const bvhcd_config* cfg, bvhcd_ctx** out);
 int  bvhcd_destroy(bvhcd_ctx* ctx);
 const char* bvhcd_last_error(const bvhcd_ctx* ctx);
 
-/* faces: T x int32[3] vertex ids. Topology is fixed until the next call (it resets BVH and front). */
+/* faces: T x int32[3] vertex ids. Topology is fixed until the next call (it resets BVH, front and
+   pairs: the read-outs report none until the next step). */
 int  bvhcd_set_topology(bvhcd_ctx* ctx, const int32_t* faces, int64_t num_tris, int64_t num_verts, int where);
-/* xyz: V x float[3]. Device memory: copied D2D on the context stream. Host memory: uploaded on
-   the context's copy stream into one of two device buffers, overlapping the step still running
-   on the GPU; returns when the copy is complete, so xyz may be reused at once. */
+/* xyz: V x float[3]. Device memory: copied D2D on the context stream. Host memory, which may be
+   reused at once: up to 1 MB (87,381 vertices) copied into a pinned buffer of the context and queued
+   on the context stream, the call does not wait; more is uploaded on the context's copy stream into
+   one of two device buffers, overlapping the step still running on the GPU, and the call returns
+   when the copy is complete. */
 int  bvhcd_update_vertices(bvhcd_ctx* ctx, const float* xyz, int64_t num_verts, int where);
 /* Box mode, the simulator-facing input of the reference (ARCSimSceneData, world/Scene.h:39-46;
    LBvhFixedDeformable::maintain, LBvhFixedDeformable.cu:89-112; calcMaxBVARCSim / calcMCsARCSim,
@@ -324,8 +327,8 @@ int  bvhcd_batch_pair_counts(bvhcd_batch* b, int64_t* counts /* num_scenes */);
 const char* bvhcd_batch_last_error(const bvhcd_batch* b);
 
 /* ---- autotuner (replaces CudaDevice::launchConfig / evalOptimalBlockSize, CudaDevice.cu:60-94) ----
-   Block sizes are fixed at 256 (wave64 x 4); the launch shapes of the grid-stride and persistent
-   kernels (grid size, for KEEP the entries per thread per loop iteration, and for KEEP and the
+   Block sizes are fixed at 256 (wave64 x 4); the launch shapes of the grid-stride kernels
+   (grid size, for KEEP the entries per thread per loop iteration, and for KEEP and the
    narrow phase the workgroup size: 128, 256 or 512 threads) are tuned by timing candidates on the
    current data, per kernel and size class ceil(log2 n), in a process-wide table used by every
    later launch. */
