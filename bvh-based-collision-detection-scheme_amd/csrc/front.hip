@@ -1782,11 +1782,12 @@ __device__ inline uint32_t desc_drain(const DevState& d, const Out& out, lds_int
 // leave many open: where the last KEEP's records left more than one entry in kOpenMost open (counted by one
 // workgroup in kOpenSample), this kernel ends at once and the one without Q that is launched after it
 // (otherwise) does the work; the count is handed on until a step without KEEP or REORDER clears it.
-// (Both loops in one kernel: 8 % slower.) Records / boxes, us: 3.9 % open 289 / 304 (sheets of 2.1M), 1073 / 1209 (of
-// 8.4M); 4.4 % 193 / 197 (cloth of 1.3M), 288 / 331 (of 2.1M); 4.6 % 297 / 305; 5.8 % 305 / 304; 6.3 %
-// 1179 / 1204; 7.6 % 322 / 301; 8.4 % 1244 / 1212; 13 % 388 / 318. KEEP, us, boxes -> Q: 2.1M triangles 432..646 -> 365..596 over ten frames of a front, sheets of
-// 2.9M 375 -> 265, of 8.4M 1150 -> 1033 (without shared-vertex pairs) and 937 -> 745; the refit that writes the records takes 9 us (2.1M) and 67 us
-// (8.4M) longer. Below a million triangles the gain is within that cost.
+// (Both loops in one kernel: 8 % slower.) Records / boxes, us: 3.9 % open 289 / 304 (sheets of 2.1M), 1073 /
+// 1209 (of 8.4M); 4.4 % 193 / 197 (cloth of 1.3M), 288 / 331 (of 2.1M); 4.6 % 297 / 305; 5.8 % 305 / 304; 6.3
+// % 1179 / 1204; 7.6 % 322 / 301; 8.4 % 1244 / 1212; 13 % 388 / 318. KEEP, us, boxes -> Q: 2.1M triangles
+// 432..646 -> 365..596 over ten frames of a front, sheets of 2.9M 375 -> 265, of 8.4M 1150 -> 1033 (without
+// shared-vertex pairs) and 937 -> 745; the refit that writes the records takes 16 us (2.1M) and 68 us (8.4M)
+// longer. Below a million triangles the gain is within that cost.
 // implicit: the current front's shared-vertex head (C_ADJ entries after the last partition) is
 // not tested when the last refit found every coordinate finite: its pairs are broad-phase hits
 // whatever the positions (both boxes hold the shared vertex) and are counted, not listed.
